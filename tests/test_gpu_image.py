@@ -101,3 +101,27 @@ def test_import_rejects_inconsistent_offsets(gpu, oracle):
         assert np.array_equal(g.export_image(), img)
     finally:
         g.close()
+
+
+@pytest.mark.parametrize("nbits", [6, 13, 14])
+@pytest.mark.parametrize("shift", [0, 1, 8, 16])
+def test_export_at_any_address(gpu, nbits, shift):
+    """The image's bytes at every alignment of the output, block counts on
+    both sides of the packing workgroup's 256 (3, 142, 282 blocks), nothing
+    written past them."""
+    import torch
+    from cqf_amd.gqf import GQF, fill_splitmix64
+    print(f"case export nbits={nbits} shift={shift}", flush=True)
+    f = GQF(nbits)
+    try:
+        keys = torch.empty(int(0.9 * (1 << nbits)), dtype=torch.int64, device="cuda")
+        fill_splitmix64(keys, 11)
+        f.bulk_insert(keys)
+        want = torch.from_numpy(f.export_image())
+        buf = torch.full((f.nbytes + 64,), 0xA5, dtype=torch.uint8, device="cuda")
+        f.export_image_device(buf[shift:shift + f.nbytes])
+        got = buf.cpu()
+        assert torch.equal(got[shift:shift + f.nbytes], want)
+        assert bool((got[:shift] == 0xA5).all()) and bool((got[shift + f.nbytes:] == 0xA5).all())
+    finally:
+        f.close()
