@@ -217,10 +217,14 @@ struct gqf_group_dev {
 };
 #define GQF_GROUP_MAX_POLLS (1u << 22)  // default bound: about 1 s of polls, far above any region's rebuild
 
-// the persistent rebuild over every filter's regions (even items, then odd
-// items that wait for their even neighbours), then the wide redo tail
-void gqf_launch_group_rebuild(const gqf_group_dev& g, const uint64_t* items, int mode, uint32_t grid,
-                              hipStream_t s);
+// whether a batch of inserts is dense enough for the workgroup-wide rebuild
+bool gqf_rebuild_is_dense(uint64_t n_items, uint64_t nregions);
+// the rebuild over every filter's regions, then the wide redo tail: dense
+// batches one workgroup per region, even regions then odd ones (n_even /
+// n_odd of them); others the persistent launch of `grid` workgroups (even
+// items, then odd items that wait for their even neighbours)
+void gqf_launch_group_rebuild(const gqf_group_dev& g, const uint64_t* items, int mode, uint32_t grid, uint64_t n_even,
+                              uint64_t n_odd, bool dense, hipStream_t s);
 #define GQF_GROUP_PER_CU 8  // workgroups per CU of the persistent rebuild unless tuned
 uint32_t gqf_group_rebuild_max_per_cu();
 uint32_t gqf_group_rebuild_grid(uint32_t per_cu);

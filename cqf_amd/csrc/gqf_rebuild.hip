@@ -35,6 +35,7 @@
 #include <type_traits>
 #include <utility>
 
+#include "gqf_flat.h"
 #include "gqf_internal.h"
 #include "gqf_launch.h"
 
@@ -1598,6 +1599,14 @@ __device__ __forceinline__ int rebuild_region(const QF& qf, uint64_t r, const ui
 // ---------------------------------------------------------------------------
 // kernels
 
+// marks region r for the wide pass
+__device__ __forceinline__ void flag_wide(uint64_t r, uint8_t* __restrict__ wide_flags,
+                                          uint32_t* __restrict__ wide_count) {
+  wide_flags[r] = 1;
+  const uint32_t k = atomicAdd(wide_count, 1u);
+  if (k < GQF_WIDE_LIST) wide_count[1 + k] = (uint32_t)r;
+}
+
 // One workgroup per non-empty region of one parity: workgroup i takes
 // region list[i] (the list gqf_region_bounds compacted; count[parity]
 // entries), so a small batch launches only as many workgroups as it has
@@ -1623,9 +1632,7 @@ __device__ __forceinline__ void rebuild_phase_item(const QF* __restrict__ qfp, c
   const int res = rebuild_region<kWinFast>(qf, r, items, counts, s, e, mode, sm, lcnt, true);
   if (lane_id() == 0) {
     if (res == kNeedWide) {
-      wide_flags[r] = 1;
-      const uint32_t k = atomicAdd(wide_count, 1u);
-      if (k < GQF_WIDE_LIST) wide_count[1 + k] = (uint32_t)r;
+      flag_wide(r, wide_flags, wide_count);
     } else if (res == kNoSpace) {
       atomicOr(qf.status, GQF_STATUS_NO_SPACE);
     }
@@ -1651,6 +1658,27 @@ gqf_rebuild_phase_counts(const QF* __restrict__ qfp, const uint64_t* __restrict_
   __shared__ uint32_t icnt[kItemCap];
   rebuild_phase_item(qfp, items, counts, region_start, region_list, list_count, parity, mode, wide_flags, wide_count,
                      sm, icnt);
+}
+
+// One workgroup of gqf_flat::kThreads per non-empty region of one parity
+// (gqf_flat.h), flagging regions for the wide pass as rebuild_phase_item does.
+extern "C" __global__ void __launch_bounds__(gqf_flat::kThreads)
+gqf_rebuild_flat(const QF* __restrict__ qfp, const uint64_t* __restrict__ items, const uint64_t* __restrict__ counts,
+                 const uint32_t* __restrict__ region_start, const uint32_t* __restrict__ region_list,
+                 const uint32_t* __restrict__ list_count, int parity, int kind, uint8_t* __restrict__ wide_flags,
+                 uint32_t* __restrict__ wide_count) {
+  __shared__ gqf_flat::Smem sm;
+  const QF qf = *qfp;
+  if (blockIdx.x >= list_count[parity]) return;
+  const uint64_t r = region_list[blockIdx.x];
+  if (r >= qf.nregions) return;
+  const uint64_t s = region_start[r], e = region_start[r + 1];
+  if (s == e) return;
+  const int res = gqf_flat::rebuild(qf, r, items, counts, s, e, kind, 0, sm);
+  if (threadIdx.x == 0) {
+    if (res == gqf_flat::kNeedWide) flag_wide(r, wide_flags, wide_count);
+    else if (res == gqf_flat::kNoSpace) atomicOr(qf.status, GQF_STATUS_NO_SPACE);
+  }
 }
 
 // Redoes flagged regions of one parity with a wider window: 128 blocks,
@@ -2032,6 +2060,32 @@ gqf_group_rebuild(gqf_group_dev g, const uint64_t* __restrict__ items, int mode)
   }
 }
 
+// The dense form of gqf_group_rebuild: one workgroup of gqf_flat::kThreads
+// per region of one parity over all filters (two launches, so an odd region
+// needs no flags to know that its even neighbours are done).
+extern "C" __global__ void __launch_bounds__(gqf_flat::kThreads)
+gqf_group_flat(gqf_group_dev g, const uint64_t* __restrict__ items, int parity) {
+  __shared__ gqf_flat::Smem sm;
+  const uint64_t* base = parity ? g.odd_base : g.even_base;
+  const uint64_t k = blockIdx.x;
+  if (k >= base[g.nf]) return;
+  const uint32_t f = item_filter(base, g.nf, k);
+  const uint64_t r = 2 * (k - base[f]) + (uint64_t)parity;
+  const QF qf = g.descs[f];
+  uint64_t s, e, tag;
+  region_hash_bounds(g, qf, f, r, items, s, e, tag);
+  if (s >= e) return;
+  const int res = gqf_flat::rebuild(qf, r, items, nullptr, s, e, gqf_flat::kAdd, tag, sm);
+  if (threadIdx.x == 0) {
+    if (res == gqf_flat::kNeedWide) {
+      g.wide[g.reg_base[f] + r] = 1;
+      atomicAdd(&g.counters[2], 1u);
+    } else if (res == gqf_flat::kNoSpace) {
+      atomicOr(qf.status, GQF_STATUS_NO_SPACE);
+    }
+  }
+}
+
 // Redoes flagged regions with the wide window, in ascending region order
 // within each filter.  Filters share no blocks, so each filter has its own
 // workgroup (one long serial tail took 7.5 ms per 256-filter insert).
@@ -2120,6 +2174,14 @@ std::atomic<uint32_t> g_wide_max_polls{kWideMaxPolls};
 
 uint32_t gqf_wide_wait_bound_set(uint32_t max_polls) { return g_wide_max_polls.exchange(max_polls); }
 
+// Batches of at least this many items per region on average take the
+// workgroup-wide rebuild (gqf_flat.h): inserts when regions start to outgrow
+// the item cache (256) and would walk their runs -- below that the shift path
+// is ahead (153 items a region at 2^26 slots: 97 us a launch against 280) --
+// and the other kinds sooner, as they always walk.
+constexpr uint64_t kFlatItems = 208, kFlatItemsMixed = 96;
+bool gqf_rebuild_is_dense(uint64_t n_items, uint64_t nregions) { return n_items >= kFlatItems * nregions; }
+
 void gqf_launch_rebuild(const QF* qf_dev, uint64_t nregions, uint64_t region_blocks, const uint64_t* items,
                         const uint64_t* counts, uint64_t n_items, const uint32_t* region_start,
                         const uint32_t* region_list, const uint32_t* list_count, int mode, uint8_t* wide_flags,
@@ -2136,10 +2198,15 @@ void gqf_launch_rebuild(const QF* qf_dev, uint64_t nregions, uint64_t region_blo
     fprintf(stderr, "gqf: %u wide classes for %llu-block regions\n", ncls, (unsigned long long)region_blocks);
     abort();
   }
+  const int kind = mode == kSeq ? gqf_flat::kTagged : (counts ? gqf_flat::kCounts : gqf_flat::kAdd);
+  const bool flat = mode != kDelete && n_items >= (kind == gqf_flat::kAdd ? kFlatItems : kFlatItemsMixed) * nregions;
   mode |= gqf_rebuild_mode_flags();
   for (int parity = 0; parity < 2; parity++) {
     gqf_prof_begin("rebuild_phase", s);
-    if (counts || (mode & ~GQF_REBUILD_NO_SHIFT) == kSeq)
+    if (flat)
+      hipLaunchKernelGGL(gqf_rebuild_flat, dim3(g), dim3(gqf_flat::kThreads), 0, s, qf_dev, items, counts, region_start,
+                         region_list + (size_t)parity * stride, list_count, parity, kind, wide_flags, wide_count);
+    else if (counts || (mode & ~GQF_REBUILD_NO_SHIFT) == kSeq)
       hipLaunchKernelGGL(gqf_rebuild_phase_counts, dim3(g), dim3(64), 0, s, qf_dev, items, counts, region_start,
                          region_list + (size_t)parity * stride, list_count, parity, mode, wide_flags, wide_count);
     else
@@ -2185,14 +2252,21 @@ uint32_t gqf_group_rebuild_grid(uint32_t per_cu) {
   return (uint32_t)cus * (per_cu < mx ? per_cu : mx);
 }
 
-void gqf_launch_group_rebuild(const gqf_group_dev& g, const uint64_t* items, int mode, uint32_t grid,
-                              hipStream_t s) {
-  mode |= gqf_rebuild_mode_flags();
+void gqf_launch_group_rebuild(const gqf_group_dev& g, const uint64_t* items, int mode, uint32_t grid, uint64_t n_even,
+                              uint64_t n_odd, bool dense, hipStream_t s) {
   gqf_prof_begin("group_rebuild", s);
-  hipLaunchKernelGGL(gqf_group_rebuild, dim3(grid ? grid : 1), dim3(64), 0, s, g, items, mode);
+  if (dense) {
+    for (int parity = 0; parity < 2; parity++) {
+      const uint64_t n = parity ? n_odd : n_even;
+      if (n)
+        hipLaunchKernelGGL(gqf_group_flat, dim3((uint32_t)n), dim3(gqf_flat::kThreads), 0, s, g, items, parity);
+    }
+  } else {
+    mode |= gqf_rebuild_mode_flags();
+    hipLaunchKernelGGL(gqf_group_rebuild, dim3(grid ? grid : 1), dim3(64), 0, s, g, items, mode);
+  }
   gqf_prof_end("group_rebuild", s);
   gqf_prof_begin("rebuild_wide", s);
   hipLaunchKernelGGL(gqf_group_wide, dim3(g.nf ? g.nf : 1), dim3(64), 0, s, g, items, mode);
   gqf_prof_end("rebuild_wide", s);
 }
-
