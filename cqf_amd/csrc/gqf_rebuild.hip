@@ -183,8 +183,8 @@ struct Items {
 // The 8 old slots from st (whatever follows a shorter run included), little
 // endian in x0 / x1: the words holding them read aligned, the row's pad
 // word dropped, and funnel-shifted to st's byte.
-template <int W>
-__device__ __forceinline__ void read_slots8(const Smem<W>& sm, int32_t st, uint32_t& x0, uint32_t& x1) {
+template <class S>
+__device__ __forceinline__ void read_slots8(const S& sm, int32_t st, uint32_t& x0, uint32_t& x1) {
   const uint32_t a = sin_off(st);
   const uint32_t* wp = sm.sin + (a >> 2);
   const uint32_t w0 = wp[0], w1 = wp[1], w2 = wp[2], w3 = wp[3];
@@ -248,43 +248,6 @@ __device__ __forceinline__ void lean_write(Smem<W>& sm, uint32_t lo, uint32_t hi
   atomicOr(&wp[0], y0);
   if (used > 4) atomicOr(&wp[pad == 1 ? 2 : 1], y1);
   if (used > 8) atomicOr(&wp[pad <= 2 ? 3 : 2], y2);
-}
-
-// The straight-line delete merge: one or two items, each removing one
-// instance (an absent key's removal is a no-op), on an old run of at most 8
-// strictly ascending bytes.  Such a run holds count-1 counters only (a
-// count of 2 or more repeats its remainder), so each item's remainder, if
-// present, loses its one byte and the rest stay in order.  Returns false
-// (the general merge, merge_quotient) otherwise; lo / hi / len as
-// lean_read's.  Reads only the old rows, so the measuring and the writing
-// pass can each call it.
-template <int W>
-__device__ __forceinline__ bool lean_delete(const Smem<W>& sm, const Items& src, uint32_t it0, uint32_t it1,
-                                            int32_t st_o, uint32_t old_len, uint32_t h_first, uint32_t& lo,
-                                            uint32_t& hi, uint32_t& len) {
-  const uint32_t n = it1 - it0;
-  if (old_len == 0 || old_len > 8 || n > 2) return false;
-  const uint32_t r0 = h_first & 0xFFu;
-  const uint32_t r1 = n == 2 ? (src.hash(sm.items, it0 + 1) & 0xFFu) : r0;
-  uint32_t x0, x1;
-  read_slots8(sm, st_o, x0, x1);
-  bool asc = true;
-  uint32_t prev = 0, kept = 0;
-  uint64_t y = 0;
-#pragma unroll
-  for (int k = 0; k < 8; k++) {
-    const uint32_t b = ((k < 4 ? x0 : x1) >> (8 * (k & 3))) & 0xFFu;
-    const bool in = (uint32_t)k < old_len;
-    if (k > 0 && in && b <= prev) asc = false;
-    prev = b;
-    const bool keep = in && b != r0 && b != r1;
-    y |= keep ? (uint64_t)b << (8u * kept) : 0ULL;
-    kept += keep ? 1u : 0u;
-  }
-  lo = (uint32_t)y;
-  hi = (uint32_t)(y >> 32);
-  len = kept;
-  return asc;
 }
 
 // ---------------------------------------------------------------------------
@@ -532,9 +495,8 @@ __device__ __forceinline__ bool walk_block(Smem<W>& sm, int j, int nwin, const I
 // quotient's items.  The per-block walk then only reads the table, so its
 // loop body is the same for every lane.
 
-template <int W>
-__device__ __forceinline__ bool locate_old_run(const Smem<W>& sm, int nwin, int32_t q, int32_t& st_o,
-                                               uint32_t& old_len) {
+template <class S>
+__device__ __forceinline__ bool locate_old_run(const S& sm, int nwin, int32_t q, int32_t& st_o, uint32_t& old_len) {
   const int j = q >> 6;
   const int bit = q & 63;
   const uint64_t occ = sm.occ_in[j];
@@ -794,12 +756,69 @@ __device__ __forceinline__ uint32_t lshl_or_c(uint32_t x, uint32_t acc) {  // (x
   return r;
 }
 
+__device__ __forceinline__ uint32_t twice_add(uint32_t bit, uint32_t acc) {  // (bit << 1) + acc
+  uint32_t r;
+  asm("v_lshl_add_u32 %0, %1, 1, %2" : "=v"(r) : "v"(bit), "v"(acc));
+  return r;
+}
+__device__ __forceinline__ int32_t cap_shift(int32_t x, int32_t cap) {  // min(x, max(cap, 0)) for x >= 0
+  int32_t r;
+  asm("v_med3_i32 %0, %1, 0, %2" : "=v"(r) : "v"(x), "v"(cap));
+  return r;
+}
+
 // ORs the low `len` bits of `bits` into the window bit array at position d
 // (len <= 64; the bits may straddle two words)
 __device__ inline void or_bits(uint64_t* arr, int32_t d, uint64_t bits, int len) {
   const int w = d >> 6, sh = d & 63;
   atomicOr((unsigned long long*)&arr[w], bits << sh);
   if (sh && sh + len > 64) atomicOr((unsigned long long*)&arr[w + 1], bits >> (64 - sh));
+}
+
+// New offset of block j = lane (j < bstar) by rank over the new run ends
+// (run_out of blocks below bstar, run_in of the rest): the runs of quotients
+// < 64 j end at the k-th run end of the window, k = the earlier regions' runs
+// that end inside the window (run ends at or before xold[0]) + the occupied
+// quotients of blocks < j.  All lanes call it; xnew is overwritten.
+template <class S>
+__device__ __forceinline__ uint32_t offset_by_rank(S& sm, int nwin, int bstar, uint64_t occ_new) {
+  const int j = lane_id();
+  const uint64_t re_w = j < bstar ? sm.run_out[j] : (j < nwin ? sm.run_in[j] : 0ULL);
+  uint32_t c_occ = (uint32_t)__popcll(occ_new), c_re = (uint32_t)__popcll(re_w);
+  uint32_t c_pre = 0;
+  {
+    const int32_t x0 = sm.xold[0];
+    if (j < nwin && x0 >= 64 * j) {
+      const int upto = x0 - 64 * j + 1;
+      c_pre = (uint32_t)__popcll(sm.run_in[j] & gqf_mask((uint64_t)(upto < 64 ? upto : 64)));
+    }
+  }
+  const uint32_t inc_occ = wave_scan_add(c_occ), inc_re = wave_scan_add(c_re);
+  const uint32_t tot_pre = (uint32_t)__builtin_amdgcn_readlane((int)wave_scan_add(c_pre), 63);
+  sm.xnew[j] = (int32_t)(inc_re - c_re);  // run ends in blocks < j
+  if (j == 63) sm.xnew[64] = (int32_t)inc_re;
+  __syncthreads();
+  uint32_t off_new = 0;
+  if (j < bstar) {
+    const uint32_t k = tot_pre + inc_occ - c_occ;  // runs of quotients < 64 j ending in the window
+    int32_t x = 64 * j - 1;
+    if (k > 0) {
+      if (k > (uint32_t)sm.xnew[nwin]) {
+        x = sm.xold[j];  // ends past the window, where nothing moved
+      } else {
+        int lo = 0, hi = nwin - 1;  // the block holding the k-th run end: cum[b] < k <= cum[b + 1]
+        while (lo < hi) {
+          const int mid = (lo + hi + 1) >> 1;
+          if ((uint32_t)sm.xnew[mid] < k) lo = mid; else hi = mid - 1;
+        }
+        const uint64_t w = lo < bstar ? sm.run_out[lo] : sm.run_in[lo];
+        const int32_t p = 64 * lo + gqf_select64(w, (int)(k - (uint32_t)sm.xnew[lo]) - 1);
+        if (p > x) x = p;
+      }
+    }
+    off_new = (uint32_t)(x - (64 * j - 1));
+  }
+  return off_new;
 }
 
 template <int W, bool kStash>
@@ -1130,45 +1149,8 @@ __device__ __forceinline__ int rebuild_insert_shift(const QF& qf, uint64_t B0, i
   }
   __syncthreads();
 
-  // ---- offsets by rank over the new run ends: occupied quotients of the
-  // window's blocks < j, plus the earlier regions' runs that end inside the
-  // window (run ends at or before xold[0])
   const uint64_t occ_new = j < nwin ? (occ | touched) : 0ULL;
-  const uint64_t re_w = j < bstar ? sm.run_out[j] : (j < nwin ? sm.run_in[j] : 0ULL);
-  uint32_t c_occ = (uint32_t)__popcll(occ_new), c_re = (uint32_t)__popcll(re_w);
-  uint32_t c_pre = 0;
-  {
-    const int32_t x0 = sm.xold[0];
-    if (j < nwin && x0 >= 64 * j) {
-      const int upto = x0 - 64 * j + 1;
-      c_pre = (uint32_t)__popcll(sm.run_in[j] & gqf_mask((uint64_t)(upto < 64 ? upto : 64)));
-    }
-  }
-  const uint32_t inc_occ = wave_scan_add(c_occ), inc_re = wave_scan_add(c_re);
-  const uint32_t tot_pre = (uint32_t)__builtin_amdgcn_readlane((int)wave_scan_add(c_pre), 63);
-  sm.xnew[j] = (int32_t)(inc_re - c_re);  // run ends in blocks < j
-  if (lane == 63) sm.xnew[64] = (int32_t)inc_re;
-  __syncthreads();
-  uint32_t off_new = 0;
-  if (j < bstar) {
-    const uint32_t k = tot_pre + inc_occ - c_occ;  // runs of quotients < 64 j ending in the window
-    int32_t x = 64 * j - 1;
-    if (k > 0) {
-      if (k > (uint32_t)sm.xnew[nwin]) {
-        x = sm.xold[j];  // ends past the window, where nothing moved
-      } else {
-        int lo = 0, hi = nwin - 1;  // the block holding the k-th run end: cum[b] < k <= cum[b + 1]
-        while (lo < hi) {
-          const int mid = (lo + hi + 1) >> 1;
-          if ((uint32_t)sm.xnew[mid] < k) lo = mid; else hi = mid - 1;
-        }
-        const uint64_t w = lo < bstar ? sm.run_out[lo] : sm.run_in[lo];
-        const int32_t p = 64 * lo + gqf_select64(w, (int)(k - (uint32_t)sm.xnew[lo]) - 1);
-        if (p > x) x = p;
-      }
-    }
-    off_new = (uint32_t)(x - (64 * j - 1));
-  }
+  const uint32_t off_new = offset_by_rank(sm, nwin, bstar, occ_new);
 
   // ---- store blocks [0, b*): lane j writes block j's line
   if (j < bstar) {
@@ -1370,16 +1352,10 @@ __device__ __forceinline__ int rebuild_region_lines(const QF& qf, uint64_t r, co
     if (shift_ok && fast && kind == kAdd)
       return rebuild_insert_shift<W, kStash>(qf, B0, R, nwin, src, m, sm, occ_w[0], used_w[0], tm_w[0], table_end_in_window);
   }
-  // With kStash, lane takes listed quotients lane + 64 k in round k (at
-  // most kItemCap = 4 x 64 of them), and a delete that takes the
-  // straight-line merge keeps its bytes in registers (del_lo / del_hi, bit k
-  // of del_lean) for the writing pass; without it (a caller short of
-  // registers) both passes call merge_quotient.
-  uint32_t del_lo[4], del_hi[4], del_lean = 0;
   if (fast) {
     // old run and new length of every listed quotient, one quotient per lane
     const uint32_t nq = sm.nq;
-    auto measure = [&](uint32_t t, int k) {
+    for (uint32_t t = lane; t < nq; t += 64) {
       const int32_t q = (int32_t)(sm.items[sm.tit0[t]] >> 8);
       int32_t st_o;
       uint32_t old_len;
@@ -1388,13 +1364,7 @@ __device__ __forceinline__ int rebuild_region_lines(const QF& qf, uint64_t r, co
         const uint32_t it0 = sm.tit0[t];
         const uint32_t it1 = t + 1 < nq ? sm.tit0[t + 1] : m;
         const uint32_t h0 = src.hash(sm.items, it0);
-        uint32_t ln;
-        if (kStash && kind == kSub && lean_delete(sm, src, it0, it1, st_o, old_len, h0, del_lo[k], del_hi[k], ln)) {
-          nl = ln;
-          del_lean |= 1u << k;
-        } else {
-          nl = merge_quotient<W, false>(sm, src, it0, it1, st_o, old_len, 0, h0);
-        }
+        nl = merge_quotient<W, false>(sm, src, it0, it1, st_o, old_len, 0, h0);
       } else {
         atomicMin(&sm.first_invalid, q >> 6);
         st_o = q;
@@ -1407,14 +1377,6 @@ __device__ __forceinline__ int rebuild_region_lines(const QF& qf, uint64_t r, co
       sm.tst[t] = (int16_t)st_o;
       sm.tol[t] = (RunLen<W>)old_len;
       sm.tnl[t] = (RunLen<W>)nl;
-    };
-    if constexpr (kStash) {
-      static_assert(kItemCap <= 4 * 64, "four rounds of listed quotients");
-#pragma unroll
-      for (int k = 0; k < 4; k++)
-        if ((uint32_t)lane + 64u * (uint32_t)k < nq) measure((uint32_t)lane + 64u * (uint32_t)k, k);
-    } else {
-      for (uint32_t t = lane; t < nq; t += 64) measure(t, 0);
     }
   }
   __syncthreads();
@@ -1530,22 +1492,11 @@ __device__ __forceinline__ int rebuild_region_lines(const QF& qf, uint64_t r, co
   if (fast) {
     // counters of the listed quotients at their new starts
     const uint32_t nq = sm.nq;
-    auto write = [&](uint32_t t, int k) {
-      if (sm.tnl[t] == 0) return;
-      if (kStash && ((del_lean >> k) & 1u)) {  // the measuring pass's straight-line delete
-        lean_write(sm, del_lo[k], del_hi[k], sm.tnl[t], sm.tsn[t]);
-        return;
-      }
+    for (uint32_t t = lane; t < nq; t += 64) {
+      if (sm.tnl[t] == 0) continue;
       const uint32_t it0 = sm.tit0[t];
       const uint32_t it1 = t + 1 < nq ? sm.tit0[t + 1] : m;
       merge_quotient<W, true>(sm, src, it0, it1, sm.tst[t], sm.tol[t], sm.tsn[t], src.hash(sm.items, it0));
-    };
-    if constexpr (kStash) {
-#pragma unroll
-      for (int k = 0; k < 4; k++)
-        if ((uint32_t)lane + 64u * (uint32_t)k < nq) write((uint32_t)lane + 64u * (uint32_t)k, k);
-    } else {
-      for (uint32_t t = lane; t < nq; t += 64) write(t, 0);
     }
   }
   __syncthreads();
@@ -1581,6 +1532,336 @@ __device__ __forceinline__ int rebuild_region_lines(const QF& qf, uint64_t r, co
         b[7] = make_uint4(row[12], row[13], row[14], row[15]);
       }
     }
+  }
+  return kOk;
+}
+
+// ---------------------------------------------------------------------------
+// Delete path: every delete batch in the fast window, one wave a region,
+// lane j on block j.  Deletes only shrink runs, so the new layout is the old
+// one with each kept byte moved left by a shift e >= 0 that
+//   * grows by one at every removed slot;
+//   * is capped, at every used slot s of a run of quotient q, by s - q (a
+//     byte never moves in front of its quotient; inside a run the cap never
+//     binds, and an empty slot's cap, against the next run's quotient, is
+//     below zero: the shift ends there).
+// Each is a map e -> min(a, e + b), so lane j folds its 64 slots into one map
+// and a wave scan gives the shift that enters every block; a second pass over
+// the slots moves the bytes.  The quotient of slot s is the k-th occupied one
+// of the window, k = run ends before s: a table in LDS holds them by rank,
+// and the caps stay in 64 registers between the two passes.
+//
+// What is removed: each item's lane finds its quotient's run; in a run of
+// strictly ascending bytes (count-1 counters only) the byte that equals its
+// remainder, if there, is marked.  Any other run is rewritten in place by the
+// lane of its quotient's first item -- no counter's encoding grows when its
+// count shrinks -- and the slots that this frees at its end are marked.
+// The run ends follow from the marks: a kept byte is its run's last if no
+// kept byte follows it up to the old run end.
+//
+// Bound by VALU issue: 2,900 instructions a region wave (128 VGPRs, 15.9 KB
+// of LDS: ten waves on a CU), a third of what the run walk below took for it
+// (8,050), which paired every run with its quotient one by one on its block's
+// lane, in both passes.  7.55 M deletes from 2^28 slots at 88% load: 770 ->
+// 304 us a launch; 5,000 from 2^24 slots: 33 -> 17 us (only blocks that change
+// are stored).  Slots in 16 bits with their flags need no bound on the shift;
+// reading the caps again in the second pass instead of keeping them would
+// cost 64 more LDS reads a lane.
+struct DeleteSmem {
+  uint32_t sin[64 * 17 + 4];  // old slots: slot p at byte sin_off(p) (+ 4: read_slots8 reads ahead)
+  union {
+    uint16_t quot[64 * 64 + 64];  // twice the k-th occupied quotient, kNoQuot past the last
+    uint32_t out[64 * 33];        // new slots, 16 bits each: byte | last of its run << 8 | unused << 15
+  };
+  uint64_t occ_in[64];
+  uint64_t run_in[64];
+  uint64_t run_out[64];
+  uint32_t rem[128];     // removed slots, 32 a word
+  uint64_t merged[64];   // quotients whose run was rewritten in place
+  int32_t xold[65];
+  int32_t xnew[65];
+  uint64_t rewritten;    // blocks with slots of such runs
+  uint32_t invalid;      // a run that ends past the window was touched
+};
+constexpr uint32_t kNoQuot = 0xFFFEu;
+
+__device__ __forceinline__ uint64_t brev64(uint64_t x) { return __brevll(x); }
+
+__device__ __forceinline__ int rebuild_delete(const QF& qf, uint64_t r, const uint64_t* __restrict__ items, uint64_t s,
+                                              uint64_t e, DeleteSmem& sm) {
+  const int lane = lane_id();
+  const int j = lane;
+  const int R = (int)qf.region_blocks;
+  const uint64_t B0 = r * (uint64_t)R;
+  const int nwin = window_blocks(qf, r, kWinFast, true);
+  const bool table_end = B0 + (uint64_t)nwin >= qf.nblocks;
+  const uint64_t base = B0 << 14;
+
+  // ---- the window
+  uint64_t occ = 0, run = 0, used = 0;
+  uint32_t off = 0;
+  {
+    const GQF_GLOBAL uint4* b = gqf_block_ptr(qf, B0) + (size_t)(j < nwin ? j : nwin - 1) * (GQF_BLOCK_BYTES / 16);
+    const uint4 h0 = b[0], h1 = b[1];
+    uint4 sl[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) sl[k] = b[4 + k];
+    if (j < nwin) {
+      occ = (uint64_t)h0.x | (uint64_t)h0.y << 32;
+      run = (uint64_t)h0.z | (uint64_t)h0.w << 32;
+      off = h1.x;
+      used = (uint64_t)h1.z | (uint64_t)h1.w << 32;
+    }
+    uint32_t* row = sm.sin + 17 * j;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      row[4 * k] = sl[k].x; row[4 * k + 1] = sl[k].y; row[4 * k + 2] = sl[k].z; row[4 * k + 3] = sl[k].w;
+    }
+  }
+  const int32_t x0 = (int32_t)__builtin_amdgcn_readfirstlane((int)off) - 1;
+  if (x0 + 1 > 64 * nwin) return kNeedWide;  // spill-in longer than the window
+  // run ends of the window's own quotients (slots [0, x0] are earlier regions')
+  const int32_t spill = x0 + 1 - 64 * j;
+  const uint64_t own_run = run & (spill <= 0 ? ~0ULL : (spill >= 64 ? 0ULL : ~0ULL << spill));
+  sm.occ_in[j] = occ;
+  sm.run_in[j] = run;
+  sm.xold[j] = 64 * j - 1 + (int32_t)off;
+  sm.merged[j] = 0;
+  sm.rem[j] = sm.rem[64 + j] = 0;
+  if (lane == 0) {
+    sm.invalid = 0;
+    sm.rewritten = 0;
+  }
+  const uint32_t n_occ = (uint32_t)__popcll(occ), n_run = (uint32_t)__popcll(own_run);
+  const uint32_t incl_occ = wave_scan_add(n_occ), rbase = wave_scan_add(n_run) - n_run;
+  {
+    // the occupied quotients by rank: a quotient without a run writes to a
+    // spare entry of its lane
+    const uint32_t ow[2] = {(uint32_t)occ, (uint32_t)(occ >> 32)};
+    uint32_t k = incl_occ - n_occ;
+    const uint32_t spare = 64 * 64 + (uint32_t)j;
+    auto put = [&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      const uint32_t m = bit_mask<i & 31>(ow[i >> 5]);
+      sm.quot[(k & m) | (spare & ~m)] = (uint16_t)(2 * (64 * j + i));
+      k -= m;  // m is 0 or -1
+    };
+    for_each_slot(put, std::make_integer_sequence<int, 64>{});
+  }
+  __syncthreads();
+  // past the last run: no quotient (entry incl_occ exists: at most 4096
+  // quotients are occupied, and the spare entries follow)
+  if (lane == 63) sm.quot[incl_occ] = (uint16_t)kNoQuot;
+  uint8_t* in = (uint8_t*)sm.sin;
+
+  // ---- the removed slots, an item a lane
+  for (uint64_t i = s; i < e; i += 64) {
+    const uint64_t ii = i + (uint64_t)lane;
+    const bool active = ii < e;
+    const uint32_t h = active ? (uint32_t)(items[ii] - base) : 0u;
+    const int32_t q = (int32_t)(h >> 8);
+    const uint32_t rr = h & 0xFFu;
+    int32_t st = 0;
+    uint32_t len = 0;
+    bool asc = true, done = false;
+    int32_t at = -1;  // the byte to remove
+    if (active) {
+      done = (sm.merged[q >> 6] >> (q & 63)) & 1ULL;
+      if (!locate_old_run(sm, nwin, q, st, len)) {
+        sm.invalid = 1;
+        len = 0;
+      }
+      if (len <= 8) {
+        uint32_t w0, w1;
+        read_slots8(sm, st, w0, w1);
+        uint32_t prev = 0;
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+          const uint32_t b = ((k < 4 ? w0 : w1) >> (8 * (k & 3))) & 0xFFu;
+          const bool inside = (uint32_t)k < len;
+          if (k > 0 && inside && b <= prev) asc = false;
+          if (inside && b == rr) at = st + k;
+          prev = b;
+        }
+      } else {
+        uint32_t prev = in[sin_off(st)];
+        if (prev == rr) at = st;
+        for (uint32_t k = 1; k < len; k++) {
+          const uint32_t b = in[sin_off(st + (int32_t)k)];
+          if (b <= prev) asc = false;
+          if (b == rr) at = st + (int32_t)k;
+          prev = b;
+        }
+      }
+    }
+    __syncthreads();  // every lane has read its run before one is rewritten
+    if (active && !done && len) {
+      if (asc) {
+        if (at >= 0) atomicOr(&sm.rem[at >> 5], 1u << (at & 31));
+      } else if (ii == s || (uint32_t)((items[ii - 1] - base) >> 8) != (uint32_t)q) {
+        // counters and the items of the quotient, both ascending
+        uint32_t rp = 0, wp = 0;
+        uint64_t it = ii;
+        auto old_slot = [&](uint32_t k) -> uint64_t { return in[sin_off(st + (int32_t)k)]; };
+        auto item = [&]() -> uint32_t {  // remainder of item `it`, 256 past the quotient's
+          if (it >= e) return 256u;
+          const uint64_t v = items[it] - base;
+          return (v >> 8) == (uint64_t)q ? (uint32_t)(v & 0xFFu) : 256u;
+        };
+        uint32_t nx = item();
+        while (rp < len) {
+          uint64_t rem, c;
+          const uint32_t last = gqf_decode_counter(old_slot, len, rp, &rem, &c);
+          while (nx < (uint32_t)rem) { it++; nx = item(); }
+          for (; nx == (uint32_t)rem; nx = item()) {
+            it++;
+            c -= c ? 1 : 0;
+          }
+          wp += gqf_emit_counter(rem, c, [&](uint32_t k, uint64_t v) {
+            in[sin_off(st + (int32_t)(wp + k))] = (uint8_t)v;
+          });
+          rp = last + 1;
+        }
+        for (uint32_t k = wp; k < len; k++) {
+          const int32_t p = st + (int32_t)k;
+          atomicOr(&sm.rem[p >> 5], 1u << (p & 31));
+        }
+        atomicOr((unsigned long long*)&sm.merged[q >> 6], 1ULL << (q & 63));
+        const int b0 = st >> 6, b1 = (st + (int32_t)len - 1) >> 6;
+        atomicOr((unsigned long long*)&sm.rewritten, range_mask(b0, b1 + 1));
+      }
+    }
+    __syncthreads();
+  }
+  if (sm.invalid) return kNeedWide;
+  const uint32_t rw[2] = {sm.rem[2 * j], sm.rem[2 * j + 1]};
+  const uint64_t rem = (uint64_t)rw[0] | (uint64_t)rw[1] << 32;
+  const bool touched = rem || ((sm.rewritten >> j) & 1ULL);
+  const uint64_t any = __ballot(touched);
+  if (!any) return kOk;  // every item was absent
+
+  // ---- last kept bytes of runs, and runs without any
+  const uint64_t keep = used & ~rem;
+  const uint64_t n = keep | run;  // kept slots and old run ends
+  const uint64_t x = run & rem;   // removed run ends
+  const uint64_t b_n = __ballot(n != 0);
+  // is the next such slot in later blocks a removed run end?  the last one in
+  // earlier blocks a run end (or none there)?
+  const uint64_t b_x = __ballot(n != 0 && (n & (0 - n) & x) != 0);
+  const uint64_t b_t = __ballot(n != 0 && ((run >> (63 - __builtin_clzll(n | 1ULL))) & 1ULL));
+  const uint64_t later = j < 63 ? b_n & (~0ULL << (j + 1)) : 0ULL, earlier = b_n & ((1ULL << j) - 1);
+  const uint64_t cx = later ? (b_x >> __builtin_ctzll(later)) & 1ULL : 0ULL;
+  const uint64_t ct = earlier ? (b_t >> (63 - __builtin_clzll(earlier))) & 1ULL : 1ULL;
+  // the slot of n before each slot of x (a carry runs through the slots
+  // between, from above), and the slot of n behind each run end
+  const uint64_t nr = brev64(n);
+  const uint64_t before_x = brev64((((brev64(x) << 1) | cx) + ~nr) & nr);
+  const uint64_t after_end = (((run << 1) | ct) + ~n) & n;
+  const uint64_t ends = keep & (run | before_x);
+  for (uint64_t dead = x & after_end; dead; dead &= dead - 1) {
+    const int b = __builtin_ctzll(dead);
+    const uint32_t k = rbase + (uint32_t)__popcll(own_run & ((1ULL << b) - 1));
+    const uint32_t q = (uint32_t)sm.quot[k] >> 1;
+    atomicAnd((unsigned long long*)&sm.occ_in[q >> 6], ~(1ULL << (q & 63)));
+  }
+
+  // ---- caps (twice the distance to the quotient), lane j's map, the scan
+  int32_t cap[64];
+  int32_t A = 1 << 24;
+  {
+    const uint32_t ew[2] = {(uint32_t)own_run, (uint32_t)(own_run >> 32)};
+    const uint8_t* qb = (const uint8_t*)sm.quot;
+    uint32_t k = 2 * rbase;
+    auto load = [&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      cap[i] = (int32_t)*(const uint16_t*)(qb + k);
+      k = twice_add(bit_u<i & 31>(ew[i >> 5]), k);
+    };
+    for_each_slot(load, std::make_integer_sequence<int, 64>{});
+    auto fold = [&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      cap[i] = 128 * j + 2 * i - cap[i];
+      A = cap_shift(A, cap[i]);
+      A = (int32_t)twice_add(bit_u<i & 31>(rw[i >> 5]), (uint32_t)A);
+    };
+    for_each_slot(fold, std::make_integer_sequence<int, 64>{});
+  }
+  int32_t ia = -A, ib = -2 * (int32_t)__popcll(rem);
+  wave_scan_compose(ia, ib);
+  const int32_t ea = wave_shr1(ia, kNegInf), eb = wave_shr1(ib, 0);
+  const int32_t e_in = ea > eb ? -ea : -eb;  // twice the shift that enters block j
+
+  // ---- b*: the first block at or after R, behind the last touched slot,
+  // that no shift reaches; blocks [0, b*) are rewritten where they change
+  const int last = 63 - __builtin_clzll(any);
+  const uint64_t bm = __ballot(j >= R && j > last && j < nwin && e_in == 0);
+  if (!bm && !table_end) return kNeedWide;
+  const int bstar = bm ? __builtin_ctzll(bm) : nwin;
+  __syncthreads();
+
+  // ---- the kept bytes at their new slots
+  {
+    uint32_t* row = sm.out + 33 * j;
+#pragma unroll
+    for (int k = 0; k < 32; k++) row[k] = 0x80008000u;
+  }
+  __syncthreads();
+  {
+    uint32_t w[16];
+    const uint32_t* row = sm.sin + 17 * j;
+#pragma unroll
+    for (int k = 0; k < 16; k++) w[k] = row[k];
+    const uint32_t kw[2] = {(uint32_t)keep, (uint32_t)(keep >> 32)};
+    const uint32_t lw[2] = {(uint32_t)ends, (uint32_t)(ends >> 32)};
+    uint8_t* dst = (uint8_t*)sm.out;
+    const uint32_t spare = 132u * (uint32_t)j + 128u;  // the row's pad
+    int32_t sh = e_in;
+    auto move = [&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      sh = cap_shift(sh, cap[i]);
+      const uint32_t p = (uint32_t)(128 * j + 2 * i - sh);
+      const uint32_t to = p + ((p >> 7) << 2);
+      const uint32_t m = bit_mask<i & 31>(kw[i >> 5]);
+      const uint32_t b = (w[i >> 2] >> (8 * (i & 3))) & 0xFFu;
+      *(uint16_t*)(dst + ((to & m) | (spare & ~m))) = (uint16_t)lshl_or_c<8>(bit_u<i & 31>(lw[i >> 5]), b);
+      sh = (int32_t)twice_add(bit_u<i & 31>(rw[i >> 5]), (uint32_t)sh);
+    };
+    for_each_slot(move, std::make_integer_sequence<int, 64>{});
+  }
+  __syncthreads();
+
+  // ---- block j's new words
+  uint32_t nb[16];
+  uint64_t run_new = 0, used_new = 0;
+  {
+    const uint32_t* row = sm.out + 33 * j;
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      const uint32_t a = row[4 * k], b = row[4 * k + 1], c = row[4 * k + 2], d = row[4 * k + 3];
+      nb[2 * k] = __builtin_amdgcn_perm(b, a, 0x06040200);
+      nb[2 * k + 1] = __builtin_amdgcn_perm(d, c, 0x06040200);
+      const uint32_t f0 = __builtin_amdgcn_perm(b, a, 0x07050301), f1 = __builtin_amdgcn_perm(d, c, 0x07050301);
+      const uint32_t last8 = __builtin_amdgcn_udot4(
+          f1 & 0x01010101u, 0x80402010u, __builtin_amdgcn_udot4(f0 & 0x01010101u, 0x08040201u, 0u, false), false);
+      const uint32_t empty8 = __builtin_amdgcn_udot4((f1 >> 7) & 0x01010101u, 0x80402010u,
+                                                     __builtin_amdgcn_udot4((f0 >> 7) & 0x01010101u, 0x08040201u, 0u, false),
+                                                     false);
+      run_new |= (uint64_t)last8 << (8 * k);
+      used_new |= (uint64_t)(empty8 ^ 0xFFu) << (8 * k);
+    }
+  }
+  sm.run_out[j] = run_new;
+  const uint64_t occ_new = j < nwin ? sm.occ_in[j] : 0ULL;
+  __syncthreads();
+  const uint32_t off_new = offset_by_rank(sm, nwin, bstar, occ_new);
+  // an untouched block that no shift enters keeps its slots (its last run may
+  // have lost what it had in the next block)
+  if (j < bstar && (touched || e_in || occ_new != occ || off_new != off || run_new != run)) {
+    GQF_GLOBAL uint4* b = gqf_gptr_mut((uint4*)(qf.blocks + B0 * GQF_BLOCK_BYTES)) + (size_t)j * (GQF_BLOCK_BYTES / 16);
+    b[0] = make_uint4((uint32_t)occ_new, (uint32_t)(occ_new >> 32), (uint32_t)run_new, (uint32_t)(run_new >> 32));
+    b[1] = make_uint4(off_new, 0, (uint32_t)used_new, (uint32_t)(used_new >> 32));
+#pragma unroll
+    for (int k = 0; k < 4; k++) b[4 + k] = make_uint4(nb[4 * k], nb[4 * k + 1], nb[4 * k + 2], nb[4 * k + 3]);
   }
   return kOk;
 }
@@ -1679,6 +1960,22 @@ gqf_rebuild_flat(const QF* __restrict__ qfp, const uint64_t* __restrict__ items,
     if (res == gqf_flat::kNeedWide) flag_wide(r, wide_flags, wide_count);
     else if (res == gqf_flat::kNoSpace) atomicOr(qf.status, GQF_STATUS_NO_SPACE);
   }
+}
+
+extern "C" __global__ void __launch_bounds__(64)
+gqf_rebuild_delete(const QF* __restrict__ qfp, const uint64_t* __restrict__ items,
+                   const uint32_t* __restrict__ region_start, const uint32_t* __restrict__ region_list,
+                   const uint32_t* __restrict__ list_count, int parity, uint8_t* __restrict__ wide_flags,
+                   uint32_t* __restrict__ wide_count) {
+  __shared__ DeleteSmem sm;
+  const QF qf = *qfp;
+  if (blockIdx.x >= list_count[parity]) return;
+  const uint64_t r = region_list[blockIdx.x];
+  if (r >= qf.nregions) return;
+  const uint64_t s = region_start[r], e = region_start[r + 1];
+  if (s == e) return;
+  const int res = rebuild_delete(qf, r, items, s, e, sm);
+  if (res == kNeedWide && lane_id() == 0) flag_wide(r, wide_flags, wide_count);
 }
 
 // Redoes flagged regions of one parity with a wider window: 128 blocks,
@@ -2199,11 +2496,14 @@ void gqf_launch_rebuild(const QF* qf_dev, uint64_t nregions, uint64_t region_blo
     abort();
   }
   const int kind = mode == kSeq ? gqf_flat::kTagged : (counts ? gqf_flat::kCounts : gqf_flat::kAdd);
-  const bool flat = mode != kDelete && n_items >= (kind == gqf_flat::kAdd ? kFlatItems : kFlatItemsMixed) * nregions;
+  const bool flat = n_items >= (kind == gqf_flat::kAdd ? kFlatItems : kFlatItemsMixed) * nregions;
   mode |= gqf_rebuild_mode_flags();
   for (int parity = 0; parity < 2; parity++) {
     gqf_prof_begin("rebuild_phase", s);
-    if (flat)
+    if ((mode & ~GQF_REBUILD_NO_SHIFT) == kDelete)
+      hipLaunchKernelGGL(gqf_rebuild_delete, dim3(g), dim3(64), 0, s, qf_dev, items, region_start,
+                         region_list + (size_t)parity * stride, list_count, parity, wide_flags, wide_count);
+    else if (flat)
       hipLaunchKernelGGL(gqf_rebuild_flat, dim3(g), dim3(gqf_flat::kThreads), 0, s, qf_dev, items, counts, region_start,
                          region_list + (size_t)parity * stride, list_count, parity, kind, wide_flags, wide_count);
     else if (counts || (mode & ~GQF_REBUILD_NO_SHIFT) == kSeq)

@@ -1,7 +1,10 @@
-"""The workgroup-wide rebuild of dense batches, on small tables against the spec model's canonical image of the multiset: batches on
+"""The workgroup-wide rebuild of dense batches and the delete path, on small
+tables against the spec model's canonical image of the multiset: batches on
 both sides of the density where a table changes path, counters of one to
 several slots (counts from 1 past 4095, more big ones in a window than its
-table of them holds).  Every test prints its case before it touches
+table of them holds), runs that cross blocks, deletes that empty runs, that
+rewrite counters in place without moving a byte, and that take a run's last
+byte out of the next block.  Every test prints its case before it touches
 the GPU."""
 import numpy as np
 import pytest
@@ -93,6 +96,61 @@ def test_dense_big_counts(gpu, nbig):
         for part in (np.repeat(univ, counts), np.repeat(univ[::2], 2), univ):
             f.bulk_insert(to_device_u64(rng.permutation(part)), flags=KEY_IS_HASH)
             _apply(ms, part, 1)
+            _check(f, q, ms)
+    finally:
+        f.close()
+
+
+@pytest.mark.parametrize("q,load,repeat", [(9, 0.9, 0.0), (10, 0.6, 0.5), (12, 0.9, 0.0), (12, 0.85, 0.2), (13, 0.5, 0.9)])
+def test_delete_batches(gpu, q, load, repeat):
+    """Deletes of one key, a few, a third with repeats and absent keys, then
+    the rest."""
+    from cqf_amd.gqf import GQF, to_device_u64
+    _say(f"case delete q={q} load={load} repeat={repeat}")
+    rng = np.random.default_rng(int(100 * load) + q)
+    n = int(load * (1 << q))
+    univ = rng.permutation(1 << (q + 8))[:max(1, int(n * (1 - repeat) * (0.6 if repeat else 1)))].astype(np.uint64)
+    hs = np.concatenate([univ, univ[rng.integers(0, univ.size, size=max(0, int(0.5 * n * repeat)))]])
+    f = GQF(q)
+    ms = {}
+    try:
+        f.bulk_insert(to_device_u64(hs), flags=KEY_IS_HASH)
+        _apply(ms, hs, 1)
+        _check(f, q, ms)
+        left = rng.permutation(hs)
+        for k in (1, 7, 100, left.size // 3, left.size):
+            batch, left = left[:k], left[k:]
+            absent = rng.integers(0, 1 << (q + 8), size=k // 4, dtype=np.uint64)
+            batch = rng.permutation(np.concatenate([batch, absent]))
+            f.bulk_delete(to_device_u64(batch), flags=KEY_IS_HASH)
+            _apply(ms, batch, -1)
+            _check(f, q, ms)
+    finally:
+        f.close()
+
+
+@pytest.mark.parametrize("home", [0, 60, 63, 64, 3071, 3072])
+def test_delete_single_places(gpu, home):
+    """One change at a time around a block's and a region's end: a count
+    lowered in place (300 -> 299), a two-slot counter halved, a run's last
+    byte removed from the next block, a run emptied in front of pushed ones."""
+    from cqf_amd.gqf import GQF, to_device_u64
+    q = 12
+    _say(f"case delete places {home}")
+    hs = [(home << 8) | 5] * 300 + [(home << 8) | r for r in (9, 9, 40)]
+    hs += [((home + k) << 8) | r for k in range(1, 7) for r in (1, 200, 255)]
+    hs = np.array(hs, dtype=np.uint64)
+    f = GQF(q)
+    ms = {}
+    try:
+        f.bulk_insert(to_device_u64(hs), flags=KEY_IS_HASH)
+        _apply(ms, hs, 1)
+        _check(f, q, ms)
+        for gone in ([(home << 8) | 5], [(home << 8) | 9], [((home + 1) << 8) | 255], [((home + 6) << 8) | 255],
+                     [((home + 2) << 8) | r for r in (1, 200, 255)], [(home << 8) | 5] * 299 + [(home << 8) | 7]):
+            g = np.array(gone, dtype=np.uint64)
+            f.bulk_delete(to_device_u64(g), flags=KEY_IS_HASH)
+            _apply(ms, g, -1)
             _check(f, q, ms)
     finally:
         f.close()
