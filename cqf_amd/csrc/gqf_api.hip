@@ -41,7 +41,7 @@ struct Workspace {
   uint64_t cap = 0;            // keys the buffers below are sized for
   uint64_t* tmp = nullptr;     // sort ping-pong, cap keys
   uint32_t* hist = nullptr;    // [digit][tile]
-  uint32_t* totals = nullptr;  // 1024 digit totals
+  uint32_t* totals = nullptr;  // GQF_SORT_TOTALS words: digit totals, bucket starts
   uint32_t* slow_buckets = nullptr;  // flags of the two-level sort, kept zero by its kernels
   uint32_t* tile_heads = nullptr;
   uint64_t* ukeys = nullptr;   // run-length reduce outputs, cap keys each
@@ -109,7 +109,7 @@ void free_workspace(Workspace& w) {
 // the per-table part of a workspace: region tables of the rebuild
 void init_region_workspace(Workspace& w, uint64_t nblocks) {
   if (!w.totals) {
-    dev_alloc(&w.totals, 1024);
+    dev_alloc(&w.totals, GQF_SORT_TOTALS);
     dev_alloc(&w.slow_buckets, GQF_SORT_MAX_BUCKETS);
     GQF_CHECK(hipMemset(w.slow_buckets, 0, GQF_SORT_MAX_BUCKETS * sizeof(uint32_t)));
     dev_alloc(&w.m_dev, 1);
@@ -227,6 +227,26 @@ void mutate(QF* qf, uint64_t n, uint64_t* keys, uint8_t flags, int mode, bool re
   run_mutation(f, f->ws, n, keys, flags, mode, reduce, s);
 }
 
+// the regions of a sorted batch in the workspace's tables: all of them, or
+// only those with keys, listed (see gqf_launch.h)
+gqf_region_args all_regions(const Filter* f, const Workspace& w) {
+  gqf_region_args ra;
+  ra.start = w.region_start;
+  ra.step = f->host.region_blocks << 14;
+  ra.nregions = f->host.nregions;
+  ra.range = f->host.range;
+  return ra;
+}
+gqf_list_args listed_regions(const Filter* f, const Workspace& w) {
+  gqf_list_args la;
+  la.list = w.region_list;
+  la.count = w.list_count;
+  la.start = w.region_start;
+  la.stride = (f->host.nregions + 1) / 2 + 1;
+  la.region_blocks = (uint32_t)f->host.region_blocks;
+  return la;
+}
+
 // The bulk pipeline of one batch (n <= GQF_MAX_PIECE) on a workspace sized
 // for it; allocates nothing itself (the counting reduce allocates its table
 // on first use, so reduce batches take workspaces that may allocate).
@@ -244,18 +264,19 @@ void run_mutation(Filter* f, Workspace& w, uint64_t n, uint64_t* keys, uint8_t f
     GQF_CHECK(hipGetLastError());
     return;
   }
-  // the two-level sort also writes the region starts of a plain batch
-  // (reduce batches index their distinct keys instead)
-  const bool two_level = hash_it && gqf_sort_two_level_fits(n, bits);
-  if (two_level) {
-    gqf_region_args ra;
-    ra.start = w.region_start;
-    ra.step = f->host.region_blocks << 14;
-    ra.nregions = f->host.nregions;
-    ra.range = f->host.range;
-    gqf_launch_sort_two_level(keys, w.tmp, n, gqf_mask(f->host.key_bits), vb, bits, w.hist, w.totals,
-                              w.slow_buckets, s, reduce ? nullptr : &ra);
-  } else
+  // the fast sort also finds the regions of a plain batch (reduce batches
+  // index their distinct keys instead)
+  // (a reduce batch of middling size most likely repeats its keys, which
+  // would put many of them into one bucket: it keeps the LSD sort)
+  const bool fast = hash_it && gqf_sort_fast_fits(n, bits, false) &&
+                    !(reduce && n > GQF_SORT_TINY && n < (1ULL << 20));
+  const bool listed = n < f->host.nregions || n <= GQF_SORT_TINY;
+  const gqf_region_args ra = all_regions(f, w);
+  const gqf_list_args la = listed_regions(f, w);
+  if (fast)
+    gqf_launch_sort_fast(keys, w.tmp, n, false, gqf_mask(f->host.key_bits), vb, bits, w.hist, w.totals, w.slow_buckets,
+                         s, reduce || listed ? nullptr : &ra, !reduce && listed ? &la : nullptr);
+  else
     gqf_launch_sort(keys, w.tmp, n, hash_it ? 1 : (vb ? 2 : 0), gqf_mask(f->host.key_bits), vb, bits, f->sort_digit,
                     w.hist, w.totals, s);
   // A sparse insert batch -- at most one key per point-lock region and one
@@ -278,13 +299,11 @@ void run_mutation(Filter* f, Workspace& w, uint64_t n, uint64_t* keys, uint8_t f
     counts = w.ucounts;
     n_dev = w.m_dev;
   }
-  if (two_level && !reduce)
-    gqf_launch_region_lists(f->dev, f->host.nregions, n, w.region_start, w.region_list, w.list_count, s);
-  else
-    gqf_launch_region_bounds(f->dev, f->host.nregions, items, n, n_dev, w.region_start, w.region_list,
-                             w.list_count, ~0ULL, s);
-  gqf_launch_rebuild(f->dev, f->host.nregions, f->host.region_blocks, items, counts, n, w.region_start,
-                     w.region_list, w.list_count, mode, w.wide_flags, w.wide_count, s);
+  uint32_t* list = listed ? w.region_list : nullptr;
+  if (!fast || reduce)
+    gqf_launch_region_bounds(f->dev, f->host.nregions, items, n, n_dev, w.region_start, list, w.list_count, ~0ULL, s);
+  gqf_launch_rebuild(f->dev, f->host.nregions, f->host.region_blocks, items, counts, n, w.region_start, list,
+                     w.list_count, mode, w.wide_flags, w.wide_count, s);
   GQF_CHECK(hipGetLastError());
 }
 
@@ -569,7 +588,7 @@ constexpr uint64_t na_round(uint64_t b) { return (b + kNoAllocAlign - 1) / kNoAl
 // sub-buffers, in order
 constexpr uint64_t kNaTmp = na_round(kNoAllocMaxKeys * 8);
 constexpr uint64_t kNaHist = na_round(1024ULL * (kNoAllocMaxKeys / 4096 + 64) * 4);  // gqf_sort_hist_words(max) words
-constexpr uint64_t kNaTotals = na_round(1024 * 4);
+constexpr uint64_t kNaTotals = na_round(GQF_SORT_TOTALS * 4);
 constexpr uint64_t kNaSlow = na_round(GQF_SORT_MAX_BUCKETS * 4);
 constexpr uint64_t kNaStart = na_round((kNoAllocMaxRegions + 2) * 4);
 constexpr uint64_t kNaList = na_round(2 * ((kNoAllocMaxRegions + 1) / 2 + 1) * 4);
@@ -712,14 +731,23 @@ extern "C" int qf_bulk_mutate_seq(QF* qf, uint64_t n, uint64_t* keys, uint32_t n
   Workspace& w = f->ws;
   const hipStream_t s = (hipStream_t)stream;
   gqf_launch_seq_tag(f->dev, keys, n, reqs, s);
-  // hash bits only: the tags above bit 48 ride along, and the passes are
-  // stable, so each hash's items stay in request order
-  gqf_launch_sort(keys, w.tmp, n, 0, 0, 0, (int)(f->host.key_bits + f->host.value_bits), f->sort_digit, w.hist,
-                  w.totals, s);
-  gqf_launch_region_bounds(f->dev, f->host.nregions, keys, n, nullptr, w.region_start, w.region_list, w.list_count,
-                           GQF_SEQ_HASH_MASK, s);
+  const int bits = (int)(f->host.key_bits + f->host.value_bits);
+  const bool listed = n < f->host.nregions || n <= GQF_SORT_TINY;
+  uint32_t* list = listed ? w.region_list : nullptr;
+  if (gqf_sort_fast_fits(n, bits, true)) {
+    const gqf_region_args ra = all_regions(f, w);
+    const gqf_list_args la = listed_regions(f, w);
+    gqf_launch_sort_fast(keys, w.tmp, n, true, 0, 0, bits, w.hist, w.totals, w.slow_buckets, s, listed ? nullptr : &ra,
+                         listed ? &la : nullptr);
+  } else {
+    // hash bits only: the tags above bit 48 ride along, and the passes are
+    // stable, so each hash's items stay in request order
+    gqf_launch_sort(keys, w.tmp, n, 0, 0, 0, bits, f->sort_digit, w.hist, w.totals, s);
+    gqf_launch_region_bounds(f->dev, f->host.nregions, keys, n, nullptr, w.region_start, list, w.list_count,
+                             GQF_SEQ_HASH_MASK, s);
+  }
   gqf_launch_rebuild(f->dev, f->host.nregions, f->host.region_blocks, keys, nullptr, n, w.region_start,
-                     w.region_list, w.list_count, GQF_REBUILD_SEQ, w.wide_flags, w.wide_count, s);
+                     list, w.list_count, GQF_REBUILD_SEQ, w.wide_flags, w.wide_count, s);
   GQF_CHECK(hipGetLastError());
   return 0;
 }

@@ -277,9 +277,9 @@ void enqueue_insert(Group* g, const gqf_group_dev& dev, uint64_t* keys, uint64_t
         if (load[j] < load[k]) k = j;
       load[k] += m;
       const QF& d = g->h_descs[f];
-      gqf_launch_sort_two_level(keys + a, g->tmp + a, m, gqf_mask(d.key_bits), (int)d.value_bits,
+      gqf_launch_sort_fast(keys + a, g->tmp + a, m, false, gqf_mask(d.key_bits), (int)d.value_bits,
                                 (int)(d.key_bits + d.value_bits), g->bhist[k], g->btotals[k], g->bslow[k],
-                                g->side[k], nullptr, (uint64_t)f << dev.tag_shift);
+                                g->side[k], nullptr, nullptr, (uint64_t)f << dev.tag_shift);
     }
     for (int k = 0; k < kSortBranches; k++) {
       GCHECK(hipEventRecord(g->join[k], g->side[k]));
@@ -317,10 +317,10 @@ extern "C" int gqf_group_create(gqf_group** out, QF* const* filters, uint32_t nf
   dalloc(&g->d_descs, nfilters);
   dalloc(&g->d_tab, 4 * (size_t)(nfilters + 1));
   dalloc(&g->d_counters, 4);
-  dalloc(&g->totals, 1024);
+  dalloc(&g->totals, GQF_SORT_TOTALS);
   bool ok = true;
   for (int k = 0; k < kSortBranches; k++) {
-    dalloc(&g->btotals[k], 1024);
+    dalloc(&g->btotals[k], GQF_SORT_TOTALS);
     dalloc(&g->bslow[k], GQF_SORT_MAX_BUCKETS);
     ok = ok && g->btotals[k] && g->bslow[k];
     if (g->bslow[k]) GCHECK(hipMemset(g->bslow[k], 0, GQF_SORT_MAX_BUCKETS * sizeof(uint32_t)));

@@ -13,31 +13,46 @@ uint64_t gqf_sort_hist_words(uint64_t n);
 // digit_bits: 6..10 fixes the radix digit (passes rounded up to even), 0 picks 4 passes
 void gqf_launch_sort(uint64_t* keys, uint64_t* tmp, uint64_t n, int hash_it, uint64_t mask, int vshift, int bits,
                      int digit_bits, uint32_t* hist, uint32_t* totals, hipStream_t s);
-// the same result for keys to be hashed (hash_it 1), for batches where
-// gqf_sort_two_level_fits: one stable pass on the top hash bits into
-// buckets of about 12K keys, then an LDS sort per bucket; not stable on
-// equal hashes (plain keys only: equal hashes are indistinguishable)
 // the low bits gqf_launch_sort orders for these arguments (passes x digit,
 // at least `bits`): bits above them ride along in their stable order
 int gqf_sort_width(int bits, int digit_bits);
-bool gqf_sort_two_level_fits(uint64_t n, int bits);
+#define GQF_SORT_TOTALS 2048  // words of the `totals` buffer: digit totals, then bucket starts
 // slow: GQF_SORT_MAX_BUCKETS flags, zero between calls (the kernels leave them so)
 #define GQF_SORT_MAX_BUCKETS 1024
-// Region starts from the bucket sort (optional): for every region r <
-// nregions whose bound r * step lies below range, start[r] = the first index
-// of the sorted keys at or above the bound (what gqf_region_bounds would
-// write); gqf_launch_region_lists then completes the table and the lists.
+// The regions of the sorted keys, in one of two forms.
+// All of them: for every region r <= nregions, start[r] = the first index of
+// the sorted keys at or above the bound r * step (n at a bound at or past
+// range, and at r = nregions): a rebuild over every region.
 struct gqf_region_args {
   uint32_t* start = nullptr;
   uint64_t step = 0;      // hash values per region: region_blocks << 14
   uint64_t nregions = 0;
   uint64_t range = 0;
 };
-// tag: ORed into every sorted key on its way out (a filter group's filter
-// index above the hash bits; the region starts are of the untagged hashes)
-void gqf_launch_sort_two_level(uint64_t* keys, uint64_t* tmp, uint64_t n, uint64_t mask, int vshift, int bits,
-                               uint32_t* hist, uint32_t* totals, uint32_t* slow, hipStream_t s,
-                               const gqf_region_args* regions = nullptr, uint64_t tag = 0);
+// Those with keys: regions in list[parity * stride ..], count[parity] of
+// them, start[r] and start[r + 1] written for the listed ones only.
+struct gqf_list_args {
+  uint32_t* list = nullptr;
+  uint32_t* count = nullptr;
+  uint32_t* start = nullptr;
+  uint64_t stride = 0;
+  uint32_t region_blocks = 1;
+};
+// the result of gqf_launch_sort for keys to be hashed (hash_it 1), or, with
+// `tagged`, for sequenced keys (hash bits below GQF_SEQ_SHIFT), for batches
+// where gqf_sort_fast_fits: one workgroup's LDS sort up to 8192 keys; above,
+// one split on the top hash bits into buckets and an LDS sort per bucket.
+// Hashed keys that compare equal are equal, and sequenced ones are ordered by
+// hash and request, so the order is the stable one.
+// tag (hashed keys): ORed into every sorted key on its way out (a filter
+// group's filter index above the hash bits; the regions are of the untagged
+// hashes).  At most one of regions (not with up to 8192 keys) and lists.
+#define GQF_SORT_TINY 8192  // keys one workgroup sorts
+bool gqf_sort_fast_fits(uint64_t n, int bits, bool tagged);
+void gqf_launch_sort_fast(uint64_t* keys, uint64_t* tmp, uint64_t n, bool tagged, uint64_t mask, int vshift, int bits,
+                          uint32_t* hist, uint32_t* totals, uint32_t* slow, hipStream_t s,
+                          const gqf_region_args* regions = nullptr, const gqf_list_args* lists = nullptr,
+                          uint64_t tag = 0);
 
 // Counting reduce of duplicate-heavy batches (gqf_agg.hip).  ctrl: 4 words
 // (distinct keys in the sample, distinct hashes, overflow flag, output
@@ -76,17 +91,11 @@ void gqf_launch_rle(const uint64_t* keys, uint64_t n, uint32_t* tile_heads, uint
                     uint64_t* upos, uint64_t* ucounts, uint64_t* m_dev, hipStream_t s);
 
 // region bounds of sorted items (count n, or *n_dev when n_dev is set),
-// plus the non-empty regions of each parity compacted into region_list
-// (2 lists of (nregions + 1) / 2 + 1 entries) with their counts
+// plus, with region_list, the non-empty regions of each parity compacted into
+// it (2 lists of (nregions + 1) / 2 + 1 entries) with their counts
 void gqf_launch_region_bounds(const QF* qf_dev, uint64_t nregions, const uint64_t* items, uint64_t n,
                               const uint64_t* n_dev, uint32_t* region_start, uint32_t* region_list,
                               uint32_t* list_count, uint64_t hmask, hipStream_t s);
-// region_start entries that gqf_launch_sort_two_level leaves (bounds at or
-// past range, and r = nregions: n) and the non-empty region lists, as
-// gqf_launch_region_bounds makes them
-void gqf_launch_region_lists(const QF* qf_dev, uint64_t nregions, uint64_t n, uint32_t* region_start,
-                             uint32_t* region_list, uint32_t* list_count, hipStream_t s);
-
 // Sequenced batches: a sorted item is its slot hash with the request tag
 // above GQF_SEQ_SHIFT -- the request's sequence number in bits 48..62 and
 // bit 63 set for a delete.  Even radix passes of any digit the sort takes
@@ -119,7 +128,8 @@ void gqf_launch_seq_adjust(const QF* qf_dev, const uint64_t* keys, uint64_t n, c
                            uint64_t* counts, const uint64_t* mut, uint64_t n_mut, hipStream_t s);
 
 // both even/odd phases (+ wide fallback passes) of a merge-rebuild over
-// the listed regions; n_items bounds the number of non-empty regions.
+// the listed regions (n_items bounds their number), or over all of them
+// where region_list is null (every entry of region_start is set).
 // wide_flags: one byte per region; wide_count: GQF_WIDE_WORDS words (the
 // number of regions flagged in a phase, the first GQF_WIDE_LIST of them, a
 // counter of finished wide workgroups, a ticket counter and one finished

@@ -1889,9 +1889,9 @@ __device__ __forceinline__ void flag_wide(uint64_t r, uint8_t* __restrict__ wide
 }
 
 // One workgroup per non-empty region of one parity: workgroup i takes
-// region list[i] (the list gqf_region_bounds compacted; count[parity]
-// entries), so a small batch launches only as many workgroups as it has
-// regions with items, and the hardware hands regions to workgroups as
+// region list[i] (count[parity] entries), so a small batch launches only as
+// many workgroups as it has regions with items (without a list it takes the
+// i-th region of its parity), and the hardware hands regions to workgroups as
 // earlier ones finish.  (A persistent grid that loads each region's window
 // while rebuilding the previous one measured slower: 6.6 against 7.5 G
 // inserts/s at 2^28 slots, with 168 registers against 85 and a static share
@@ -1905,8 +1905,8 @@ __device__ __forceinline__ void rebuild_phase_item(const QF* __restrict__ qfp, c
                                                    uint8_t* __restrict__ wide_flags, uint32_t* __restrict__ wide_count,
                                                    Smem<kWinFast>& sm, uint32_t* lcnt) {
   const QF qf = *qfp;
-  if (blockIdx.x >= list_count[parity]) return;
-  const uint64_t r = region_list[blockIdx.x];
+  if (region_list && blockIdx.x >= list_count[parity]) return;
+  const uint64_t r = region_list ? region_list[blockIdx.x] : 2 * (uint64_t)blockIdx.x + (uint64_t)parity;
   if (r >= qf.nregions) return;
   const uint64_t s = region_start[r], e = region_start[r + 1];
   if (s == e) return;
@@ -1950,8 +1950,8 @@ gqf_rebuild_flat(const QF* __restrict__ qfp, const uint64_t* __restrict__ items,
                  uint32_t* __restrict__ wide_count) {
   __shared__ gqf_flat::Smem sm;
   const QF qf = *qfp;
-  if (blockIdx.x >= list_count[parity]) return;
-  const uint64_t r = region_list[blockIdx.x];
+  if (region_list && blockIdx.x >= list_count[parity]) return;
+  const uint64_t r = region_list ? region_list[blockIdx.x] : 2 * (uint64_t)blockIdx.x + (uint64_t)parity;
   if (r >= qf.nregions) return;
   const uint64_t s = region_start[r], e = region_start[r + 1];
   if (s == e) return;
@@ -1969,8 +1969,8 @@ gqf_rebuild_delete(const QF* __restrict__ qfp, const uint64_t* __restrict__ item
                    uint32_t* __restrict__ wide_count) {
   __shared__ DeleteSmem sm;
   const QF qf = *qfp;
-  if (blockIdx.x >= list_count[parity]) return;
-  const uint64_t r = region_list[blockIdx.x];
+  if (region_list && blockIdx.x >= list_count[parity]) return;
+  const uint64_t r = region_list ? region_list[blockIdx.x] : 2 * (uint64_t)blockIdx.x + (uint64_t)parity;
   if (r >= qf.nregions) return;
   const uint64_t s = region_start[r], e = region_start[r + 1];
   if (s == e) return;
@@ -2207,32 +2207,7 @@ gqf_region_bounds(const QF* __restrict__ qfp, const uint64_t* __restrict__ items
     region_start[r] = (uint32_t)lo;  // a wave's last lane repeats the next wave's first
     if (r == qf.nregions && lo < n) atomicOr(qf.status, GQF_STATUS_BAD_HASH);
   }
-  const uint64_t next = __shfl_down(lo, 1, 64);
-  const bool nonempty = valid && lane < (uint32_t)kBoundsPerWave && r < qf.nregions && next > lo;
-  append_region_lists(nonempty, r, region_list, list_count, list_stride);
-}
-
-// The region table after a two-level sort that wrote start[r] for every
-// region whose bound lies below range: the other entries (bounds at or past
-// range, and r = nregions) are n, and the non-empty regions are listed as
-// gqf_region_bounds lists them (same wave layout, no search).
-extern "C" __global__ void __launch_bounds__(kBoundsThreads)
-gqf_region_lists(const QF* __restrict__ qfp, uint64_t n, uint32_t* __restrict__ region_start,
-                 uint32_t* __restrict__ region_list, uint32_t* __restrict__ list_count, uint64_t list_stride) {
-  const QF qf = *qfp;
-  const uint32_t lane = threadIdx.x & 63;
-  const uint64_t wave = (uint64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  const uint64_t r = wave * kBoundsPerWave + lane;
-  const bool valid = r <= qf.nregions;
-  uint64_t lo = 0;
-  if (valid) {
-    if (r == qf.nregions || ((r * qf.region_blocks) << 14) >= qf.range) {
-      lo = n;
-      region_start[r] = (uint32_t)n;
-    } else {
-      lo = region_start[r];
-    }
-  }
+  if (!region_list) return;
   const uint64_t next = __shfl_down(lo, 1, 64);
   const bool nonempty = valid && lane < (uint32_t)kBoundsPerWave && r < qf.nregions && next > lo;
   append_region_lists(nonempty, r, region_list, list_count, list_stride);
@@ -2448,20 +2423,9 @@ void gqf_launch_region_bounds(const QF* qf_dev, uint64_t nregions, const uint64_
   const uint64_t waves = (nregions + 1 + kBoundsPerWave - 1) / kBoundsPerWave;
   const uint32_t g = (uint32_t)((waves + kBoundsThreads / 64 - 1) / (kBoundsThreads / 64));
   gqf_prof_begin("region_bounds", s);
-  hipLaunchKernelGGL(gqf_region_lists_reset, dim3(1), dim3(64), 0, s, list_count);
+  if (region_list) hipLaunchKernelGGL(gqf_region_lists_reset, dim3(1), dim3(64), 0, s, list_count);
   hipLaunchKernelGGL(gqf_region_bounds, dim3(g), dim3(kBoundsThreads), 0, s, qf_dev, items, n, n_dev, region_start,
                      region_list, list_count, (uint64_t)((nregions + 1) / 2 + 1), hmask);
-  gqf_prof_end("region_bounds", s);
-}
-
-void gqf_launch_region_lists(const QF* qf_dev, uint64_t nregions, uint64_t n, uint32_t* region_start,
-                             uint32_t* region_list, uint32_t* list_count, hipStream_t s) {
-  const uint64_t waves = (nregions + 1 + kBoundsPerWave - 1) / kBoundsPerWave;
-  const uint32_t g = (uint32_t)((waves + kBoundsThreads / 64 - 1) / (kBoundsThreads / 64));
-  gqf_prof_begin("region_bounds", s);
-  hipLaunchKernelGGL(gqf_region_lists_reset, dim3(1), dim3(64), 0, s, list_count);
-  hipLaunchKernelGGL(gqf_region_lists, dim3(g), dim3(kBoundsThreads), 0, s, qf_dev, n, region_start, region_list, list_count,
-                     (uint64_t)((nregions + 1) / 2 + 1));
   gqf_prof_end("region_bounds", s);
 }
 
@@ -2486,7 +2450,7 @@ void gqf_launch_rebuild(const QF* qf_dev, uint64_t nregions, uint64_t region_blo
   // at most one workgroup per non-empty region: no more than the regions
   // of a parity, nor than the items
   const uint64_t per_parity = (nregions + 1) / 2;
-  const uint32_t g = (uint32_t)(n_items < per_parity ? (n_items ? n_items : 1) : per_parity);
+  const uint32_t g = (uint32_t)(region_list && n_items < per_parity ? (n_items ? n_items : 1) : per_parity);
   const uint64_t stride = per_parity + 1;
   // classes of the wide pass (regions whose widest windows are disjoint)
   const uint32_t apart = (uint32_t)((kWinWide + region_blocks - 1) / region_blocks);
@@ -2499,19 +2463,20 @@ void gqf_launch_rebuild(const QF* qf_dev, uint64_t nregions, uint64_t region_blo
   const bool flat = n_items >= (kind == gqf_flat::kAdd ? kFlatItems : kFlatItemsMixed) * nregions;
   mode |= gqf_rebuild_mode_flags();
   for (int parity = 0; parity < 2; parity++) {
+    const uint32_t* list = region_list ? region_list + (size_t)parity * stride : nullptr;
     gqf_prof_begin("rebuild_phase", s);
     if ((mode & ~GQF_REBUILD_NO_SHIFT) == kDelete)
       hipLaunchKernelGGL(gqf_rebuild_delete, dim3(g), dim3(64), 0, s, qf_dev, items, region_start,
-                         region_list + (size_t)parity * stride, list_count, parity, wide_flags, wide_count);
+                         list, list_count, parity, wide_flags, wide_count);
     else if (flat)
       hipLaunchKernelGGL(gqf_rebuild_flat, dim3(g), dim3(gqf_flat::kThreads), 0, s, qf_dev, items, counts, region_start,
-                         region_list + (size_t)parity * stride, list_count, parity, kind, wide_flags, wide_count);
+                         list, list_count, parity, kind, wide_flags, wide_count);
     else if (counts || (mode & ~GQF_REBUILD_NO_SHIFT) == kSeq)
       hipLaunchKernelGGL(gqf_rebuild_phase_counts, dim3(g), dim3(64), 0, s, qf_dev, items, counts, region_start,
-                         region_list + (size_t)parity * stride, list_count, parity, mode, wide_flags, wide_count);
+                         list, list_count, parity, mode, wide_flags, wide_count);
     else
       hipLaunchKernelGGL(gqf_rebuild_phase, dim3(g), dim3(64), 0, s, qf_dev, items, region_start,
-                         region_list + (size_t)parity * stride, list_count, parity, mode, wide_flags, wide_count);
+                         list, list_count, parity, mode, wide_flags, wide_count);
     gqf_prof_end("rebuild_phase", s);
     gqf_prof_begin("rebuild_wide", s);
     hipLaunchKernelGGL(gqf_rebuild_wide, dim3(GQF_WIDE_LIST), dim3(64), 0, s, qf_dev, items, counts, region_start,

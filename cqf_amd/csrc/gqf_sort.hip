@@ -11,6 +11,8 @@
 // [digit][tile] matrix -> downsweep (stable rank with wave ballots, staged in
 // LDS so each digit's keys leave the tile as one contiguous run).
 // The first pass hashes on the fly.
+#include <type_traits>
+
 #include "gqf_internal.h"
 #include "gqf_launch.h"
 
@@ -272,91 +274,172 @@ constexpr int kMThreads = 1024;
 constexpr int kMWaves = kMThreads / 64;
 constexpr int kMItems = 8;
 constexpr uint32_t kMRound = kMThreads * kMItems;  // 8192 keys, 64 KB staged
+constexpr int kMItemsSmall = 2;                    // rounds of 2048 keys below kMSmallN: more, shorter tiles
+constexpr uint64_t kMSmallN = 1ULL << 18;
 constexpr int kMRankShift = 48;                    // ranks < kMRound ride above the hash bits
 static_assert(kMRound <= (1u << (64 - kMRankShift)), "rank fits above the hash");
 static_assert(kMaxRadix <= kMThreads, "one digit per thread");
+// Up to this many tiles, each scatter workgroup adds up its digits' counts
+// over the tiles before its own by itself ([tile][digit] histogram, read from
+// L2); more go through gqf_sort_scan_rows ([digit][tile])
+constexpr uint32_t kMScanTiles = 128;
+
+// The sorts below order by (hash bits, request tag) for sequenced keys (tag
+// above bit GQF_SEQ_SHIFT: sequence number, delete bit), which is the stable
+// order: a request's sequence number grows with its position, and equal
+// (hash, tag) are equal keys.  order_bits turns such a key's tag into 16 low
+// bits, sequence number first.
+__device__ __forceinline__ uint64_t seq_order(uint64_t hash_bits, uint64_t key) {
+  const uint32_t tag = (uint32_t)(key >> GQF_SEQ_SHIFT);
+  return hash_bits << 16 | ((tag << 1 | tag >> 15) & 0xFFFFu);
+}
+__device__ __forceinline__ uint64_t seq_tag_of(uint64_t order) {  // the tag in its place
+  const uint32_t r = (uint32_t)order & 0xFFFFu;
+  return (uint64_t)((r >> 1 | r << 15) & 0xFFFFu) << GQF_SEQ_SHIFT;
+}
 }  // namespace
 
-// per-tile digit histogram of the hashed keys -> hist[d * ntiles + tile]
-extern "C" __global__ void __launch_bounds__(kMThreads)
-gqf_msd_count(const uint64_t* __restrict__ in, uint64_t n, uint64_t tile_keys, int shift, int bits, uint64_t mask,
-              int vshift, uint32_t* __restrict__ hist, uint32_t ntiles) {
+// per-tile digit histogram of the hashed (kTagged: tagged) keys; workgroup 0
+// also clears the region list counts
+template <int ITEMS, bool kTagged>
+__device__ __forceinline__ void msd_count_body(const uint64_t* __restrict__ in, uint64_t n, uint64_t tile_keys,
+                                               int shift, int bits, uint64_t mask, int vshift,
+                                               uint32_t* __restrict__ hist, uint32_t ntiles,
+                                               uint32_t* __restrict__ list_count) {
+  constexpr uint32_t kRound = kMThreads * ITEMS;
   __shared__ uint32_t h[kMaxRadix];
   const int radix = 1 << bits;
   const int t = threadIdx.x;
   if (t < radix) h[t] = 0;
+  if (list_count && blockIdx.x == 0 && t < 2) list_count[t] = 0;
   __syncthreads();
   const uint64_t base = (uint64_t)blockIdx.x * tile_keys;
   const uint64_t end = min(n, base + tile_keys);
-  for (uint64_t r0 = base; r0 < end; r0 += kMRound) {
-    uint64_t key[kMItems];
+  for (uint64_t r0 = base; r0 < end; r0 += kRound) {
+    uint64_t key[ITEMS];
 #pragma unroll
-    for (int k = 0; k < kMItems; k++) {
-      const uint64_t i = r0 + (uint64_t)(k * kMThreads + t);
-      key[k] = i < end ? in[i] : 0;
-    }
+    for (int k = 0; k < ITEMS; k++) key[k] = in[min(r0 + (uint64_t)(k * kMThreads + t), end - 1)];
 #pragma unroll
-    for (int k = 0; k < kMItems; k++) {
+    for (int k = 0; k < ITEMS; k++) {
       const uint64_t i = r0 + (uint64_t)(k * kMThreads + t);
-      if (i < end) atomicAdd(&h[(uint32_t)((gqf_hash64(key[k], mask) << vshift) >> shift) & (radix - 1)], 1u);
+      const uint64_t v = kTagged ? key[k] : gqf_hash64(key[k], mask) << vshift;
+      if (i < end) atomicAdd(&h[(uint32_t)(v >> shift) & (radix - 1)], 1u);
     }
   }
   __syncthreads();
-  if (t < radix) hist[(uint64_t)t * ntiles + blockIdx.x] = h[t];
+  if (t < radix)
+    hist[ntiles <= kMScanTiles ? (uint64_t)blockIdx.x * (uint32_t)radix + (uint32_t)t : (uint64_t)t * ntiles + blockIdx.x] = h[t];
 }
 
-// scatter of one tile into the digit buckets (hist scanned per digit row,
-// bin_base the exclusive scan of the digit totals)
-extern "C" __global__ void __launch_bounds__(kMThreads, 8)
-gqf_msd_scatter(const uint64_t* __restrict__ in, uint64_t* __restrict__ out, uint64_t n, uint64_t tile_keys,
-                int shift, int bits, uint64_t mask, int vshift, const uint32_t* __restrict__ hist,
-                const uint32_t* __restrict__ bin_base, uint32_t ntiles) {
-  __shared__ uint64_t stage[kMRound];
+extern "C" __global__ void __launch_bounds__(kMThreads)
+gqf_msd_count(const uint64_t* __restrict__ in, uint64_t n, uint64_t tile_keys, int shift, int bits, uint64_t mask,
+              int vshift, uint32_t* __restrict__ hist, uint32_t ntiles, uint32_t* __restrict__ list_count) {
+  msd_count_body<kMItems, false>(in, n, tile_keys, shift, bits, mask, vshift, hist, ntiles, list_count);
+}
+extern "C" __global__ void __launch_bounds__(kMThreads)
+gqf_msd_count_small(const uint64_t* __restrict__ in, uint64_t n, uint64_t tile_keys, int shift, int bits, uint64_t mask,
+                    int vshift, uint32_t* __restrict__ hist, uint32_t ntiles, uint32_t* __restrict__ list_count) {
+  msd_count_body<kMItemsSmall, false>(in, n, tile_keys, shift, bits, mask, vshift, hist, ntiles, list_count);
+}
+extern "C" __global__ void __launch_bounds__(kMThreads)
+gqf_msd_count_tagged(const uint64_t* __restrict__ in, uint64_t n, uint64_t tile_keys, int shift, int bits, uint64_t mask,
+                     int vshift, uint32_t* __restrict__ hist, uint32_t ntiles, uint32_t* __restrict__ list_count) {
+  msd_count_body<kMItemsSmall, true>(in, n, tile_keys, shift, bits, mask, vshift, hist, ntiles, list_count);
+}
+
+// scatter of one tile into the digit buckets.  hist: the counts of
+// gqf_msd_count, or, above kMScanTiles tiles, its rows scanned per digit, with
+// the digit totals in `totals`.  starts[d] (written by workgroup 0) = first
+// index of digit d's keys.
+template <int ITEMS, bool kTagged>
+__device__ __forceinline__ void msd_scatter_body(const uint64_t* __restrict__ in, uint64_t* __restrict__ out,
+                                                 uint64_t n, uint64_t tile_keys, int shift, int bits, uint64_t mask,
+                                                 int vshift, const uint32_t* __restrict__ hist,
+                                                 const uint32_t* __restrict__ totals, uint32_t* __restrict__ starts,
+                                                 uint32_t ntiles) {
+  constexpr uint32_t kRound = kMThreads * ITEMS;
+  __shared__ uint64_t stage[kRound];
   __shared__ uint32_t cnt[kMaxRadix];     // keys of the round per digit
   __shared__ uint32_t lstart[kMaxRadix];  // their first index in stage
   __shared__ uint32_t glob[kMaxRadix];    // next output index of each digit
   __shared__ uint32_t wsum[kMWaves];
   const int radix = 1 << bits;
   const int t = threadIdx.x, w = t >> 6, lane = t & 63;
-  if (t < radix) glob[t] = bin_base[t] + hist[(uint64_t)t * ntiles + blockIdx.x];
+  // exclusive scan over the digits, one digit per thread (threads past the
+  // radix bring 0)
+  auto scan_digits = [&](uint32_t c) -> uint32_t {
+    const uint32_t incl = wave_scan_add(c);
+    __syncthreads();
+    if (lane == 63) wsum[w] = incl;
+    __syncthreads();
+    uint32_t before = incl - c;
+    for (int k = 0; k < w; k++) before += wsum[k];
+    return before;
+  };
+  {
+    uint32_t mine = 0, total = 0;  // digit t: keys in earlier tiles, in all
+    if (ntiles <= kMScanTiles) {
+      // the threads split into kMThreads / radix groups, each adding up every
+      // so-many-th tile
+      if (t < radix) cnt[t] = lstart[t] = 0;
+      __syncthreads();
+      const int d = t & (radix - 1), groups = kMThreads >> bits;
+      for (uint32_t i = (uint32_t)(t >> bits); i < ntiles; i += (uint32_t)groups) {
+        const uint32_t c = hist[(uint64_t)i * (uint32_t)radix + (uint32_t)d];
+        total += c;
+        mine += i < blockIdx.x ? c : 0u;
+      }
+      if (groups > 1) {
+        atomicAdd(&cnt[d], mine);
+        atomicAdd(&lstart[d], total);
+        __syncthreads();
+        mine = t < radix ? cnt[t] : 0u;
+        total = t < radix ? lstart[t] : 0u;
+      }
+    } else if (t < radix) {
+      mine = hist[(uint64_t)t * ntiles + blockIdx.x];
+      total = totals[t];
+    }
+    const uint32_t start = scan_digits(t < radix ? total : 0u);
+    if (t < radix) {
+      glob[t] = start + mine;
+      if (blockIdx.x == 0) starts[t] = start;
+    }
+  }
   const uint64_t base = (uint64_t)blockIdx.x * tile_keys;
   const uint64_t end = min(n, base + tile_keys);
-  for (uint64_t r0 = base; r0 < end; r0 += kMRound) {
+  for (uint64_t r0 = base; r0 < end; r0 += kRound) {
     // 32-bit offsets from the round's (uniform) base: one VGPR per address
     const uint64_t* __restrict__ src = in + r0;
-    const uint32_t m = (uint32_t)min((uint64_t)kMRound, end - r0);
+    const uint32_t m = (uint32_t)min((uint64_t)kRound, end - r0);
     if (t < radix) cnt[t] = 0;
     __syncthreads();
     // each key's rank within its digit rides in bits 48.. of the key (the
-    // hashes here are below 2^42), which keeps the kernel within 64 VGPRs
-    uint64_t key[kMItems];
+    // hashes here are below 2^42), which keeps the kernel within 64 VGPRs;
+    // tagged keys keep theirs beside them
+    uint64_t key[ITEMS];
+    uint32_t rank[kTagged ? ITEMS : 1];
 #pragma unroll
-    for (int k = 0; k < kMItems; k++) {
-      const uint32_t i = (uint32_t)(k * kMThreads + t);
-      key[k] = i < m ? src[i] : 0;
-    }
+    for (int k = 0; k < ITEMS; k++) key[k] = src[min((uint32_t)(k * kMThreads + t), m - 1)];
 #pragma unroll
-    for (int k = 0; k < kMItems; k++) {
+    for (int k = 0; k < ITEMS; k++) {
       const uint32_t i = (uint32_t)(k * kMThreads + t);
-      const uint64_t h = gqf_hash64(key[k], mask) << vshift;
-      const uint32_t rank = i < m ? atomicAdd(&cnt[(uint32_t)(h >> shift) & (radix - 1)], 1u) : 0u;
-      key[k] = h | ((uint64_t)rank << kMRankShift);
+      const uint64_t h = kTagged ? key[k] : gqf_hash64(key[k], mask) << vshift;
+      const uint32_t r = i < m ? atomicAdd(&cnt[(uint32_t)(h >> shift) & (radix - 1)], 1u) : 0u;
+      if (kTagged) rank[k] = r;
+      else key[k] = h | ((uint64_t)r << kMRankShift);
     }
     __syncthreads();
-    // exclusive scan of the digit counts, one digit per thread
     const uint32_t c = t < radix ? cnt[t] : 0u;
-    uint32_t incl = wave_scan_add(c);
-    if (lane == 63) wsum[w] = incl;
-    __syncthreads();
-    uint32_t before = 0;
-    for (int k = 0; k < w; k++) before += wsum[k];
-    if (t < radix) lstart[t] = before + incl - c;
+    const uint32_t first = scan_digits(c);
+    if (t < radix) lstart[t] = first;
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < kMItems; k++) {
+    for (int k = 0; k < ITEMS; k++) {
       const uint32_t i = (uint32_t)(k * kMThreads + t);
-      const uint64_t h = key[k] & ((1ULL << kMRankShift) - 1);
-      if (i < m) stage[lstart[(uint32_t)(h >> shift) & (radix - 1)] + (uint32_t)(key[k] >> kMRankShift)] = h;
+      const uint64_t h = kTagged ? key[k] : key[k] & ((1ULL << kMRankShift) - 1);
+      const uint32_t r = kTagged ? rank[k] : (uint32_t)(key[k] >> kMRankShift);
+      if (i < m) stage[lstart[(uint32_t)(h >> shift) & (radix - 1)] + r] = h;
     }
     __syncthreads();
     for (uint32_t i = t; i < m; i += kMThreads) {
@@ -369,8 +452,27 @@ gqf_msd_scatter(const uint64_t* __restrict__ in, uint64_t* __restrict__ out, uin
   }
 }
 
+extern "C" __global__ void __launch_bounds__(kMThreads, 8)
+gqf_msd_scatter(const uint64_t* __restrict__ in, uint64_t* __restrict__ out, uint64_t n, uint64_t tile_keys,
+                int shift, int bits, uint64_t mask, int vshift, const uint32_t* __restrict__ hist,
+                const uint32_t* __restrict__ totals, uint32_t* __restrict__ starts, uint32_t ntiles) {
+  msd_scatter_body<kMItems, false>(in, out, n, tile_keys, shift, bits, mask, vshift, hist, totals, starts, ntiles);
+}
+extern "C" __global__ void __launch_bounds__(kMThreads, 8)
+gqf_msd_scatter_small(const uint64_t* __restrict__ in, uint64_t* __restrict__ out, uint64_t n, uint64_t tile_keys,
+                      int shift, int bits, uint64_t mask, int vshift, const uint32_t* __restrict__ hist,
+                      const uint32_t* __restrict__ totals, uint32_t* __restrict__ starts, uint32_t ntiles) {
+  msd_scatter_body<kMItemsSmall, false>(in, out, n, tile_keys, shift, bits, mask, vshift, hist, totals, starts, ntiles);
+}
+extern "C" __global__ void __launch_bounds__(kMThreads, 8)
+gqf_msd_scatter_tagged(const uint64_t* __restrict__ in, uint64_t* __restrict__ out, uint64_t n, uint64_t tile_keys,
+                       int shift, int bits, uint64_t mask, int vshift, const uint32_t* __restrict__ hist,
+                       const uint32_t* __restrict__ totals, uint32_t* __restrict__ starts, uint32_t ntiles) {
+  msd_scatter_body<kMItemsSmall, true>(in, out, n, tile_keys, shift, bits, mask, vshift, hist, totals, starts, ntiles);
+}
+
 // ---------------------------------------------------------------------------
-// Two-level sort of hashed keys (batches of 2^20..2^24): the top-digit
+// Two-level sort of hashed or tagged keys (batches of up to 2^24): the top-digit
 // split above (gqf_msd_count / gqf_msd_scatter) puts the keys into 2^msd
 // buckets by their top `msd` hash bits; then one workgroup per bucket sorts the bucket's remaining
 // low bits (at most 32) in LDS -- up to kBucketCap keys as 32-bit values in
@@ -386,7 +488,7 @@ constexpr int kBWaves = kBThreads / 64;
 constexpr int kBItems = 8;                           // keys per lane per round
 constexpr uint32_t kBRound = kBThreads * kBItems;    // 8192
 constexpr uint32_t kBucketCap = 17408;               // 2^24 keys in 1024 buckets: mean 16384, sd 128
-constexpr int kBMaxPasses = 5;
+constexpr int kBMaxPasses = 7;
 
 struct BucketSmem {
   uint32_t buf[2][kBucketCap];
@@ -464,10 +566,11 @@ __device__ __forceinline__ void bucket_pass(const V* src, V* dst, uint32_t m, in
 // start[r] of the regions whose bounds lie in bucket b's hash range
 // [b << low_bits, (b + 1) << low_bits): the bucket's first index s plus
 // below(bound - bucket base), the number of its keys whose low bits are
-// below that (a bound at or past range is left to gqf_region_lists)
+// below that; the last bucket's workgroup also writes n at the bounds at or
+// past range and at r = nregions
 template <typename F>
-__device__ __forceinline__ void bucket_region_starts(const gqf_region_args& ra, uint32_t b, int low_bits, uint64_t s,
-                                                     F below) {
+__device__ __forceinline__ void bucket_region_starts(const gqf_region_args& ra, uint32_t b, uint32_t nbuckets,
+                                                     int low_bits, uint64_t s, uint64_t n, F below) {
   if (!ra.start) return;
   const uint64_t lo = (uint64_t)b << low_bits;
   const uint64_t hi = lo + (1ULL << low_bits);
@@ -478,6 +581,9 @@ __device__ __forceinline__ void bucket_region_starts(const gqf_region_args& ra, 
     const uint64_t bound = r * ra.step;
     if (bound < ra.range) ra.start[r] = (uint32_t)(s + below((uint32_t)(bound - lo)));
   }
+  if (b + 1 == nbuckets)
+    for (uint64_t r = (ra.range + ra.step - 1) / ra.step + threadIdx.x; r <= ra.nregions; r += blockDim.x)
+      ra.start[r] = (uint32_t)n;
 }
 
 // Common case, two workgroups per CU: the bucket's keys stay in registers
@@ -488,17 +594,52 @@ __device__ __forceinline__ void bucket_region_starts(const gqf_region_args& ra, 
 // index), so every key is written straight to its sorted position.  A
 // bucket above kBucketCap keys, or with a sub-bucket above kSubCap
 // (repeated keys), is flagged for gqf_sort_buckets_slow.
-constexpr int kBLoad = (int)((kBucketCap + kBThreads - 1) / kBThreads);  // 17
 constexpr int kSubBitsMax = 11;
 constexpr uint32_t kSubMax = 1u << kSubBitsMax;
 constexpr uint32_t kSubCap = 64;
 static_assert(kSubMax == 2 * kBThreads, "two sub-buckets per thread in the scan");
 
-extern "C" __global__ void __launch_bounds__(kBThreads)
-gqf_sort_buckets(const uint64_t* __restrict__ in, uint64_t* __restrict__ out, uint64_t n, int low_bits,
-                 const uint32_t* __restrict__ starts, uint32_t nbuckets, uint32_t* __restrict__ slow,
-                 gqf_region_args ra, uint64_t tag) {
-  __shared__ uint32_t buf[kBucketCap];
+// A key as the bucket sort orders it: the bucket's low bits, for tagged keys
+// with the 16 tag bits below them (8-byte values: kBucketCapTagged of them)
+constexpr uint32_t kBucketCapTagged = 8192;
+
+template <bool kTagged>
+struct BucketKey {
+  using V = std::conditional_t<kTagged, uint64_t, uint32_t>;
+  static constexpr uint32_t kCap = kTagged ? kBucketCapTagged : kBucketCap;
+  static constexpr int kLoad = (int)((kCap + kBThreads - 1) / kBThreads);
+  static constexpr int kExtra = kTagged ? 16 : 0;  // bits below the hash's
+  static __device__ __forceinline__ V of(uint64_t key, uint64_t hi) {
+    if constexpr (kTagged) return seq_order((key & GQF_SEQ_HASH_MASK) - hi, key);
+    else return (uint32_t)(key - hi);
+  }
+  static __device__ __forceinline__ uint64_t key(V v, uint64_t hi) {
+    if constexpr (kTagged) return hi | v >> 16 | seq_tag_of(v);
+    else return hi | v;
+  }
+  // `of` in two steps, the load by itself first (of an untagged key, its low
+  // word: the bucket's low bits are its low bits)
+  static __device__ __forceinline__ V load(const uint64_t* __restrict__ in, uint32_t i) {
+    if constexpr (kTagged) return in[i];
+    else return ((const uint32_t*)in)[2 * (size_t)i];
+  }
+  static __device__ __forceinline__ V loaded(V x, uint64_t hi, int low_bits) {
+    if constexpr (kTagged) return of(x, hi);
+    else return x & (0xFFFFFFFFu >> (32 - low_bits));
+  }
+  static __device__ __forceinline__ V bound(uint32_t x) { return (V)x << kExtra; }  // first value at low bits x
+};
+
+// Eight waves per SIMD (two workgroups a CU) need at most 80 SGPRs as well as
+// 64 VGPRs: with 82 one workgroup was resident, and 2^24 keys took 104 us in
+// place of 79 (hence the second launch bound).
+template <bool kTagged>
+__device__ __forceinline__ void sort_bucket(const uint64_t* __restrict__ in, uint64_t* __restrict__ out, uint64_t n,
+                                            int low_bits, const uint32_t* __restrict__ starts, uint32_t nbuckets,
+                                            uint32_t* __restrict__ slow, const gqf_region_args& ra, uint64_t tag) {
+  using K = BucketKey<kTagged>;
+  using V = typename K::V;
+  __shared__ V buf[K::kCap];
   __shared__ uint32_t sub_end[kSubMax];  // counts, then cursors: after the scatter, each sub-bucket's end
   __shared__ uint32_t wsum[kBWaves];
   __shared__ uint32_t oversize;
@@ -506,31 +647,31 @@ gqf_sort_buckets(const uint64_t* __restrict__ in, uint64_t* __restrict__ out, ui
   const uint64_t s = starts[b];
   const uint64_t e = b + 1 < nbuckets ? (uint64_t)starts[b + 1] : n;
   if (e <= s) {
-    bucket_region_starts(ra, b, low_bits, s, [](uint32_t) { return 0u; });
+    bucket_region_starts(ra, b, nbuckets, low_bits, s, n, [](uint32_t) { return 0u; });
     return;
   }
   const uint32_t m = (uint32_t)(e - s);
   const int t = threadIdx.x, w = t >> 6, lane = t & 63;
-  if (m > kBucketCap) {
+  if (m > K::kCap) {
     if (t == 0) slow[b] = 1;
     return;
   }
   const uint64_t hi = (uint64_t)b << low_bits;  // the bucket's top bits
   const int db = low_bits < kSubBitsMax ? low_bits : kSubBitsMax;
-  const int sb = low_bits - db;
+  const int sb = low_bits - db + K::kExtra;
   const uint32_t nsub = 1u << db;
   for (uint32_t d = t; d < nsub; d += kBThreads) sub_end[d] = 0;
   if (t == 0) oversize = 0;
-  uint32_t v[kBLoad];
+  // clamped indexes: every load is in flight before the first is used
+  V v[K::kLoad];
 #pragma unroll
-  for (int k = 0; k < kBLoad; k++) {
-    const uint32_t i = (uint32_t)(k * kBThreads + t);
-    v[k] = i < m ? (uint32_t)(in[s + i] - hi) : 0u;
-  }
+  for (int k = 0; k < K::kLoad; k++) v[k] = K::load(in + s, min((uint32_t)(k * kBThreads + t), m - 1));
+#pragma unroll
+  for (int k = 0; k < K::kLoad; k++) v[k] = K::loaded(v[k], hi, low_bits);
   __syncthreads();
 #pragma unroll
-  for (int k = 0; k < kBLoad; k++)
-    if ((uint32_t)(k * kBThreads + t) < m) atomicAdd(&sub_end[v[k] >> sb], 1u);
+  for (int k = 0; k < K::kLoad; k++)
+    if ((uint32_t)(k * kBThreads + t) < m) atomicAdd(&sub_end[(uint32_t)(v[k] >> sb)], 1u);
   __syncthreads();
   {  // exclusive scan of the counts, two sub-buckets per thread
     const uint32_t d0 = 2 * (uint32_t)t;
@@ -552,44 +693,189 @@ gqf_sort_buckets(const uint64_t* __restrict__ in, uint64_t* __restrict__ out, ui
     return;
   }
 #pragma unroll
-  for (int k = 0; k < kBLoad; k++)
-    if ((uint32_t)(k * kBThreads + t) < m) buf[atomicAdd(&sub_end[v[k] >> sb], 1u)] = v[k];
+  for (int k = 0; k < K::kLoad; k++)
+    if ((uint32_t)(k * kBThreads + t) < m) buf[atomicAdd(&sub_end[(uint32_t)(v[k] >> sb)], 1u)] = v[k];
   __syncthreads();
   for (uint32_t i = t; i < m; i += kBThreads) {
-    const uint32_t x = buf[i];
-    const uint32_t d = x >> sb;
+    const V x = buf[i];
+    const uint32_t d = (uint32_t)(x >> sb);
     const uint32_t st = d ? sub_end[d - 1] : 0u;
     const uint32_t en = sub_end[d];
     uint32_t r = 0;
     for (uint32_t j = st; j < en; j++) {
-      const uint32_t y = buf[j];
+      const V y = buf[j];
       r += (y < x || (y == x && j < i)) ? 1u : 0u;
     }
-    out[s + st + r] = tag | hi | x;
+    out[s + st + r] = tag | K::key(x, hi);
   }
-  bucket_region_starts(ra, b, low_bits, s, [&](uint32_t x) {
-    const uint32_t d = x >> sb;
+  bucket_region_starts(ra, b, nbuckets, low_bits, s, n, [&](uint32_t x) {
+    const V v0 = K::bound(x);
+    const uint32_t d = (uint32_t)(v0 >> sb);
     const uint32_t st = d ? sub_end[d - 1] : 0u, en = sub_end[d];
     uint32_t c = st;
-    for (uint32_t j = st; j < en; j++) c += buf[j] < x ? 1u : 0u;
+    for (uint32_t j = st; j < en; j++) c += buf[j] < v0 ? 1u : 0u;
     return c;
   });
 }
 
+extern "C" __global__ void __launch_bounds__(kBThreads, 8)
+gqf_sort_buckets(const uint64_t* __restrict__ in, uint64_t* __restrict__ out, uint64_t n, int low_bits,
+                 const uint32_t* __restrict__ starts, uint32_t nbuckets, uint32_t* __restrict__ slow,
+                 gqf_region_args ra, uint64_t tag) {
+  sort_bucket<false>(in, out, n, low_bits, starts, nbuckets, slow, ra, tag);
+}
+extern "C" __global__ void __launch_bounds__(kBThreads, 8)
+gqf_sort_buckets_tagged(const uint64_t* __restrict__ in, uint64_t* __restrict__ out, uint64_t n, int low_bits,
+                        const uint32_t* __restrict__ starts, uint32_t nbuckets, uint32_t* __restrict__ slow,
+                        gqf_region_args ra) {
+  sort_bucket<true>(in, out, n, low_bits, starts, nbuckets, slow, ra, 0);
+}
+
+// A bucket that repeats few keys (at most kTableMax distinct ones, however
+// many times each): its distinct values are counted in an LDS hash table, the
+// table is sorted, and every value is written as often as it came.  Returns
+// false, with nothing written, if there are more.
+constexpr uint32_t kTableCap = 8192;
+constexpr uint32_t kTableMax = 6144;
+struct BucketTable {
+  uint64_t val[kTableCap];  // ~0: free
+  uint32_t cnt[kTableCap];  // then the values' first output indexes
+  uint32_t wsum[kBWaves];
+  uint32_t used;
+};
+static_assert(sizeof(BucketTable) <= sizeof(BucketSmem), "shares the passes' LDS");
+
+template <bool kTagged>
+__device__ __forceinline__ bool sort_by_table(const uint64_t* in, uint64_t* out, uint64_t s, uint64_t n, uint32_t m,
+                                              int low_bits, uint32_t b, uint32_t nbuckets, BucketTable& tb,
+                                              const gqf_region_args& ra, uint64_t tag) {
+  using K = BucketKey<kTagged>;
+  const uint32_t t = threadIdx.x, w = t >> 6, lane = t & 63;
+  const uint64_t hi = (uint64_t)b << low_bits;
+  for (uint32_t i = t; i < kTableCap; i += kBThreads) {
+    tb.val[i] = ~0ULL;
+    tb.cnt[i] = 0;
+  }
+  if (t == 0) tb.used = 0;
+  __syncthreads();
+  for (uint32_t i0 = 0; i0 < m; i0 += kBThreads) {
+    if (*(volatile uint32_t*)&tb.used > kTableMax) break;  // checked again below
+    const uint32_t i = i0 + t;
+    bool left = i < m;
+    const uint64_t v = left ? (uint64_t)K::of(in[s + i], hi) : 0ULL;
+    // a wave's repeats of one value are added together (two values' worth,
+    // the rest one by one)
+    uint32_t add = left ? 1u : 0u;
+    uint64_t open = __ballot(left);
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+      if (!open) break;
+      const int first = __builtin_ctzll(open);
+      const uint64_t lead = __shfl(v, first, 64);
+      const uint64_t same = __ballot(((open >> lane) & 1) && v == lead);
+      if ((same >> lane) & 1) add = lane == (uint32_t)first ? (uint32_t)__popcll(same) : 0u;
+      open &= ~same;
+    }
+    if (add) {
+      uint32_t at = (uint32_t)((v * 0x9E3779B97F4A7C15ULL) >> 51);
+      for (uint32_t k = 0; k < kTableCap; k++) {
+        const uint64_t old = atomicCAS((unsigned long long*)&tb.val[at], ~0ULL, (unsigned long long)v);
+        if (old == ~0ULL) atomicAdd(&tb.used, 1u);
+        if (old == ~0ULL || old == v) {
+          atomicAdd(&tb.cnt[at], add);
+          break;
+        }
+        if (*(volatile uint32_t*)&tb.used > kTableMax) break;
+        at = (at + 1) & (kTableCap - 1);
+      }
+    }
+  }
+  __syncthreads();
+  if (tb.used > kTableMax) return false;
+  // bitonic, the free entries (~0) last
+  for (uint32_t k = 2; k <= kTableCap; k *= 2) {
+    for (uint32_t j = k / 2; j > 0; j /= 2) {
+      for (uint32_t i = t; i < kTableCap / 2; i += kBThreads) {
+        const uint32_t a = (i / j) * 2 * j + i % j, c = a + j;
+        const uint64_t x = tb.val[a], y = tb.val[c];
+        if ((x > y) == ((a & k) == 0)) {
+          tb.val[a] = y;
+          tb.val[c] = x;
+          const uint32_t z = tb.cnt[a];
+          tb.cnt[a] = tb.cnt[c];
+          tb.cnt[c] = z;
+        }
+      }
+      __syncthreads();
+    }
+  }
+  // counts -> first indexes, eight entries a thread
+  constexpr int kE = kTableCap / kBThreads;
+  uint32_t c[kE], sum = 0;
+#pragma unroll
+  for (int k = 0; k < kE; k++) {
+    c[k] = tb.cnt[kE * t + (uint32_t)k];
+    sum += c[k];
+  }
+  const uint32_t incl = wave_scan_add(sum);
+  if (lane == 63) tb.wsum[w] = incl;
+  __syncthreads();
+  uint32_t run = incl - sum;
+  for (uint32_t k = 0; k < w; k++) run += tb.wsum[k];
+#pragma unroll
+  for (int k = 0; k < kE; k++) {
+    tb.cnt[kE * t + (uint32_t)k] = run;
+    run += c[k];
+  }
+  __syncthreads();
+  const uint32_t used = tb.used;
+  auto begin = [&](uint32_t e) { return e < used ? tb.cnt[e] : m; };
+  // a value's copies: a wave each, or, for many, the workgroup
+  constexpr uint32_t kMany = 4096;
+  for (uint32_t e = w; e < used; e += kBWaves) {
+    const uint32_t a = begin(e), z = begin(e + 1);
+    if (z - a >= kMany) continue;
+    const uint64_t key = tag | K::key((typename K::V)tb.val[e], hi);
+    for (uint32_t i = a + lane; i < z; i += 64) out[s + i] = key;
+  }
+  for (uint32_t e = 0; e < used; e++) {
+    const uint32_t a = begin(e), z = begin(e + 1);
+    if (z - a < kMany) continue;
+    const uint64_t key = tag | K::key((typename K::V)tb.val[e], hi);
+    for (uint32_t i = a + t; i < z; i += kBThreads) out[s + i] = key;
+  }
+  bucket_region_starts(ra, b, nbuckets, low_bits, s, n, [&](uint32_t x) {
+    uint32_t lo = 0, up = used;  // first value at or above the bound
+    while (lo < up) {
+      const uint32_t mid = (lo + up) >> 1;
+      if (tb.val[mid] < (uint64_t)K::bound(x)) lo = mid + 1; else up = mid;
+    }
+    return begin(lo);
+  });
+  return true;
+}
+
+template <bool kTagged>
 __device__ __forceinline__ void sort_flagged_bucket(uint64_t* in, uint64_t* out, uint64_t n, int low_bits,
                                                  const uint32_t* __restrict__ starts, uint32_t nbuckets,
                                                  uint32_t* __restrict__ slow, uint32_t b, BucketSmem& sm,
                                                  const gqf_region_args& ra, uint64_t tag) {
+  using K = BucketKey<kTagged>;
   const uint64_t s = starts[b];
   const uint64_t e = b + 1 < nbuckets ? (uint64_t)starts[b + 1] : n;
   const uint32_t m = (uint32_t)(e - s);
+  const uint64_t hi = (uint64_t)b << low_bits;
   const int t = threadIdx.x;
-  const int passes = (low_bits + 7) / 8;
+  const int passes = (low_bits + K::kExtra + 7) / 8;
+  __syncthreads();  // every thread has read the flag
+  if (t == 0) slow[b] = 0;
+  if ((kTagged || m > kBucketCap) &&
+      sort_by_table<kTagged>(in, out, s, n, m, low_bits, b, nbuckets, *(BucketTable*)&sm, ra, tag))
+    return;
+  __syncthreads();
   for (int k = t; k < kBMaxPasses * 256; k += kBThreads) (&sm.tot[0][0])[k] = 0;
   __syncthreads();
-  if (t == 0) slow[b] = 0;
-  if (m <= kBucketCap) {
-    const uint64_t hi = (uint64_t)b << low_bits;
+  if (!kTagged && m <= kBucketCap) {
     for (uint32_t i = t; i < m; i += kBThreads) {
       const uint32_t v = (uint32_t)(in[s + i] - hi);
       sm.buf[0][i] = v;
@@ -604,7 +890,7 @@ __device__ __forceinline__ void sort_flagged_bucket(uint64_t* in, uint64_t* out,
     }
     for (uint32_t i = t; i < m; i += kBThreads) out[s + i] = tag | hi | sm.buf[src][i];
     const uint32_t* sorted = sm.buf[src];
-    bucket_region_starts(ra, b, low_bits, s, [&](uint32_t x) {
+    bucket_region_starts(ra, b, nbuckets, low_bits, s, n, [&](uint32_t x) {
       uint32_t lo = 0, hi2 = m;
       while (lo < hi2) {
         const uint32_t mid = (lo + hi2) >> 1;
@@ -614,38 +900,38 @@ __device__ __forceinline__ void sort_flagged_bucket(uint64_t* in, uint64_t* out,
     });
     return;
   }
-  // too large for LDS: the same passes between the bucket's ranges of in and
-  // out, plus a copy pass on the (shared) top bits when the count is even, so
-  // the result lands in out; other waves' stores are published between
-  // passes with agent-scope fences around the barrier
+  // too large for LDS, or tagged: the same passes, over the keys as they are
+  // ordered, between the bucket's ranges of in and out, plus a pass on a zero
+  // digit when the count is even, so the result lands in out; other waves'
+  // stores are published between passes with agent-scope fences around the
+  // barrier
   const int gpasses = passes | 1;
   uint64_t* a = in + s;
   uint64_t* o = out + s;
   for (uint32_t i = t; i < m; i += kBThreads) {
-    const uint64_t v = a[i];
+    const uint64_t v = K::of(a[i], hi);
+    a[i] = v;
     for (int p = 0; p < gpasses; p++) atomicAdd(&sm.tot[p][(uint32_t)(v >> (8 * p)) & 255u], 1u);
   }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
   __syncthreads();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   for (int p = 0; p < gpasses; p++) {
     bucket_pass<uint64_t>(p & 1 ? o : a, p & 1 ? a : o, m, 8 * p, sm.tot[p], sm);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
     __syncthreads();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   }
-  // the bucket's keys now ascend in o (their top bits are the bucket's)
-  const uint64_t base = (uint64_t)b << low_bits;
-  bucket_region_starts(ra, b, low_bits, s, [&](uint32_t x) {
+  bucket_region_starts(ra, b, nbuckets, low_bits, s, n, [&](uint32_t x) {
     uint32_t lo = 0, hi2 = m;
     while (lo < hi2) {
       const uint32_t mid = (lo + hi2) >> 1;
-      if (o[mid] - base < (uint64_t)x) lo = mid + 1; else hi2 = mid;
+      if (o[mid] < (uint64_t)K::bound(x)) lo = mid + 1; else hi2 = mid;
     }
     return lo;
   });
-  if (tag) {
-    __syncthreads();  // the searches above read o untagged
-    for (uint32_t i = t; i < m; i += kBThreads) o[i] |= tag;
-  }
+  __syncthreads();  // the searches above read o as ordered
+  for (uint32_t i = t; i < m; i += kBThreads) o[i] = tag | K::key((typename K::V)o[i], hi);
 }
 
 // The flagged buckets (skips the others, and clears the flags it takes):
@@ -659,9 +945,199 @@ gqf_sort_buckets_slow(uint64_t* in, uint64_t* out, uint64_t n, int low_bits, con
                       uint32_t nbuckets, uint32_t* __restrict__ slow, gqf_region_args ra, uint64_t tag) {
   __shared__ BucketSmem sm;
   for (uint32_t b = blockIdx.x; b < nbuckets; b += gridDim.x) {
-    if (slow[b]) sort_flagged_bucket(in, out, n, low_bits, starts, nbuckets, slow, b, sm, ra, tag);
+    if (slow[b]) sort_flagged_bucket<false>(in, out, n, low_bits, starts, nbuckets, slow, b, sm, ra, tag);
     __syncthreads();
   }
+}
+extern "C" __global__ void __launch_bounds__(kBThreads)
+gqf_sort_buckets_slow_tagged(uint64_t* in, uint64_t* out, uint64_t n, int low_bits, const uint32_t* __restrict__ starts,
+                             uint32_t nbuckets, uint32_t* __restrict__ slow, gqf_region_args ra) {
+  __shared__ BucketSmem sm;
+  for (uint32_t b = blockIdx.x; b < nbuckets; b += gridDim.x) {
+    if (slow[b]) sort_flagged_bucket<true>(in, out, n, low_bits, starts, nbuckets, slow, b, sm, ra, 0);
+    __syncthreads();
+  }
+}
+
+// ---------------------------------------------------------------------------
+// One-workgroup sort of up to kTinyCap keys (hashed here, or tagged), which
+// also lists their regions: a batch of a few thousand keys is then one launch
+// instead of a dozen.  As the bucket sort: the keys are counted by their top
+// (up to) 12 bits, put into sub-bucket order in LDS, and each one's place is
+// its rank among the keys of its sub-bucket (two on average at 8192 uniform
+// keys).  A sub-bucket above kSubCap keys (repeats) makes the workgroup run a
+// bitonic network over all of them instead.  Latency bound: 12 us for 5000
+// keys, against 63 us for the four passes (12 launches) of the LSD sort plus 9
+// for the region bounds.
+
+namespace {
+constexpr int kTThreads = 1024;
+constexpr uint32_t kTinyCap = GQF_SORT_TINY;
+constexpr int kTLoad = kTinyCap / kTThreads;
+constexpr int kTSubBits = 12;
+constexpr uint32_t kTSub = 1u << kTSubBits;
+static_assert(kTSub == 4 * kTThreads, "four sub-buckets per thread in the scan");
+}  // namespace
+
+template <bool kTagged>
+__device__ __forceinline__ void sort_tiny(uint64_t* __restrict__ keys, uint32_t n, uint64_t mask, int vshift, int bits,
+                                          const gqf_list_args& la) {
+  __shared__ uint64_t buf[kTinyCap];
+  __shared__ uint64_t sorted[kTinyCap];
+  __shared__ uint32_t sub_end[kTSub];
+  __shared__ uint32_t wsum[kTThreads / 64];
+  __shared__ uint32_t oversize, nlist[2];
+  const uint32_t t = threadIdx.x, w = t >> 6, lane = t & 63;
+  // tagged keys as seq_order has them: hash bits above 16 tag bits
+  const int all = bits + (kTagged ? 16 : 0);
+  const int sb = bits > kTSubBits ? all - kTSubBits : all - bits;
+  uint64_t v[kTLoad];
+#pragma unroll
+  for (int k = 0; k < kTLoad; k++) v[k] = keys[min((uint32_t)k * kTThreads + t, n - 1)];
+#pragma unroll
+  for (int k = 0; k < 4; k++) sub_end[(uint32_t)k * kTThreads + t] = 0;
+  if (t == 0) oversize = nlist[0] = nlist[1] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < kTLoad; k++) {
+    const uint32_t i = (uint32_t)k * kTThreads + t;
+    v[k] = kTagged ? seq_order(v[k] & GQF_SEQ_HASH_MASK, v[k]) : gqf_hash64(v[k], mask) << vshift;
+    if (i < n) atomicAdd(&sub_end[(uint32_t)(v[k] >> sb)], 1u);
+  }
+  __syncthreads();
+  {
+    uint32_t c[4], sum = 0;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      c[k] = sub_end[4 * t + k];
+      sum += c[k];
+      if (c[k] > kSubCap) oversize = 1;
+    }
+    const uint32_t incl = wave_scan_add(sum);
+    if (lane == 63) wsum[w] = incl;
+    __syncthreads();
+    uint32_t run = incl - sum;
+    for (uint32_t k = 0; k < w; k++) run += wsum[k];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      sub_end[4 * t + k] = run;
+      run += c[k];
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < kTLoad; k++)
+    if ((uint32_t)k * kTThreads + t < n) buf[atomicAdd(&sub_end[(uint32_t)(v[k] >> sb)], 1u)] = v[k];
+  const uint64_t* res = sorted;
+  if (oversize) {
+    uint32_t p = 2;
+    while (p < n) p *= 2;
+    for (uint32_t i = n + t; i < p; i += kTThreads) buf[i] = ~0ULL;
+    __syncthreads();
+    for (uint32_t k = 2; k <= p; k *= 2) {
+      for (uint32_t j = k / 2; j > 0; j /= 2) {
+        for (uint32_t i = t; i < p / 2; i += kTThreads) {
+          const uint32_t a = (i / j) * 2 * j + i % j, b = a + j;  // the i-th pair at distance j
+          const uint64_t x = buf[a], y = buf[b];
+          if ((x > y) == ((a & k) == 0)) {
+            buf[a] = y;
+            buf[b] = x;
+          }
+        }
+        __syncthreads();
+      }
+    }
+    res = buf;
+  } else {
+    __syncthreads();
+    for (uint32_t i = t; i < n; i += kTThreads) {
+      const uint64_t x = buf[i];
+      const uint32_t d = (uint32_t)(x >> sb);
+      const uint32_t st = d ? sub_end[d - 1] : 0u, en = sub_end[d];
+      uint32_t r = st;
+      for (uint32_t j = st; j < en; j++) {
+        const uint64_t y = buf[j];
+        r += (y < x || (y == x && j < i)) ? 1u : 0u;
+      }
+      sorted[r] = x;
+    }
+    __syncthreads();
+  }
+  constexpr int kExtra = kTagged ? 16 : 0;
+  for (uint32_t i0 = 0; i0 < n; i0 += kTThreads) {
+    const uint32_t i = i0 + t;
+    const bool in = i < n;
+    const uint64_t x = in ? res[i] : 0;
+    if (in) keys[i] = kTagged ? (x >> 16 | seq_tag_of(x)) : x;
+    if (!la.list) continue;
+    // a key that opens its region lists it; it also ends the region of the
+    // key before it
+    const uint32_t r = (uint32_t)(x >> (kExtra + 14)) / la.region_blocks;
+    const uint32_t before = in && i ? (uint32_t)(res[i - 1] >> (kExtra + 14)) / la.region_blocks : 0u;
+    const bool head = in && (i == 0 || r != before);
+#pragma unroll
+    for (uint32_t par = 0; par < 2; par++) {
+      const uint64_t hm = __ballot(head && (r & 1u) == par);
+      if (!hm) continue;
+      uint32_t at = 0;
+      if (lane == 0) at = atomicAdd(&nlist[par], (uint32_t)__popcll(hm));
+      at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at);
+      if (head && (r & 1u) == par)
+        la.list[par * la.stride + at + (uint32_t)__popcll(hm & ((1ULL << lane) - 1))] = r;
+    }
+    if (head) {
+      la.start[r] = i;
+      if (i) la.start[before + 1] = i;
+    }
+    if (in && i + 1 == n) la.start[r + 1] = n;
+  }
+  if (la.list) {
+    __syncthreads();
+    if (t < 2) la.count[t] = nlist[t];
+  }
+}
+
+extern "C" __global__ void __launch_bounds__(kTThreads)
+gqf_sort_tiny(uint64_t* __restrict__ keys, uint32_t n, uint64_t mask, int vshift, int bits, gqf_list_args la) {
+  sort_tiny<false>(keys, n, mask, vshift, bits, la);
+}
+extern "C" __global__ void __launch_bounds__(kTThreads)
+gqf_sort_tiny_tagged(uint64_t* __restrict__ keys, uint32_t n, int bits, gqf_list_args la) {
+  sort_tiny<true>(keys, n, 0, 0, bits, la);
+}
+
+// The regions of n sorted keys, listed by the keys that open them (as
+// gqf_sort_tiny lists them; counts cleared before): start[r] and start[r + 1]
+// are written for the listed regions only.
+extern "C" __global__ void __launch_bounds__(kTThreads)
+gqf_region_heads(const uint64_t* __restrict__ keys, uint32_t n, uint64_t hmask, gqf_list_args la) {
+  __shared__ uint32_t cnt[2], base[2];
+  const uint32_t t = threadIdx.x, lane = t & 63;
+  const uint32_t i = blockIdx.x * kTThreads + t;
+  const bool in = i < n;
+  const uint32_t r = in ? (uint32_t)((keys[i] & hmask) >> 14) / la.region_blocks : 0u;
+  const uint32_t before = in && i ? (uint32_t)((keys[i - 1] & hmask) >> 14) / la.region_blocks : 0u;
+  const bool head = in && (i == 0 || r != before);
+  if (t < 2) cnt[t] = 0;
+  __syncthreads();
+  uint32_t at = 0;
+#pragma unroll
+  for (uint32_t par = 0; par < 2; par++) {
+    const uint64_t hm = __ballot(head && (r & 1u) == par);
+    uint32_t a = 0;
+    if (lane == 0 && hm) a = atomicAdd(&cnt[par], (uint32_t)__popcll(hm));
+    a = (uint32_t)__builtin_amdgcn_readfirstlane((int)a);
+    if (head && (r & 1u) == par) at = a + (uint32_t)__popcll(hm & ((1ULL << lane) - 1));
+  }
+  __syncthreads();
+  if (t < 2) base[t] = cnt[t] ? atomicAdd(&la.count[t], cnt[t]) : 0u;
+  __syncthreads();
+  if (head) {
+    la.list[(r & 1u) * la.stride + base[r & 1u] + at] = r;
+    la.start[r] = i;
+    if (i) la.start[before + 1] = i;
+  }
+  if (in && i + 1 == n) la.start[r + 1] = n;
 }
 
 // ---------------------------------------------------------------------------
@@ -752,10 +1228,11 @@ extern "C" __global__ void gqf_rle_counts(const uint64_t* __restrict__ upos, con
 
 static inline uint32_t sort_ntiles(uint64_t n) { return (uint32_t)((n + kTile - 1) / kTile); }
 
-// sized for the larger of the 4096-key tiling and the small-input tiling
+// sized for the larger of the 4096-key tiling and the small-input tilings
 uint64_t gqf_sort_hist_words(uint64_t n) {
   const uint64_t t = sort_ntiles(n);
-  return (uint64_t)kMaxRadix * (t > kScanSmallTiles ? t : kScanSmallTiles);
+  static_assert(kMScanTiles >= kScanSmallTiles, "the larger of the small tilings");
+  return (uint64_t)kMaxRadix * (t > kMScanTiles ? t : kMScanTiles);
 }
 
 namespace {
@@ -817,40 +1294,75 @@ void gqf_launch_sort(uint64_t* keys, uint64_t* tmp, uint64_t n, int hash_it, uin
   }
 }
 
-bool gqf_sort_two_level_fits(uint64_t n, int bits) {
-  return n >= (1ULL << 20) && n <= (1ULL << 24) && bits >= 18 && bits <= 42;
+bool gqf_sort_fast_fits(uint64_t n, int bits, bool tagged) {
+  if (n <= kTinyCap) return bits <= 42;
+  return n <= (tagged ? 1ULL << 22 : 1ULL << 24) && bits >= 18 && bits <= 42;  // 1024 buckets of 4K / 16K keys
 }
 
-void gqf_launch_sort_two_level(uint64_t* keys, uint64_t* tmp, uint64_t n, uint64_t mask, int vshift, int bits,
-                               uint32_t* hist, uint32_t* totals, uint32_t* slow, hipStream_t s,
-                               const gqf_region_args* regions, uint64_t tag) {
+void gqf_launch_sort_fast(uint64_t* keys, uint64_t* tmp, uint64_t n, bool tagged, uint64_t mask, int vshift, int bits,
+                          uint32_t* hist, uint32_t* totals, uint32_t* slow, hipStream_t s,
+                          const gqf_region_args* regions, const gqf_list_args* lists, uint64_t tag) {
+  if (n == 0) return;
+  const gqf_list_args la = lists ? *lists : gqf_list_args{};
   const gqf_region_args ra = regions ? *regions : gqf_region_args{};
-  // 2^msd buckets of about 12K keys (at most 1024), low bits <= 32
-  int msd = 4;
-  while (msd < 10 && (n >> msd) > 12288) msd++;
+  if (n <= kTinyCap && !tag && !regions) {
+    gqf_prof_begin("sort_pass", s);
+    if (tagged)
+      hipLaunchKernelGGL(gqf_sort_tiny_tagged, dim3(1), dim3(kTThreads), 0, s, keys, (uint32_t)n, bits, la);
+    else
+      hipLaunchKernelGGL(gqf_sort_tiny, dim3(1), dim3(kTThreads), 0, s, keys, (uint32_t)n, mask, vshift, bits, la);
+    gqf_prof_end("sort_pass", s);
+    return;
+  }
+  // 2^msd buckets (at most 1024), low bits <= 32: of about 12K keys, or 4K
+  // below 2^20 keys (more workgroups) and for tagged ones (8 bytes in LDS)
+  const uint64_t want = tagged || n < (1ULL << 20) ? 4096 : 12288;
+  int msd = 2;
+  while (msd < 10 && (n >> msd) > want) msd++;
   if (bits - msd > 32) msd = bits - 32;
   const int radix = 1 << msd;
-  // about 512 tiles of 1..8 rounds: 32K keys per tile at 2^24 keys.  The
-  // histogram (radix x ntiles <= 1024 x n / 8192 words) fits the LSD
-  // sort's (gqf_sort_hist_words)
-  uint64_t rounds = n / ((uint64_t)kMRound * 512);
+  const uint32_t* starts = totals + kMaxRadix;
+  // tiles of one short round below kMSmallN keys; above, about 512 tiles of
+  // 1..8 rounds: 32K keys per tile at 2^24 keys.  The histogram (radix x
+  // ntiles <= 1024 x n / 8192 words, or 128 x 128) fits the LSD sort's
+  // (gqf_sort_hist_words)
+  const bool small = tagged || n < kMSmallN;
+  const uint64_t round = (uint64_t)kMThreads * (small ? kMItemsSmall : kMItems);
+  uint64_t rounds = n / (round * 512);
   rounds = rounds < 1 ? 1 : (rounds > 8 ? 8 : rounds);
-  const uint64_t tile_keys = rounds * kMRound;
+  if (small && n > round * kMScanTiles) rounds = (n + round * kMScanTiles - 1) / (round * kMScanTiles);
+  const uint64_t tile_keys = rounds * round;
   const uint32_t ntiles = (uint32_t)((n + tile_keys - 1) / tile_keys);
   gqf_prof_begin("sort_pass", s);
-  hipLaunchKernelGGL(gqf_msd_count, dim3(ntiles), dim3(kMThreads), 0, s, (const uint64_t*)keys, n, tile_keys,
-                     bits - msd, msd, mask, vshift, hist, ntiles);
-  hipLaunchKernelGGL(gqf_sort_scan_rows, dim3(radix), dim3(kThreads), 0, s, hist, ntiles, totals);
-  hipLaunchKernelGGL(gqf_sort_scan_totals, dim3(1), dim3(kThreads), 0, s, totals, radix);
-  hipLaunchKernelGGL(gqf_msd_scatter, dim3(ntiles), dim3(kMThreads), 0, s, (const uint64_t*)keys, tmp, n, tile_keys,
-                     bits - msd, msd, mask, vshift, (const uint32_t*)hist, (const uint32_t*)totals, ntiles);
+  hipLaunchKernelGGL(tagged ? gqf_msd_count_tagged : (small ? gqf_msd_count_small : gqf_msd_count), dim3(ntiles),
+                     dim3(kMThreads), 0, s, (const uint64_t*)keys, n, tile_keys, bits - msd, msd, mask, vshift, hist,
+                     ntiles, la.count);
+  if (ntiles > kMScanTiles)
+    hipLaunchKernelGGL(gqf_sort_scan_rows, dim3(radix), dim3(kThreads), 0, s, hist, ntiles, totals);
+  hipLaunchKernelGGL(tagged ? gqf_msd_scatter_tagged : (small ? gqf_msd_scatter_small : gqf_msd_scatter), dim3(ntiles),
+                     dim3(kMThreads), 0, s, (const uint64_t*)keys, tmp, n, tile_keys, bits - msd, msd, mask, vshift,
+                     (const uint32_t*)hist, (const uint32_t*)totals, totals + kMaxRadix, ntiles);
   gqf_prof_end("sort_pass", s);
   gqf_prof_begin("sort_buckets", s);
-  hipLaunchKernelGGL(gqf_sort_buckets, dim3(radix), dim3(kBThreads), 0, s, (const uint64_t*)tmp, keys, n, bits - msd,
-                     (const uint32_t*)totals, (uint32_t)radix, slow, ra, tag);
-  hipLaunchKernelGGL(gqf_sort_buckets_slow, dim3(radix < 256 ? radix : 256), dim3(kBThreads), 0, s, tmp, keys, n, bits - msd,
-                     (const uint32_t*)totals, (uint32_t)radix, slow, ra, tag);
+  const dim3 gslow(radix < 256 ? radix : 256);
+  if (tagged) {
+    hipLaunchKernelGGL(gqf_sort_buckets_tagged, dim3(radix), dim3(kBThreads), 0, s, (const uint64_t*)tmp, keys, n,
+                       bits - msd, starts, (uint32_t)radix, slow, ra);
+    hipLaunchKernelGGL(gqf_sort_buckets_slow_tagged, gslow, dim3(kBThreads), 0, s, tmp, keys, n, bits - msd, starts,
+                       (uint32_t)radix, slow, ra);
+  } else {
+    hipLaunchKernelGGL(gqf_sort_buckets, dim3(radix), dim3(kBThreads), 0, s, (const uint64_t*)tmp, keys, n, bits - msd,
+                       starts, (uint32_t)radix, slow, ra, tag);
+    hipLaunchKernelGGL(gqf_sort_buckets_slow, gslow, dim3(kBThreads), 0, s, tmp, keys, n, bits - msd, starts,
+                       (uint32_t)radix, slow, ra, tag);
+  }
   gqf_prof_end("sort_buckets", s);
+  if (la.list) {
+    gqf_prof_begin("region_bounds", s);
+    hipLaunchKernelGGL(gqf_region_heads, dim3((uint32_t)((n + kTThreads - 1) / kTThreads)), dim3(kTThreads), 0, s,
+                       (const uint64_t*)keys, (uint32_t)n, tagged ? GQF_SEQ_HASH_MASK : ~0ULL, la);
+    gqf_prof_end("region_bounds", s);
+  }
 }
 
 void gqf_launch_rle(const uint64_t* keys, uint64_t n, uint32_t* tile_heads, uint64_t* ukeys, uint64_t* upos,
