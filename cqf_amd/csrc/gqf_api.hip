@@ -11,6 +11,7 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <algorithm>
 #include <mutex>
 #include <string>
 #include <unordered_map>
@@ -63,12 +64,26 @@ struct Workspace {
   uint32_t* agg_ctrl = nullptr;    // 4 control words, then the bucket fills
 };
 
+// Tables of the whole-table passes (allocated on first use, grown for a
+// larger table) and the items of one chunk of a merge into this filter.  A
+// pass holds `mu` from its first launch until its results are on the host, so
+// passes over one filter from several threads take turns.
+struct EnumSpace {
+  std::mutex mu;
+  uint64_t groups = 0;
+  gqf_enum_tables t;
+  uint64_t move_cap = 0;
+  uint64_t* move_items = nullptr;
+  uint64_t* move_counts = nullptr;
+};
+
 struct Filter {
   QF host;           // host mirror of the device descriptor
   QF* dev = nullptr; // the public handle
   int sort_digit = 0;  // radix digit bits of the bulk sort (0: chosen from the key bits)
   Workspace ws;
   std::mutex mu;     // serialises workspace growth
+  EnumSpace es;
 };
 
 std::unordered_map<QF*, Filter*> g_filters;
@@ -104,6 +119,35 @@ void free_workspace(Workspace& w) {
   dev_free(w.upos);
   dev_free(w.ucounts);
   w.cap = 0;
+}
+
+void free_enum_space(EnumSpace& e) {
+  dev_free(e.t.items);
+  dev_free(e.t.slots);
+  dev_free(e.t.sums);
+  dev_free(e.t.base);
+  dev_free(e.t.stats);
+  dev_free(e.move_items);
+  dev_free(e.move_counts);
+  e.groups = e.move_cap = 0;
+}
+
+// room for `groups` groups (the caller holds e.mu)
+bool ensure_enum_space(EnumSpace& e, uint64_t groups) {
+  if (groups <= e.groups) return true;
+  dev_free(e.t.items);
+  dev_free(e.t.slots);
+  dev_free(e.t.sums);
+  dev_free(e.t.base);
+  dev_free(e.t.stats);
+  dev_alloc(&e.t.items, groups);
+  dev_alloc(&e.t.slots, groups);
+  dev_alloc(&e.t.sums, groups);
+  dev_alloc(&e.t.base, groups + 1);
+  dev_alloc(&e.t.stats, 3);
+  const bool ok = e.t.items && e.t.slots && e.t.sums && e.t.base && e.t.stats;
+  e.groups = ok ? groups : 0;
+  return ok;
 }
 
 // the per-table part of a workspace: region tables of the rebuild
@@ -478,6 +522,7 @@ extern "C" void qf_destroy_device(QF* qf) {
   }
   GQF_CHECK(hipDeviceSynchronize());
   free_all_workspace(f->ws);
+  free_enum_space(f->es);
   dev_free(f->host.blocks);
   dev_free(f->host.status);
   dev_free(f->host.locks);
@@ -1033,106 +1078,53 @@ extern "C" void gqf_fill_splitmix64(uint64_t* dev_out, uint64_t n, uint64_t seed
 
 namespace {
 
-// device scratch of one count pass over nblocks blocks
-struct EnumScratch {
-  uint64_t nwg = 0;
-  uint32_t* wg_items = nullptr;
-  uint64_t* wg_base = nullptr;           // nwg + 1
-  unsigned long long* stats = nullptr;   // items, sum of counts, used slots, spare
-  // marks of item starts for the write pass: one word per block from the
-  // first enumerated block to the end of the table
-  uint64_t nwords = 0;
-  unsigned long long* starts = nullptr;
-  unsigned long long* max_word = nullptr;
-  uint32_t* local_prefix = nullptr;
-  uint32_t* group_sums = nullptr;
-  uint64_t* group_base = nullptr;
-  bool init(uint64_t nblocks) {
-    nwg = gqf_enum_wg_count(nblocks);
-    dev_alloc(&wg_items, nwg);
-    dev_alloc(&wg_base, nwg + 1);
-    dev_alloc(&stats, 4);
-    return wg_items && wg_base && stats;
-  }
-  bool init_marks(uint64_t words, hipStream_t s) {
-    nwords = words;
-    const uint64_t ng = gqf_enum_wg_count(words);
-    dev_alloc(&starts, words);
-    dev_alloc(&max_word, 1);
-    dev_alloc(&local_prefix, words);
-    dev_alloc(&group_sums, ng);
-    dev_alloc(&group_base, ng + 1);
-    if (!starts || !max_word || !local_prefix || !group_sums || !group_base) return false;
-    GQF_CHECK(hipMemsetAsync(starts, 0, words * sizeof(unsigned long long), s));
-    return true;
-  }
-  ~EnumScratch() {
-    dev_free(wg_items);
-    dev_free(wg_base);
-    dev_free(stats);
-    dev_free(starts);
-    dev_free(max_word);
-    dev_free(local_prefix);
-    dev_free(group_sums);
-    dev_free(group_base);
-  }
-};
-
 uint64_t quotient_blocks(const QF& h) { return (h.nslots + GQF_SLOTS_PER_BLOCK - 1) / GQF_SLOTS_PER_BLOCK; }
 
-// Counted insert of every item of `src` into `dst` (dst_dev / dst, with the
-// region tables of dst_ws): the items are enumerated in chunks of whole
-// 256-block groups, each chunk written as ascending unique slot hashes of
-// dst with their counts and merged into dst by the rebuild.  Returns the
+// Counted insert of every item of filter `f` into `dst` (dst_dev / dst, with
+// the region tables of dst_ws and the item buffers of dst_es): the items are
+// written in chunks of whole groups, ascending unique slot hashes of dst with
+// their counts, each merged into dst by the rebuild.  Chunks of kMoveItems
+// bound the buffers a merged-into filter keeps (64 MB), and are enough items
+// for every CU; the chunks run one behind the other on the stream.  Returns the
 // number of items moved, or < 0.  Synchronises.
-int64_t move_items(const QF* src_dev, const QF& src, const QF* dst_dev, const QF& dst, Workspace& dst_ws,
-                   hipStream_t s) {
+constexpr uint64_t kMoveItems = 1ULL << 22;
+
+int64_t move_items(Filter* f, const QF* dst_dev, const QF& dst, Workspace& dst_ws, EnumSpace& dst_es, hipStream_t s) {
+  std::lock_guard<std::mutex> lk(f->es.mu);
+  const QF& src = f->host;
   const uint64_t nb = quotient_blocks(src);
-  EnumScratch sc;
-  if (!sc.init(nb)) return -3;
-  GQF_CHECK(hipMemsetAsync(sc.stats, 0, 4 * sizeof(unsigned long long), s));
-  gqf_launch_enum_count(src_dev, 0, nb, 0, src.nslots, sc.wg_items, sc.wg_base, sc.stats, nullptr, nullptr, s);
-  std::vector<uint64_t> base(sc.nwg + 1);
-  GQF_CHECK(hipMemcpyAsync(base.data(), sc.wg_base, base.size() * sizeof(uint64_t), hipMemcpyDeviceToHost, s));
-  GQF_CHECK(hipStreamSynchronize(s));
-  const uint64_t total = base[sc.nwg];
+  const uint64_t groups = gqf_enum_groups(nb);
+  if (!ensure_enum_space(f->es, groups)) return -3;
+  const gqf_enum_tables& t = f->es.t;
+  gqf_launch_enum_count(f->dev, 0, nb, 0, src.nslots, t, s);
+  std::vector<uint64_t> base(groups + 1);
+  hipError_t e = hipMemcpyAsync(base.data(), t.base, base.size() * sizeof(uint64_t), hipMemcpyDeviceToHost, s);
+  if (e == hipSuccess) e = hipStreamSynchronize(s);
+  note_error(e, "move_items");
+  if (e != hipSuccess) return -3;
+  const uint64_t total = base[groups];
   if (total == 0) return 0;
-  uint64_t cap = total < (1ULL << 24) ? total : (1ULL << 24);
-  for (uint64_t u = 0; u < sc.nwg; u++)
-    if (base[u + 1] - base[u] > cap) cap = base[u + 1] - base[u];
-  uint64_t* items = nullptr;
-  uint64_t* counts = nullptr;
-  dev_alloc(&items, cap);
-  dev_alloc(&counts, cap);
-  if (!items || !counts) {
-    dev_free(items);
-    dev_free(counts);
-    return -3;
+  uint64_t cap = std::min(total, kMoveItems);
+  for (uint64_t u = 0; u < groups; u++) cap = std::max(cap, base[u + 1] - base[u]);
+  if (cap > dst_es.move_cap) {
+    GQF_CHECK(hipStreamSynchronize(s));  // a merge before this one may still use them
+    dev_free(dst_es.move_items);
+    dev_free(dst_es.move_counts);
+    dev_alloc(&dst_es.move_items, cap);
+    dev_alloc(&dst_es.move_counts, cap);
+    dst_es.move_cap = dst_es.move_items && dst_es.move_counts ? cap : 0;
+    if (!dst_es.move_cap) return -3;
   }
+  uint64_t* items = dst_es.move_items;
+  uint64_t* counts = dst_es.move_counts;
   init_region_workspace(dst_ws, dst.nblocks);
-  if (!sc.init_marks(src.nblocks, s)) {
-    dev_free(items);
-    dev_free(counts);
-    return -3;
-  }
-  for (uint64_t u = 0; u < sc.nwg;) {
+  for (uint64_t u = 0; u < groups;) {
     uint64_t v = u + 1;
-    while (v < sc.nwg && base[v + 1] - base[u] <= cap) v++;
+    while (v < groups && base[v + 1] - base[u] <= cap) v++;
     const uint64_t n = base[v] - base[u];
     if (n) {
-      const uint64_t b_lo = u * GQF_ENUM_WG_BLOCKS, b_hi = v * GQF_ENUM_WG_BLOCKS < nb ? v * GQF_ENUM_WG_BLOCKS : nb;
-      const uint64_t q_hi = b_hi * 64 < src.nslots ? b_hi * 64 : src.nslots;
-      GQF_CHECK(hipMemsetAsync(sc.max_word, 0, sizeof(unsigned long long), s));
-      unsigned long long* marks = sc.starts + b_lo;  // word 0 of this pass is block b_lo
-      gqf_launch_enum_count(src_dev, b_lo, b_hi, b_lo * 64, q_hi, sc.wg_items, sc.wg_base, sc.stats, marks,
-                            sc.max_word, s);
-      // the write pass covers the marked words only: up to the last one
-      unsigned long long last = 0;
-      GQF_CHECK(hipMemcpyAsync(&last, sc.max_word, sizeof(last), hipMemcpyDeviceToHost, s));
-      GQF_CHECK(hipStreamSynchronize(s));
-      gqf_launch_enum_emit(src_dev, b_lo, (uint64_t)last + 1, marks, sc.max_word, sc.local_prefix, sc.group_sums,
-                           sc.group_base, GQF_ENUM_OUT_MOVE, (int)src.value_bits, (int)dst.value_bits,
-                           gqf_mask(src.key_bits), items, counts, nullptr, cap, s);
+      gqf_launch_enum_emit(f->dev, 0, nb, 0, src.nslots, u, v, t.base, base[u], GQF_ENUM_OUT_MOVE, (int)src.value_bits,
+                           (int)dst.value_bits, gqf_mask(src.key_bits), items, counts, nullptr, cap, s);
       gqf_launch_region_bounds(dst_dev, dst.nregions, items, n, nullptr, dst_ws.region_start, dst_ws.region_list,
                                dst_ws.list_count, ~0ULL, s);
       gqf_launch_rebuild(dst_dev, dst.nregions, dst.region_blocks, items, counts, n, dst_ws.region_start, dst_ws.region_list,
@@ -1141,8 +1133,6 @@ int64_t move_items(const QF* src_dev, const QF& src, const QF* dst_dev, const QF
     u = v;
   }
   GQF_CHECK(hipStreamSynchronize(s));
-  dev_free(items);
-  dev_free(counts);
   return (int64_t)total;
 }
 
@@ -1181,24 +1171,17 @@ extern "C" int qf_enumerate(QF* qf, uint64_t q_lo, uint64_t q_hi, int form, uint
   if (q_hi > h.nslots) q_hi = h.nslots;
   if (q_lo >= q_hi) return 0;
   const uint64_t b_lo = q_lo / 64, b_hi = (q_hi + 63) / 64;
-  EnumScratch sc;
-  const bool write = cap && (hashes || counts || values);
-  if (!sc.init(b_hi - b_lo) || (write && !sc.init_marks(h.nblocks - b_lo, s))) return -3;
-  GQF_CHECK(hipMemsetAsync(sc.stats, 0, 4 * sizeof(unsigned long long), s));
-  if (write) GQF_CHECK(hipMemsetAsync(sc.max_word, 0, sizeof(unsigned long long), s));
-  gqf_launch_enum_count(f->dev, b_lo, b_hi, q_lo, q_hi, sc.wg_items, sc.wg_base, sc.stats, sc.starts, sc.max_word,
-                        s);
-  unsigned long long last = 0;
-  if (write) {
-    GQF_CHECK(hipMemcpyAsync(&last, sc.max_word, sizeof(last), hipMemcpyDeviceToHost, s));
-    GQF_CHECK(hipStreamSynchronize(s));
-  }
-  if (write)
-    gqf_launch_enum_emit(f->dev, b_lo, (uint64_t)last + 1, sc.starts, sc.max_word, sc.local_prefix, sc.group_sums,
-                         sc.group_base, form == QF_ENUM_KEY ? GQF_ENUM_OUT_KEY : GQF_ENUM_OUT_HASH,
-                         (int)h.value_bits, 0, gqf_mask(h.key_bits), hashes, counts, values, cap, s);
+  const uint64_t groups = gqf_enum_groups(b_hi - b_lo);
+  std::lock_guard<std::mutex> lk(f->es.mu);
+  if (!ensure_enum_space(f->es, groups)) return -3;
+  const gqf_enum_tables& t = f->es.t;
+  gqf_launch_enum_count(f->dev, b_lo, b_hi, q_lo, q_hi, t, s);
+  if (cap && (hashes || counts || values))
+    gqf_launch_enum_emit(f->dev, b_lo, b_hi, q_lo, q_hi, 0, groups, t.base, 0,
+                         form == QF_ENUM_KEY ? GQF_ENUM_OUT_KEY : GQF_ENUM_OUT_HASH, (int)h.value_bits, 0,
+                         gqf_mask(h.key_bits), hashes, counts, values, cap, s);
   uint64_t total = 0;
-  hipError_t e = hipMemcpyAsync(&total, sc.wg_base + sc.nwg, sizeof(total), hipMemcpyDeviceToHost, s);
+  hipError_t e = hipMemcpyAsync(&total, t.stats, sizeof(total), hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   note_error(e, "qf_enumerate");
   if (e != hipSuccess) return -3;
@@ -1210,14 +1193,12 @@ extern "C" int qf_get_stats(QF* qf, uint64_t* nelts, uint64_t* ndistinct_elts, u
   Filter* f = lookup(qf);
   if (!f) return -1;
   const uint64_t nb = quotient_blocks(f->host);
-  EnumScratch sc;
-  if (!sc.init(nb)) return -3;
+  std::lock_guard<std::mutex> lk(f->es.mu);
+  if (!ensure_enum_space(f->es, gqf_enum_groups(nb))) return -3;
   GQF_CHECK(hipDeviceSynchronize());
-  GQF_CHECK(hipMemset(sc.stats, 0, 4 * sizeof(unsigned long long)));
-  gqf_launch_enum_count(f->dev, 0, nb, 0, f->host.nslots, sc.wg_items, sc.wg_base, sc.stats, nullptr, nullptr,
-                        nullptr);
-  unsigned long long st[4] = {0, 0, 0, 0};
-  hipError_t e = hipMemcpy(st, sc.stats, sizeof(st), hipMemcpyDeviceToHost);
+  gqf_launch_enum_count(f->dev, 0, nb, 0, f->host.nslots, f->es.t, nullptr);
+  uint64_t st[3] = {0, 0, 0};
+  hipError_t e = hipMemcpy(st, f->es.t.stats, sizeof(st), hipMemcpyDeviceToHost);
   note_error(e, "qf_get_stats");
   if (e != hipSuccess) return -3;
   if (ndistinct_elts) *ndistinct_elts = st[0];
@@ -1249,7 +1230,7 @@ extern "C" int qf_cluster_census(QF* qf, uint64_t* lengths, uint64_t cap, uint64
   if (!f) return -1;
   if (hist && (nbins == 0 || nbins > 4096)) return -2;
   const uint64_t nb = f->host.nblocks;
-  const uint64_t nwg = gqf_enum_wg_count(nb);
+  const uint64_t nwg = gqf_census_wgs(nb);
   uint64_t* used = nullptr;
   uint32_t* wg_starts = nullptr;
   uint64_t* wg_base = nullptr;
@@ -1365,9 +1346,11 @@ extern "C" int64_t qf_resize_device(QF* qf, int new_nbits) {
   QF* ndev = nullptr;
   dev_alloc(&ndev, 1);
   Workspace nws;
+  EnumSpace nes;  // the move's item buffers
   int64_t moved = -3;
   if (ndev && hipMemcpy(ndev, &nh, sizeof(QF), hipMemcpyHostToDevice) == hipSuccess)
-    moved = move_items(f->dev, old, ndev, nh, nws, nullptr);
+    moved = move_items(f, ndev, nh, nws, nes, nullptr);
+  free_enum_space(nes);
   if (moved < 0) {
     free_all_workspace(nws);
     dev_free(nh.blocks);
@@ -1402,7 +1385,7 @@ extern "C" int64_t qf_multi_merge_device(QF* const* qfs, int nqf, QF* qfr) {
   int64_t total = 0;
   for (Filter* f : src) {
     std::lock_guard<std::mutex> lk(r->mu);
-    const int64_t m = move_items(f->dev, f->host, r->dev, r->host, r->ws, nullptr);
+    const int64_t m = move_items(f, r->dev, r->host, r->ws, r->es, nullptr);
     if (m < 0) return m;
     total += m;
   }

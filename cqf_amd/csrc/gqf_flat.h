@@ -78,7 +78,7 @@ struct Head {
   int32_t xblk[kWin];       // last slot of the new runs of block j's quotients
   uint32_t wsum[2][kWaves];
   int32_t wmax[2][kWaves];
-  uint32_t n_old, any_multi, n_big, over;
+  uint32_t n_old, n_slots, any_multi, n_big, over;
   int32_t xend, bstar, bwrite, keep, result;
   uint32_t big_hash[kBig];
   uint64_t big_count[kBig];
@@ -159,6 +159,212 @@ __device__ __forceinline__ uint64_t full_count(const Head& sm, uint32_t h, uint3
   return kAuxBig;
 }
 
+// What a thread keeps of its window: the eight slots 8 t .. 8 t + 7 (eight
+// threads a block), and, in wave 0, block `lane`'s old offset; the end x0 of the
+// earlier blocks' runs; the entries.
+struct Window {
+  uint2 slots;
+  uint32_t off;
+  int32_t x0;
+  bool any;     // some run of the window's quotients
+  uint32_t n;   // entries
+};
+
+// 1. Loads the window of nwin blocks from block B0 and makes the entries of
+// its runs, in order, in sm.old; sm.rend[k] = entries of the runs of rank <= k.
+// kRange: only the runs of quotients [q_lo, q_hi) of the window (which must
+// end inside it).  All kThreads threads call it.  Returns false if the runs of
+// earlier blocks, or those of the range, reach past the window.
+template <bool kRange, class S>
+__device__ __forceinline__ bool window_entries(const QF& qf, uint64_t B0, int nwin, int32_t q_lo, int32_t q_hi, S& sm,
+                                               Window& out) {
+  const int tid = (int)threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nslots = 64 * nwin;
+  const int j = tid >> 3, sh = (tid & 7) * 8;
+  const GQF_GLOBAL uint4* g = gqf_block_ptr(qf, B0);
+  uint2 x = make_uint2(0, 0);
+  if (j < nwin) x = ((const GQF_GLOBAL uint2*)(g + (size_t)j * (GQF_BLOCK_BYTES / 16) + 4))[tid & 7];
+  uint32_t off_j = 0;
+  if (wave == 0) {
+    uint4 h0 = make_uint4(0, 0, 0, 0), h1 = h0;
+    if (lane < nwin) {
+      h0 = g[(size_t)lane * (GQF_BLOCK_BYTES / 16)];
+      h1 = g[(size_t)lane * (GQF_BLOCK_BYTES / 16) + 1];
+    }
+    const uint64_t occ = (uint64_t)h0.x | (uint64_t)h0.y << 32, run = (uint64_t)h0.z | (uint64_t)h0.w << 32;
+    const uint64_t used = (uint64_t)h1.z | (uint64_t)h1.w << 32;
+    off_j = h1.x;
+    // slots [0, x0] of the window belong to earlier blocks' runs
+    const int32_t first = (int32_t)__builtin_amdgcn_readfirstlane((int)off_j);
+    auto from = [&](int32_t p) -> uint64_t {  // this block's slots at or after window slot p
+      const int32_t d = p - 64 * lane;
+      return d <= 0 ? ~0ULL : (d >= 64 ? 0ULL : ~0ULL << d);
+    };
+    const uint64_t own = used & from(first);
+    const uint32_t nr = (uint32_t)__popcll(run & own), no = (uint32_t)__popcll(occ);
+    const uint32_t rb = wave_scan_add(nr) - nr, ob = wave_scan_add(no) - no;
+    uint64_t part = own;
+    if (kRange) {
+      // the runs of quotients < q end at the k-th own run end, k = occupied
+      // quotients below q
+      bool inside = true;
+      auto end_before = [&](int32_t q) -> int32_t {  // first slot behind them
+        uint32_t k = 0;
+        if (q > 0) {
+          const int l = q < 64 * kWin ? q >> 6 : kWin - 1;
+          const uint64_t m = q < 64 * kWin ? (1ULL << (q & 63)) - 1 : ~0ULL;
+          k = (uint32_t)__builtin_amdgcn_readlane((int)(ob + (uint32_t)__popcll(occ & m)), l);
+        }
+        if (k == 0) return first;
+        const uint64_t has = __ballot(rb < k && k <= rb + nr);
+        if (!has) {
+          inside = false;
+          return 64 * kWin;
+        }
+        const int l = __builtin_ctzll(has);
+        const int32_t p = (rb < k && k <= rb + nr) ? 64 * lane + gqf_select64(run & own, (int)(k - rb) - 1) : 0;
+        return __builtin_amdgcn_readlane(p, l) + 1;
+      };
+      const int32_t lo = end_before(q_lo), hi = end_before(q_hi);
+      part = own & from(lo) & ~from(hi);
+      if (lane == 0) sm.over = inside ? 0u : 1u;
+    } else if (lane == 0) {
+      sm.over = 0;
+    }
+    sm.occ[lane] = occ;
+    sm.run[lane] = run;
+    sm.used[lane] = used;
+    sm.own[lane] = own;
+    sm.cont[lane] = own & (own << 1 | below_u64(own) >> 63) & ~(run << 1 | below_u64(run) >> 63);
+    sm.start[lane] = part;
+    sm.multi[lane] = 0;
+    sm.occ_new[lane] = 0;
+    sm.xblk[lane] = kNone;
+    sm.xold[lane] = 64 * lane - 1 + (int32_t)off_j;
+    sm.rbase[lane] = rb;
+    sm.obase[lane] = ob;
+    const bool any = __ballot(part != 0) != 0;
+    const uint32_t slots = (uint32_t)__popcll(part);
+    const uint32_t all = wave_scan_add(slots);
+    if (lane == 63) sm.n_slots = all;
+    if (lane == 0) {
+      sm.start[kWin] = 0;
+      sm.n_old = any ? 1u : 0u;
+      sm.any_multi = 0;
+      sm.n_big = 0;
+      sm.xend = (int32_t)off_j - 1;
+    }
+  }
+  ((uint2*)sm.sin)[tid] = x;
+  __syncthreads();
+  out.slots = x;
+  out.off = off_j;
+  out.x0 = sm.xold[0];
+  out.any = sm.n_old != 0;
+  out.n = 0;
+  if (out.x0 + 1 > nslots) return false;
+  if (kRange && sm.over) return false;
+  if (!out.any) return true;
+  const uint64_t below = (1ULL << sh) - 1;
+  // the occupied quotients by rank (the thread's eight quotients)
+  {
+    const uint64_t occ = sm.occ[j];
+    uint32_t k = sm.obase[j] + (uint32_t)__popcll(occ & below);
+    for (uint32_t b = (uint32_t)(occ >> sh) & 0xFFu; b; b &= b - 1)
+      sm.quot[k++] = (uint16_t)(64 * j + sh + __builtin_ctz(b));
+  }
+  // a byte not above its predecessor in the run: the run holds a counter
+  // of more than one slot
+  {
+    const uint32_t c = (uint32_t)((sm.cont[j] & sm.start[j]) >> sh) & 0xFFu;
+    uint32_t prev = tid ? sm.sin[8 * tid - 1] : 0u;
+    uint32_t viol = 0;
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      const uint32_t b = ((k < 4 ? x.x : x.y) >> (8 * (k & 3))) & 0xFFu;
+      viol |= b <= prev ? 1u << k : 0u;
+      prev = b;
+    }
+    for (viol &= c; viol; viol &= viol - 1) {
+      // the run starts behind the last run end or unused slot before the byte
+      const int at = sh + __builtin_ctz(viol);
+      int b = j;
+      uint64_t w = (sm.run[j] | ~sm.used[j]) & ((1ULL << at) - 1);
+      while (!w && b > 0) {
+        b--;
+        w = sm.run[b] | ~sm.used[b];
+      }
+      const int32_t rs = w ? 64 * b + 64 - __builtin_clzll(w) : 0;
+      atomicOr((unsigned long long*)&sm.multi[rs >> 6], 1ULL << (rs & 63));
+      sm.any_multi = 1;
+    }
+  }
+  __syncthreads();
+  if (sm.any_multi) {
+    for (uint32_t mb = (uint32_t)(sm.multi[j] >> sh) & 0xFFu; mb; mb &= mb - 1) {
+      const int32_t p = 8 * tid + __builtin_ctz(mb);
+      const uint32_t len = (uint32_t)(run_end_of(sm, p, nwin) - p + 1);
+      auto slot = [&](uint32_t k) -> uint64_t { return sm.sin[p + (int32_t)k]; };
+      for (uint32_t k = 0; k < len;) {
+        uint64_t rem, c;
+        const uint32_t last = gqf_decode_counter(slot, len, k, &rem, &c);
+        for (uint32_t y = k + 1; y <= last; y++) {
+          const int32_t q = p + (int32_t)y;
+          atomicAnd((unsigned long long*)&sm.start[q >> 6], ~(1ULL << (q & 63)));
+        }
+        k = last + 1;
+      }
+    }
+    __syncthreads();
+  }
+  if (wave == 0) {
+    const uint32_t n = (uint32_t)__popcll(sm.start[lane]);
+    const uint32_t incl = wave_scan_add(n);
+    sm.ebase[lane] = incl - n;
+    if (lane == 63) sm.n_old = incl;
+  }
+  __syncthreads();
+  out.n = sm.n_old;
+  {
+    const uint64_t st = sm.start[j], own = sm.own[j], run = sm.run[j] & own;
+    const uint32_t e0 = sm.ebase[j] + (uint32_t)__popcll(st & below);
+    const uint32_t k0 = sm.rbase[j] + (uint32_t)__popcll(run & below);
+    const uint32_t stb = (uint32_t)(st >> sh) & 0xFFu, runb = (uint32_t)(run >> sh) & 0xFFu;
+    // slots whose next slot continues their counter
+    const uint64_t inner = own & ~st;
+    const uint32_t nextb = (uint32_t)((inner >> sh) >> 1) & 0x7Fu;
+    const uint32_t after = sh < 56 ? (uint32_t)(inner >> (sh + 8)) & 1u
+                                   : (j + 1 < nwin ? (uint32_t)(sm.own[j + 1] & ~sm.start[j + 1]) & 1u : 0u);
+    const uint32_t moreb = stb & ~runb & (nextb | after << 7);
+    uint32_t q[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+      if ((stb >> i) & 1u) q[i] = sm.quot[k0 + (uint32_t)__builtin_popcount(runb & ((1u << i) - 1))];
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const uint32_t ei = e0 + (uint32_t)__builtin_popcount(stb & ((1u << i) - 1));
+      if ((stb >> i) & 1u) {
+        const uint32_t h = q[i] << 8 | (((i < 4 ? x.x : x.y) >> (8 * (i & 3))) & 0xFFu);
+        uint32_t aux = 1;
+        if ((moreb >> i) & 1u) {
+          const int32_t p = 8 * tid + i;
+          const uint32_t len = (uint32_t)(run_end_of(sm, p, nwin) - p + 1);
+          uint64_t rem, c;
+          gqf_decode_counter([&](uint32_t k) -> uint64_t { return sm.sin[p + (int32_t)k]; }, len, 0, &rem, &c);
+          aux = push_count(sm, h, c);
+        }
+        sm.old[ei] = h << 12 | aux;
+      }
+      if ((runb >> i) & 1u)
+        sm.rend[k0 + (uint32_t)__builtin_popcount(runb & ((1u << i) - 1))] = (uint16_t)(ei + ((stb >> i) & 1u));
+    }
+  }
+  __syncthreads();
+  return true;
+}
+
 // Rebuilds region r of `qf` with its items [s, e) of `items` (sorted hashes
 // + tag; per-item counts for kCounts).  All kThreads threads call it; nothing
 // is written unless it returns kOk.  Window and result as rebuild_region
@@ -177,156 +383,15 @@ __device__ __forceinline__ int rebuild(const QF& qf, uint64_t r, const uint64_t*
   const uint64_t hmask = kind == kTagged ? GQF_SEQ_HASH_MASK : ~0ULL;
   const uint64_t base = tag + (B0 << 14);
 
-  // ---- the window: thread t holds slots 8 t .. 8 t + 7 (eight threads a
-  // block); wave 0 the headers, a block a lane
-  const int j = tid >> 3, sh = (tid & 7) * 8;
-  const GQF_GLOBAL uint4* g = gqf_block_ptr(qf, B0);
-  uint2 x = make_uint2(0, 0);
-  if (j < nwin) x = ((const GQF_GLOBAL uint2*)(g + (size_t)j * (GQF_BLOCK_BYTES / 16) + 4))[tid & 7];
-  uint32_t off_j = 0;  // wave 0: block `lane`'s old offset
-  if (wave == 0) {
-    uint4 h0 = make_uint4(0, 0, 0, 0), h1 = h0;
-    if (lane < nwin) {
-      h0 = g[(size_t)lane * (GQF_BLOCK_BYTES / 16)];
-      h1 = g[(size_t)lane * (GQF_BLOCK_BYTES / 16) + 1];
-    }
-    const uint64_t occ = (uint64_t)h0.x | (uint64_t)h0.y << 32, run = (uint64_t)h0.z | (uint64_t)h0.w << 32;
-    const uint64_t used = (uint64_t)h1.z | (uint64_t)h1.w << 32;
-    off_j = h1.x;
-    // slots [0, x0] of the window belong to earlier regions' runs
-    const int32_t spill = (int32_t)__builtin_amdgcn_readfirstlane((int)off_j) - 64 * lane;
-    const uint64_t mine = spill <= 0 ? ~0ULL : (spill >= 64 ? 0ULL : ~0ULL << spill);
-    const uint64_t own = used & mine;
-    const uint32_t nr = (uint32_t)__popcll(run & own), no = (uint32_t)__popcll(occ);
-    sm.occ[lane] = occ;
-    sm.run[lane] = run;
-    sm.used[lane] = used;
-    sm.own[lane] = own;
-    sm.cont[lane] = own & (own << 1 | below_u64(own) >> 63) & ~(run << 1 | below_u64(run) >> 63);
-    sm.start[lane] = own;
-    sm.multi[lane] = 0;
-    sm.occ_new[lane] = 0;
-    sm.xblk[lane] = kNone;
-    sm.xold[lane] = 64 * lane - 1 + (int32_t)off_j;
-    sm.rbase[lane] = wave_scan_add(nr) - nr;
-    sm.obase[lane] = wave_scan_add(no) - no;
-    const bool any = __ballot(own != 0) != 0;
-    if (lane == 0) {
-      sm.start[kWin] = 0;
-      sm.n_old = any ? 1u : 0u;
-      sm.any_multi = 0;
-      sm.n_big = 0;
-      sm.over = 0;
-      sm.xend = (int32_t)off_j - 1;
-    }
-  }
-  ((uint2*)sm.sin)[tid] = x;
   for (int k = tid; k < kSlots / 2 + 1; k += kThreads) sm.place[k] = 0;
-  __syncthreads();
-  const int32_t x0 = sm.xold[0];
-  if (x0 + 1 > nslots) return kNeedWide;  // spill-in longer than the window
-  const bool any_old = sm.n_old != 0;
-  const uint64_t below = (1ULL << sh) - 1;
-
-  // ---- 1. old entries
-  uint32_t n_old = 0;
-  if (any_old) {
-    // the occupied quotients by rank (the thread's eight quotients)
-    {
-      const uint64_t occ = sm.occ[j];
-      uint32_t k = sm.obase[j] + (uint32_t)__popcll(occ & below);
-      for (uint32_t b = (uint32_t)(occ >> sh) & 0xFFu; b; b &= b - 1)
-        sm.quot[k++] = (uint16_t)(64 * j + sh + __builtin_ctz(b));
-    }
-    // a byte not above its predecessor in the run: the run holds a counter
-    // of more than one slot
-    {
-      const uint32_t c = (uint32_t)(sm.cont[j] >> sh) & 0xFFu;
-      uint32_t prev = tid ? sm.sin[8 * tid - 1] : 0u;
-      uint32_t viol = 0;
-#pragma unroll
-      for (int k = 0; k < 8; k++) {
-        const uint32_t b = ((k < 4 ? x.x : x.y) >> (8 * (k & 3))) & 0xFFu;
-        viol |= b <= prev ? 1u << k : 0u;
-        prev = b;
-      }
-      for (viol &= c; viol; viol &= viol - 1) {
-        // the run starts behind the last run end or unused slot before the byte
-        const int at = sh + __builtin_ctz(viol);
-        int b = j;
-        uint64_t w = (sm.run[j] | ~sm.used[j]) & ((1ULL << at) - 1);
-        while (!w && b > 0) {
-          b--;
-          w = sm.run[b] | ~sm.used[b];
-        }
-        const int32_t rs = w ? 64 * b + 64 - __builtin_clzll(w) : 0;
-        atomicOr((unsigned long long*)&sm.multi[rs >> 6], 1ULL << (rs & 63));
-        sm.any_multi = 1;
-      }
-    }
-    __syncthreads();
-    if (sm.any_multi) {
-      for (uint32_t mb = (uint32_t)(sm.multi[j] >> sh) & 0xFFu; mb; mb &= mb - 1) {
-        const int32_t p = 8 * tid + __builtin_ctz(mb);
-        const uint32_t len = (uint32_t)(run_end_of(sm, p, nwin) - p + 1);
-        auto slot = [&](uint32_t k) -> uint64_t { return sm.sin[p + (int32_t)k]; };
-        for (uint32_t k = 0; k < len;) {
-          uint64_t rem, c;
-          const uint32_t last = gqf_decode_counter(slot, len, k, &rem, &c);
-          for (uint32_t y = k + 1; y <= last; y++) {
-            const int32_t q = p + (int32_t)y;
-            atomicAnd((unsigned long long*)&sm.start[q >> 6], ~(1ULL << (q & 63)));
-          }
-          k = last + 1;
-        }
-      }
-      __syncthreads();
-    }
-    if (wave == 0) {
-      const uint32_t n = (uint32_t)__popcll(sm.start[lane]);
-      const uint32_t incl = wave_scan_add(n);
-      sm.ebase[lane] = incl - n;
-      if (lane == 63) sm.n_old = incl;
-    }
-    __syncthreads();
-    n_old = sm.n_old;
-    {
-      const uint64_t st = sm.start[j], own = sm.own[j], run = sm.run[j] & own;
-      const uint32_t e0 = sm.ebase[j] + (uint32_t)__popcll(st & below);
-      const uint32_t k0 = sm.rbase[j] + (uint32_t)__popcll(run & below);
-      const uint32_t stb = (uint32_t)(st >> sh) & 0xFFu, runb = (uint32_t)(run >> sh) & 0xFFu;
-      // slots whose next slot continues their counter
-      const uint64_t inner = own & ~st;
-      const uint32_t nextb = (uint32_t)((inner >> sh) >> 1) & 0x7Fu;
-      const uint32_t after = sh < 56 ? (uint32_t)(inner >> (sh + 8)) & 1u
-                                     : (j + 1 < nwin ? (uint32_t)(sm.own[j + 1] & ~sm.start[j + 1]) & 1u : 0u);
-      const uint32_t moreb = stb & (nextb | after << 7);
-      uint32_t q[8];
-#pragma unroll
-      for (int i = 0; i < 8; i++)
-        if ((stb >> i) & 1u) q[i] = sm.quot[k0 + (uint32_t)__builtin_popcount(runb & ((1u << i) - 1))];
-#pragma unroll
-      for (int i = 0; i < 8; i++) {
-        const uint32_t ei = e0 + (uint32_t)__builtin_popcount(stb & ((1u << i) - 1));
-        if ((stb >> i) & 1u) {
-          const uint32_t h = q[i] << 8 | (((i < 4 ? x.x : x.y) >> (8 * (i & 3))) & 0xFFu);
-          uint32_t aux = 1;
-          if ((moreb >> i) & 1u) {
-            const int32_t p = 8 * tid + i;
-            const uint32_t len = (uint32_t)(run_end_of(sm, p, nwin) - p + 1);
-            uint64_t rem, c;
-            gqf_decode_counter([&](uint32_t k) -> uint64_t { return sm.sin[p + (int32_t)k]; }, len, 0, &rem, &c);
-            aux = push_count(sm, h, c);
-          }
-          sm.old[ei] = h << 12 | aux;
-        }
-        if ((runb >> i) & 1u)
-          sm.rend[k0 + (uint32_t)__builtin_popcount(runb & ((1u << i) - 1))] =
-              (uint16_t)(ei + ((stb >> i) & 1u));
-      }
-    }
-    __syncthreads();
-  }
+  Window w;
+  if (!window_entries<false>(qf, B0, nwin, 0, 0, sm, w)) return kNeedWide;  // spill-in longer than the window
+  const int j = tid >> 3, sh = (tid & 7) * 8;
+  const uint2 x = w.slots;
+  const uint32_t off_j = w.off;
+  const int32_t x0 = w.x0;
+  const bool any_old = w.any;
+  const uint32_t n_old = w.n;
   const uint32_t big_old = sm.n_big;
   __syncthreads();
 

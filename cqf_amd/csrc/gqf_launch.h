@@ -164,31 +164,34 @@ void gqf_launch_point_query(QF* qf_dev, const uint64_t* keys, uint64_t n, uint8_
 void gqf_launch_splitmix64(uint64_t* out, uint64_t n, uint64_t seed, uint64_t skip, hipStream_t s);
 
 // ---------------------------------------------------------------------------
-// Whole-table passes (gqf_enum.hip).  One thread per table block, 256
-// blocks per workgroup.
-
-#define GQF_ENUM_WG_BLOCKS 256  // table blocks per workgroup of these passes
+// Whole-table passes (gqf_enum.hip).  An enumeration's quotients are taken in
+// groups of GQF_ENUM_BLOCKS blocks', a workgroup each.
+#define GQF_ENUM_BLOCKS 62
 // output forms of the enumeration write pass
 enum { GQF_ENUM_OUT_HASH = 0, GQF_ENUM_OUT_KEY = 1, GQF_ENUM_OUT_MOVE = 2 };
-uint64_t gqf_enum_wg_count(uint64_t nblocks);
-// count pass over blocks [b_lo, b_hi), items of quotients [q_lo, q_hi):
-// items per workgroup -> wg_items, their exclusive prefix sums -> wg_base
-// (nwg + 1 entries, the last the total); stats[0..2] += items, sum of
-// counts, slots used by the runs.  With `starts` (zeroed, one word per
-// block from b_lo to the end of the table) it also sets the bit of every
-// item's first slot and raises *max_word to the last word it marked.
+uint64_t gqf_enum_groups(uint64_t nblocks);
+// items, used slots and sums of counts of every group, the groups' first
+// ranks (groups + 1, the last the total), stats[0..2] = items, sum of counts,
+// used slots
+struct gqf_enum_tables {
+  uint32_t* items = nullptr;
+  uint32_t* slots = nullptr;
+  uint64_t* sums = nullptr;
+  uint64_t* base = nullptr;
+  uint64_t* stats = nullptr;
+};
+// count pass over the items of quotients [q_lo, q_hi), all in blocks [b_lo, b_hi)
 void gqf_launch_enum_count(const QF* qf_dev, uint64_t b_lo, uint64_t b_hi, uint64_t q_lo, uint64_t q_hi,
-                           uint32_t* wg_items, uint64_t* wg_base, unsigned long long* stats,
-                           unsigned long long* starts, unsigned long long* max_word, hipStream_t s);
-// write pass over those marks (words w_lo .. w_lo + nwords): the item whose
-// counter starts at the r-th mark -> hashes[r] / counts[r] / values[r] when
-// r < cap, in the form `mode` (MOVE: the slot hash the item has in a filter
-// with dst_vb value bits); clears the marks.  Scratch: local_prefix nwords
-// words, group_sums and group_base (+1) one per 256 words.
-void gqf_launch_enum_emit(const QF* qf_dev, uint64_t w_lo, uint64_t nwords, unsigned long long* starts,
-                          const unsigned long long* max_word, uint32_t* local_prefix, uint32_t* group_sums,
-                          uint64_t* group_base, int mode, int vb, int dst_vb, uint64_t key_mask, uint64_t* hashes,
-                          uint64_t* counts, uint64_t* values, uint64_t cap, hipStream_t s);
+                           const gqf_enum_tables& t, hipStream_t s);
+// write pass over groups [u0, u1) of the same ranges, with the count pass's
+// first ranks: item i -> hashes[i - skip] / counts[..] / values[..] where that
+// index is below cap, in the form `mode` (MOVE: the slot hash the item has in
+// a filter with dst_vb value bits)
+void gqf_launch_enum_emit(const QF* qf_dev, uint64_t b_lo, uint64_t b_hi, uint64_t q_lo, uint64_t q_hi, uint64_t u0,
+                          uint64_t u1, const uint64_t* base, uint64_t skip, int mode, int vb, int dst_vb,
+                          uint64_t key_mask, uint64_t* hashes, uint64_t* counts, uint64_t* values, uint64_t cap,
+                          hipStream_t s);
+uint64_t gqf_census_wgs(uint64_t nblocks);
 // cluster census: used-slot masks (nblocks words), cluster starts per
 // workgroup and their bases (nwg + 1, the last = number of clusters);
 // lengths[rank] (rank < cap), hist[min(len, nbins - 1)] += 1 (nbins <= 4096,
