@@ -136,12 +136,15 @@ static __device__ inline uint64_t form_hash(const gqf_out_form& o, uint64_t s) {
 constexpr int kGroupWaves = gqf_flat::kThreads / 64;
 static_assert(GQF_ENUM_BLOCKS < gqf_flat::kWin, "blocks of the window past the group's");
 
+struct CountSmem : gqf_flat::Head {
+  alignas(16) uint8_t sin[gqf_flat::kSlots];
+  uint64_t sums[kGroupWaves];
+};
 struct EnumSmem : gqf_flat::Head {
   alignas(16) uint8_t sin[gqf_flat::kSlots];
   uint16_t rend[gqf_flat::kSlots];
   uint16_t quot[gqf_flat::kSlots];
   uint32_t old[gqf_flat::kSlots];
-  uint64_t sums[kGroupWaves];
 };
 
 struct EnumRange {
@@ -150,14 +153,15 @@ struct EnumRange {
 
 // Makes group u's entries; false where they do not fit the window or its
 // table of large counts.  b0: the group's first block.
-static __device__ __forceinline__ bool group_entries(const QF& f, const EnumRange& r, uint64_t u, EnumSmem& sm,
+template <bool kStore, class S>
+static __device__ __forceinline__ bool group_entries(const QF& f, const EnumRange& r, uint64_t u, S& sm,
                                                      gqf_flat::Window& w, uint64_t& b0) {
   b0 = r.b_lo + u * GQF_ENUM_BLOCKS;
   const int nwin = (int)min((uint64_t)gqf_flat::kWin, f.nblocks - b0);
   const uint64_t q0 = b0 * 64;
   const int32_t lo = r.q_lo > q0 ? (int32_t)min(r.q_lo - q0, (uint64_t)(64 * GQF_ENUM_BLOCKS)) : 0;
   const uint64_t end = min(min((uint64_t)(64 * GQF_ENUM_BLOCKS), 64 * (r.b_hi - b0)), r.q_hi > q0 ? r.q_hi - q0 : 0ULL);
-  return gqf_flat::window_entries<true>(f, b0, nwin, lo, (int32_t)min(end, (uint64_t)(64 * nwin)), sm, w) && !sm.over;
+  return gqf_flat::window_entries<true, kStore>(f, b0, nwin, lo, (int32_t)min(end, (uint64_t)(64 * nwin)), sm, w) && !sm.over;
 }
 
 // The group's items block by block, from the table (wave 0, a block a lane):
@@ -183,28 +187,22 @@ static __device__ inline uint32_t walk_group(const QF& f, const EnumRange& r, ui
 extern "C" __global__ void __launch_bounds__(gqf_flat::kThreads)
 gqf_enum_count(const QF* __restrict__ qfp, EnumRange r, uint32_t* __restrict__ items, uint32_t* __restrict__ slots,
                uint64_t* __restrict__ sums) {
-  __shared__ EnumSmem sm;
+  __shared__ CountSmem sm;
   const QF& f = *qfp;
   const uint64_t u = blockIdx.x;
   const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   gqf_flat::Window w;
   uint64_t b0;
-  const bool fits = group_entries(f, r, u, sm, w, b0);
+  const bool fits = group_entries<false>(f, r, u, sm, w, b0);
   if (fits) {
-    uint64_t sum = 0;
+    uint64_t sum = w.n;
     if (sm.any_multi) {  // else every entry counts one
-      const uint32_t nbig = sm.n_big;
-      for (uint32_t e = tid; e < w.n; e += gqf_flat::kThreads) {
-        const uint32_t y = sm.old[e];
-        sum += gqf_flat::full_count(sm, y >> 12, y & 0xFFFu, nbig);
-      }
+      sum = w.sum;
       for (int d = 32; d >= 1; d >>= 1) sum += __shfl_xor(sum, d, 64);
       if (lane == 0) sm.sums[wave] = sum;
       __syncthreads();
       sum = 0;
       for (int k = 0; k < kGroupWaves; k++) sum += sm.sums[k];
-    } else {
-      sum = w.n;
     }
     if (tid == 0) {
       items[u] = w.n;
@@ -313,7 +311,7 @@ gqf_enum_emit(const QF* __restrict__ qfp, EnumRange r, uint64_t u0, const uint64
   if (base[u + 1] == base[u] || first >= cap) return;
   gqf_flat::Window w;
   uint64_t b0;
-  const bool fits = group_entries(f, r, u, sm, w, b0);
+  const bool fits = group_entries<true>(f, r, u, sm, w, b0);
   auto put = [&](uint64_t i, uint64_t s, uint64_t c) {
     if (i >= cap) return;
     if (hashes) hashes[i] = form_hash(o, s);

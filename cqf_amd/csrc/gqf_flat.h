@@ -15,8 +15,7 @@
 //      the run's counter starts first;
 //   2. every distinct item hash finds its place among the old entries of its
 //      quotient's run; an entry that is there takes the new count, the others
-//      are inserted: entry e moves up by the number of items placed before
-//      it (a histogram and a prefix sum);
+//      get a place among them (a bit map of the merged sequence);
 //   3. with L(e) slots per entry and S(e) the slots of the entries before it,
 //      entry e starts at S(e) + max over e' <= e of (quotient(e') - S(e')):
 //      each entry starts at its quotient or behind its predecessor, whichever
@@ -51,7 +50,7 @@ constexpr int kWin = 64;                 // window blocks: the region and its pu
 constexpr int kSlots = kWin * 64;
 constexpr int kPer = kSlots / kThreads;  // slots per thread
 static_assert(kPer == 8, "a thread's slots are one 8-byte word of its block");
-constexpr int kCap = 7168;               // merged entries: a full window's and a full region's items
+constexpr int kItems = 3968;             // items of a region held as entries (with more, three workgroups would not fit a CU)
 constexpr int kBig = 64;                 // counts of kAuxBig or more in a window
 constexpr uint32_t kAuxBig = 4095;       // a larger count is in the big table
 constexpr int32_t kNone = INT32_MIN / 4;
@@ -84,18 +83,21 @@ struct Head {
   uint64_t big_count[kBig];
 };
 
+constexpr int kSeqWords = (kSlots + kItems + 31) / 32;
+
 struct Smem : Head {
   alignas(16) uint8_t sin[kSlots];  // old slots
-  uint16_t rend[kSlots];            // old entries of the runs of rank <= k
+  uint32_t old[kSlots];             // old entries, hash << 12 | min(count, kAuxBig)
   union {
-    uint32_t old[kSlots];             // old entries, hash << 12 | min(count, kAuxBig)
-    alignas(16) uint16_t out[kSlots + 8];  // the new slots, once the entries are merged
+    uint16_t rend[kSlots];          // old entries of the runs of rank <= k
+    alignas(16) uint16_t out[kSlots + 8];  // the new slots, once the items have their places
   };
   union {
-    uint16_t quot[kSlots];            // the occupied quotients by rank (until the entries are made)
-    uint32_t m[kCap];                 // merged entries
+    uint16_t quot[kSlots];          // the occupied quotients by rank (until the entries are made)
+    uint32_t item[kItems];          // the items' entries
   };
-  uint32_t place[kSlots / 2 + 1];   // 16-bit counts: items placed before old entry e
+  uint32_t is_item[kSeqWords];      // places of the merged sequence that items take
+  uint32_t items_before[kSeqWords]; // items in earlier words of it
 };
 
 __device__ __forceinline__ int32_t max_i(int32_t a, int32_t b) { return a > b ? a : b; }
@@ -168,6 +170,7 @@ struct Window {
   int32_t x0;
   bool any;     // some run of the window's quotients
   uint32_t n;   // entries
+  uint64_t sum; // !kStore: the counts of the entries in the thread's slots
 };
 
 // 1. Loads the window of nwin blocks from block B0 and makes the entries of
@@ -175,7 +178,9 @@ struct Window {
 // kRange: only the runs of quotients [q_lo, q_hi) of the window (which must
 // end inside it).  All kThreads threads call it.  Returns false if the runs of
 // earlier blocks, or those of the range, reach past the window.
-template <bool kRange, class S>
+// kStore: make the entries; else only count them, with the sum of this thread's
+// counts in out.sum (no quotients needed: sm has no quot, old and rend then).
+template <bool kRange, bool kStore, class S>
 __device__ __forceinline__ bool window_entries(const QF& qf, uint64_t B0, int nwin, int32_t q_lo, int32_t q_hi, S& sm,
                                                Window& out) {
   const int tid = (int)threadIdx.x;
@@ -264,12 +269,13 @@ __device__ __forceinline__ bool window_entries(const QF& qf, uint64_t B0, int nw
   out.x0 = sm.xold[0];
   out.any = sm.n_old != 0;
   out.n = 0;
+  out.sum = 0;
   if (out.x0 + 1 > nslots) return false;
   if (kRange && sm.over) return false;
   if (!out.any) return true;
   const uint64_t below = (1ULL << sh) - 1;
   // the occupied quotients by rank (the thread's eight quotients)
-  {
+  if constexpr (kStore) {
     const uint64_t occ = sm.occ[j];
     uint32_t k = sm.obase[j] + (uint32_t)__popcll(occ & below);
     for (uint32_t b = (uint32_t)(occ >> sh) & 0xFFu; b; b &= b - 1)
@@ -338,6 +344,17 @@ __device__ __forceinline__ bool window_entries(const QF& qf, uint64_t B0, int nw
     const uint32_t after = sh < 56 ? (uint32_t)(inner >> (sh + 8)) & 1u
                                    : (j + 1 < nwin ? (uint32_t)(sm.own[j + 1] & ~sm.start[j + 1]) & 1u : 0u);
     const uint32_t moreb = stb & ~runb & (nextb | after << 7);
+    auto count_at = [&](int32_t p) -> uint64_t {  // of the counter of several slots at slot p
+      const uint32_t len = (uint32_t)(run_end_of(sm, p, nwin) - p + 1);
+      uint64_t rem, c;
+      gqf_decode_counter([&](uint32_t k) -> uint64_t { return sm.sin[p + (int32_t)k]; }, len, 0, &rem, &c);
+      return c;
+    };
+    if constexpr (!kStore) {
+      out.sum = (uint64_t)__builtin_popcount(stb & ~moreb);
+      for (uint32_t m = moreb; m; m &= m - 1) out.sum += count_at(8 * tid + __builtin_ctz(m));
+      return true;
+    } else {
     uint32_t q[8];
 #pragma unroll
     for (int i = 0; i < 8; i++)
@@ -348,17 +365,12 @@ __device__ __forceinline__ bool window_entries(const QF& qf, uint64_t B0, int nw
       if ((stb >> i) & 1u) {
         const uint32_t h = q[i] << 8 | (((i < 4 ? x.x : x.y) >> (8 * (i & 3))) & 0xFFu);
         uint32_t aux = 1;
-        if ((moreb >> i) & 1u) {
-          const int32_t p = 8 * tid + i;
-          const uint32_t len = (uint32_t)(run_end_of(sm, p, nwin) - p + 1);
-          uint64_t rem, c;
-          gqf_decode_counter([&](uint32_t k) -> uint64_t { return sm.sin[p + (int32_t)k]; }, len, 0, &rem, &c);
-          aux = push_count(sm, h, c);
-        }
+        if ((moreb >> i) & 1u) aux = push_count(sm, h, count_at(8 * tid + i));
         sm.old[ei] = h << 12 | aux;
       }
       if ((runb >> i) & 1u)
         sm.rend[k0 + (uint32_t)__builtin_popcount(runb & ((1u << i) - 1))] = (uint16_t)(ei + ((stb >> i) & 1u));
+    }
     }
   }
   __syncthreads();
@@ -383,9 +395,9 @@ __device__ __forceinline__ int rebuild(const QF& qf, uint64_t r, const uint64_t*
   const uint64_t hmask = kind == kTagged ? GQF_SEQ_HASH_MASK : ~0ULL;
   const uint64_t base = tag + (B0 << 14);
 
-  for (int k = tid; k < kSlots / 2 + 1; k += kThreads) sm.place[k] = 0;
+  for (int k = tid; k < kSeqWords; k += kThreads) sm.is_item[k] = 0;
   Window w;
-  if (!window_entries<false>(qf, B0, nwin, 0, 0, sm, w)) return kNeedWide;  // spill-in longer than the window
+  if (!window_entries<false, true>(qf, B0, nwin, 0, 0, sm, w)) return kNeedWide;  // spill-in longer than the window
   const int j = tid >> 3, sh = (tid & 7) * 8;
   const uint2 x = w.slots;
   const uint32_t off_j = w.off;
@@ -395,11 +407,11 @@ __device__ __forceinline__ int rebuild(const QF& qf, uint64_t r, const uint64_t*
   const uint32_t big_old = sm.n_big;
   __syncthreads();
 
-  // ---- 2. the items, each wave a contiguous share, 64 at a time.  An item
-  // takes the place (its ordinal + the old entries before it) in the merged
-  // sequence; a repeat, or an item whose hash has an old entry, leaves its
-  // place empty.  Where that would not fit the sequence, the ordinals count
-  // distinct hashes only.
+  // ---- 2. the items, each wave a contiguous share, 64 at a time.  Item k
+  // becomes entry k of sm.item and takes the place (k + the old entries before
+  // it) in the merged sequence, marked in sm.is_item; a repeat, or an item
+  // whose hash has an old entry, is an empty entry.  Where the entries would
+  // not hold all items, the ordinals count distinct hashes only.
   const uint64_t n_items = e - s;
   const uint64_t share = ((n_items + kThreads - 1) / kThreads) * 64;
   const uint64_t i0 = s + min(n_items, share * (uint64_t)wave), i1 = s + min(n_items, share * (uint64_t)(wave + 1));
@@ -410,7 +422,7 @@ __device__ __forceinline__ int rebuild(const QF& qf, uint64_t r, const uint64_t*
     return i < i1 && (i == s || prev != v);
   };
   uint32_t ord = (uint32_t)(i0 - s), n_new = (uint32_t)n_items;  // ordinal of the wave's next item, all ordinals
-  const bool sparse = n_old + n_items > (uint64_t)kCap;
+  const bool sparse = n_items > (uint64_t)kItems;
   if (sparse) {
     uint32_t heads = 0;
     for (uint64_t i = i0; i < i1; i += 64) {
@@ -425,7 +437,7 @@ __device__ __forceinline__ int rebuild(const QF& qf, uint64_t r, const uint64_t*
       ord += w < wave ? c : 0u;
       n_new += c;
     }
-    if (n_old + n_new > (uint32_t)kCap) return kNeedWide;
+    if (n_new > (uint32_t)kItems) return kNeedWide;
   }
   for (uint64_t i = i0; i < i1; i += 64) {
     const uint64_t ii = i + (uint64_t)lane;
@@ -498,57 +510,71 @@ __device__ __forceinline__ int rebuild(const QF& qf, uint64_t r, const uint64_t*
       }
       const uint32_t k = sparse ? ord + (uint32_t)__popcll(hm & ((1ULL << lane) - 1)) : ord + (uint32_t)lane;
       const uint32_t at = lo + (there ? 1u : 0u);
-      sm.m[k + at] = entry;
-      atomicAdd(&sm.place[at >> 1], 1u << (16 * (at & 1)));
+      sm.item[k] = entry;
+      atomicOr(&sm.is_item[(k + at) >> 5], 1u << ((k + at) & 31));
     }
     ord += sparse ? (uint32_t)__popcll(hm) : 64u;
   }
   __syncthreads();
   if (sm.over) return kNeedWide;
 
-  // ---- the old entries' places.  From here on a thread takes an odd number
-  // of consecutive entries (odd strides spread the lanes over the LDS banks):
-  // it adds them up by itself, and one scan over the threads places its share.
+  // ---- the merged sequence: place i holds item k, k = items marked before
+  // it, or old entry i - k
   const uint32_t n_all = n_old + n_new;
-  auto scan_add = [&](uint32_t v, int buf) -> uint32_t {  // exclusive, over the workgroup; one barrier
+  if (wave == 0) {
+    constexpr int kW = (kSeqWords + 63) / 64;  // words a lane
+    uint32_t c[kW], sum = 0;
+#pragma unroll
+    for (int k = 0; k < kW; k++) {
+      c[k] = kW * lane + k < kSeqWords ? (uint32_t)__popc(sm.is_item[kW * lane + k]) : 0u;
+      sum += c[k];
+    }
+    uint32_t before = wave_scan_add(sum) - sum;
+#pragma unroll
+    for (int k = 0; k < kW; k++) {
+      if (kW * lane + k < kSeqWords) sm.items_before[kW * lane + k] = before;
+      before += c[k];
+    }
+  }
+  auto scan_add = [&](uint32_t v) -> uint32_t {  // exclusive, over the workgroup; one barrier
     const uint32_t incl = wave_scan_add(v);
-    if (lane == 63) sm.wsum[buf][wave] = incl;
+    if (lane == 63) sm.wsum[1][wave] = incl;
     __syncthreads();
     uint32_t before = incl - v;
 #pragma unroll
-    for (int w = 0; w < kWaves; w++) before += w < wave ? sm.wsum[buf][w] : 0u;
+    for (int w = 0; w < kWaves; w++) before += w < wave ? sm.wsum[1][w] : 0u;
     return before;
   };
-  if (n_old) {
-    const uint32_t per = ((n_old + kThreads - 1) / kThreads) | 1u;
-    const uint32_t a = min(n_old, per * (uint32_t)tid), b = min(n_old, a + per);
-    auto placed = [&](uint32_t i) { return (sm.place[i >> 1] >> (16 * (i & 1))) & 0xFFFFu; };
-    uint32_t sum = 0;
-    for (uint32_t i = a; i < b; i++) sum += placed(i);
-    uint32_t at = scan_add(sum, 0);
-    for (uint32_t i = a; i < b; i++) {
-      at += placed(i);
-      sm.m[i + at] = sm.old[i];
-    }
-    __syncthreads();
-  }
-  const uint32_t* seq = sm.m;
   uint16_t* out = sm.out;  // new slots: byte | 1 << 8 | (first of its run) << 9
   const uint32_t n_big = sm.n_big;
   ((uint4*)out)[tid] = make_uint4(0, 0, 0, 0);
+  __syncthreads();
 
-  // ---- 3. positions
+  // ---- 3. positions.  A thread takes an odd number of consecutive places (odd
+  // strides spread the lanes over the LDS banks): it adds them up by itself,
+  // and one scan over the threads places its share.
   {
     const uint32_t per = ((n_all + kThreads - 1) / kThreads) | 1u;
     const uint32_t a = min(n_all, per * (uint32_t)tid), b = min(n_all, a + per);
+    const uint32_t ka = a < n_all ? sm.items_before[a >> 5] +
+                                        (uint32_t)__popc(sm.is_item[a >> 5] & ((1u << (a & 31)) - 1))
+                                  : 0u;
+    // the entry at place i, k items before it
+    auto entry_at = [&](uint32_t i, uint32_t& k) -> uint32_t {
+      const bool item = (sm.is_item[i >> 5] >> (i & 31)) & 1u;
+      const uint32_t y = item ? sm.item[k] : sm.old[i - k];
+      k += item ? 1u : 0u;
+      return y;
+    };
     auto slots_of = [&](uint32_t y) -> uint32_t {
       const uint32_t rem = (y >> 12) & 0xFFu, aux = y & 0xFFFu;
       return aux < kAuxBig ? entry_len(rem, aux) : gqf_counter_len(rem, full_count(sm, y >> 12, aux, n_big));
     };
     uint32_t sum = 0;
     int32_t lead = kNone, lastq = -1;  // max of quotient - slots before it in the share; the last quotient
+    uint32_t ki = ka;
     for (uint32_t i = a; i < b; i++) {
-      const uint32_t y = seq[i];
+      const uint32_t y = entry_at(i, ki);
       const uint32_t len = slots_of(y);
       const int32_t q = (int32_t)(y >> 20);
       if (len) {
@@ -557,7 +583,7 @@ __device__ __forceinline__ int rebuild(const QF& qf, uint64_t r, const uint64_t*
       }
       sum += len;
     }
-    uint32_t before = scan_add(sum, 1);
+    uint32_t before = scan_add(sum);
     // the same over the threads before this one: largest quotient - slots
     // before it, and the last quotient (they ascend)
     const int32_t li = wave_scan_max(lead == kNone ? kNone : lead - (int32_t)before), qi = wave_scan_max(lastq);
@@ -574,8 +600,9 @@ __device__ __forceinline__ int rebuild(const QF& qf, uint64_t r, const uint64_t*
       lastq = w < wave ? max_i(lastq, sm.wmax[1][w]) : lastq;
     }
     int32_t last = kNone, blk = -1;  // last new slot, of quotients of block blk
+    ki = ka;
     for (uint32_t i = a; i < b; i++) {
-      const uint32_t y = seq[i];
+      const uint32_t y = entry_at(i, ki);
       const uint32_t len = slots_of(y);
       if (!len) continue;
       const int32_t q = (int32_t)(y >> 20);
