@@ -44,7 +44,7 @@ namespace {
 constexpr int kWinFast = 64;          // region blocks + push blocks
 constexpr int kWinMid = 128;          // first fallback window (80 push blocks)
 constexpr int kWinWide = 256;         // last fallback window (208 push blocks)
-constexpr int kWideClassGrid = 256;  // workgroups of a class launch of the wide pass
+constexpr int kWideClassGrid = 256;  // workgroups of a stage of the wide pass
 constexpr int kItemCap = 256;         // items cached in LDS per region (fast path): 192 +- 14 at 2^24 keys into 2^28 slots
 constexpr int32_t kNegInf = INT32_MIN / 4;
 
@@ -1170,33 +1170,49 @@ __device__ __forceinline__ int rebuild_insert_shift(const QF& qf, uint64_t B0, i
 }
 
 // ---------------------------------------------------------------------------
-// A region's window lines and cached items, in registers: lane j holds
-// window block j's 128-byte line (round k: block j + 64 k) and items
-// lane + 64 k (when the region's items fit the LDS cache).  Loading them
-// is split from using them so that the persistent phase kernel can load the
-// next region while it rebuilds the current one.
+// A window's lines and cached items, in registers: lane j holds window block
+// j's 128-byte line (round k: block j + 64 k) and items lane + 64 k (when the
+// items fit the LDS cache), all loaded before the first is used.
 template <int kRounds>
 struct Lines {
   uint4 hv[kRounds], h1[kRounds], s0[kRounds], s1[kRounds], s2[kRounds], s3[kRounds];
   uint64_t iv[4];
 };
 
-// blocks in region r's window: W, or 2 R when other waves rebuild the
-// regions of the same parity at the same time (see rebuild_region), cut at
-// the end of the table
-__device__ inline int window_blocks(const QF& qf, uint64_t r, int W, bool concurrent) {
+// What one rebuild takes: the quotients of R blocks from B0 on, in a window of
+// nwin blocks
+struct Span {
+  uint64_t B0;
+  int R;
+  int nwin;
+};
+// Region r: a window of W blocks, or of 2 R where other waves rebuild the
+// regions of the same parity at the same time (see rebuild_region), cut at the
+// end of the table
+__device__ inline Span region_span(const QF& qf, uint64_t r, int W, bool concurrent) {
   const uint64_t R = qf.region_blocks;
   const uint64_t wmax = concurrent && 2 * R < (uint64_t)W ? 2 * R : (uint64_t)W;
-  return (int)min(wmax, qf.nblocks - r * R);
+  return {r * R, (int)R, (int)min(wmax, qf.nblocks - r * R)};
+}
+// Its first or second half, with what of the fast window stays inside the 2 R
+// blocks that are region r's while the other regions of its parity run: more
+// push blocks (40 behind the first half of 48 blocks, 40 behind the second).
+// nwin = 0 where the table ends before the half.
+__device__ inline Span half_span(const QF& qf, uint64_t r, int half) {
+  const int R = (int)qf.region_blocks, first = R / 2;
+  const uint64_t B0 = r * (uint64_t)R + (half ? (uint64_t)first : 0ULL);
+  if (B0 >= qf.nblocks) return {B0, 0, 0};
+  const int room = half ? 2 * R - first : 2 * R;
+  return {B0, half ? R - first : first, (int)min((uint64_t)(room < kWinFast ? room : kWinFast), qf.nblocks - B0)};
 }
 
 template <int W>
-__device__ __forceinline__ void load_lines(const QF& qf, uint64_t r, uint64_t s, uint64_t e, bool concurrent,
+__device__ __forceinline__ void load_lines(const QF& qf, const Span& sp, uint64_t s, uint64_t e,
                                            const uint64_t* __restrict__ items, Lines<W / 64>& L) {
   constexpr int kRounds = W / 64;
   const int lane = lane_id();
-  const int nwin = window_blocks(qf, r, W, concurrent);
-  const GQF_GLOBAL uint4* g = gqf_block_ptr(qf, r * qf.region_blocks);
+  const int nwin = sp.nwin;
+  const GQF_GLOBAL uint4* g = gqf_block_ptr(qf, sp.B0);
 #pragma unroll
   for (int k = 0; k < kRounds; k++) {
     const int j = lane + 64 * k;
@@ -1234,22 +1250,17 @@ __device__ __forceinline__ void load_lines(const QF& qf, uint64_t r, uint64_t s,
 // would push into region r + 2 while that region's wave rebuilds it.  A push
 // the cut window cannot absorb is redone by the serial wide pass.
 //
-// `L`: the region's lines, already loaded by load_lines when `loaded`,
-// else loaded here.  With `has_next`, the lines of the region (rn, sn, en)
-// are loaded into L as soon as this region's lines are in LDS, so they
-// arrive while this one is rebuilt.
 template <int W, bool kStash = true>
-__device__ __forceinline__ int rebuild_region_lines(const QF& qf, uint64_t r, const uint64_t* __restrict__ items,
-                              const uint64_t* __restrict__ counts, uint64_t s, uint64_t e, int mode,
-                              Smem<W>& sm, uint32_t* lcnt, bool concurrent, uint64_t tag, Lines<W / 64>& L,
-                              bool loaded, bool has_next, uint64_t rn, uint64_t sn, uint64_t en) {
+__device__ __forceinline__ int rebuild_span(const QF& qf, const Span& sp, const uint64_t* __restrict__ items,
+                                            const uint64_t* __restrict__ counts, uint64_t s, uint64_t e, int mode,
+                                            Smem<W>& sm, uint32_t* lcnt, uint64_t tag) {
   constexpr int kRounds = W / 64;
   const bool shift_ok = !(mode & GQF_REBUILD_NO_SHIFT);
   mode &= ~GQF_REBUILD_NO_SHIFT;
   const int lane = lane_id();
-  const int R = (int)qf.region_blocks;
-  const uint64_t B0 = r * (uint64_t)R;
-  const int nwin = window_blocks(qf, r, W, concurrent);
+  const int R = sp.R;
+  const uint64_t B0 = sp.B0;
+  const int nwin = sp.nwin;
   const int nreg = (int)min((uint64_t)R, qf.nblocks - B0);
   const int64_t win_base = (int64_t)(B0 * 64);
   const bool table_end_in_window = B0 + (uint64_t)nwin >= qf.nblocks;
@@ -1264,7 +1275,8 @@ __device__ __forceinline__ int rebuild_region_lines(const QF& qf, uint64_t r, co
   uint32_t off_w[kRounds];
   uint64_t used_w[kRounds];
   {
-    if (!loaded) load_lines<W>(qf, r, s, e, concurrent, items, L);
+    Lines<W / 64> L;
+    load_lines<W>(qf, sp, s, e, items, L);
     uint32_t ov[kRounds];
 #pragma unroll
     for (int k = 0; k < kRounds; k++) ov[k] = L.h1[k].x;
@@ -1304,8 +1316,6 @@ __device__ __forceinline__ int rebuild_region_lines(const QF& qf, uint64_t r, co
       }
     }
   }
-  // the next region's lines start loading now (this region's are in LDS)
-  if (has_next) load_lines<W>(qf, rn, sn, en, concurrent, items, L);
   __syncthreads();
 
   // ---- 2. per-block item ranges / quotient table ----
@@ -1591,9 +1601,10 @@ __device__ __forceinline__ int rebuild_delete(const QF& qf, uint64_t r, const ui
                                               uint64_t e, DeleteSmem& sm) {
   const int lane = lane_id();
   const int j = lane;
-  const int R = (int)qf.region_blocks;
-  const uint64_t B0 = r * (uint64_t)R;
-  const int nwin = window_blocks(qf, r, kWinFast, true);
+  const Span sp = region_span(qf, r, kWinFast, true);
+  const int R = sp.R;
+  const uint64_t B0 = sp.B0;
+  const int nwin = sp.nwin;
   const bool table_end = B0 + (uint64_t)nwin >= qf.nblocks;
   const uint64_t base = B0 << 14;
 
@@ -1866,13 +1877,11 @@ __device__ __forceinline__ int rebuild_delete(const QF& qf, uint64_t r, const ui
   return kOk;
 }
 
-// rebuild_region_lines with the lines loaded here
 template <int W, bool kStash = true>
 __device__ __forceinline__ int rebuild_region(const QF& qf, uint64_t r, const uint64_t* __restrict__ items,
                                               const uint64_t* __restrict__ counts, uint64_t s, uint64_t e, int mode,
                                               Smem<W>& sm, uint32_t* lcnt, bool concurrent, uint64_t tag = 0) {
-  Lines<W / 64> L;
-  return rebuild_region_lines<W, kStash>(qf, r, items, counts, s, e, mode, sm, lcnt, concurrent, tag, L, false, false, 0, 0, 0);
+  return rebuild_span<W, kStash>(qf, region_span(qf, r, W, concurrent), items, counts, s, e, mode, sm, lcnt, tag);
 }
 
 }  // namespace
@@ -1978,34 +1987,82 @@ gqf_rebuild_delete(const QF* __restrict__ qfp, const uint64_t* __restrict__ item
   if (res == kNeedWide && lane_id() == 0) flag_wide(r, wide_flags, wide_count);
 }
 
-// Redoes flagged regions of one parity with a wider window: 128 blocks,
-// then 256 for a push that outruns that too (a region that needs a wider
-// window has not written anything).  Regions whose windows could meet are
-// redone in ascending order; regions kWinWide blocks or more apart cannot
-// touch each other's blocks, so the flagged regions are cut into chains of
-// closer ones, and each chain runs on its own workgroup (up to
-// GQF_WIDE_LIST of them).  Up to GQF_WIDE_LIST flagged regions come from
-// the phase's list, ordered by rank; more go to gqf_rebuild_wide_class.
-// Every workgroup exits at once when nothing was flagged; otherwise the
-// last one to finish clears the count for the next phase.
+constexpr uint32_t kWideMaxPolls = 1u << 24;
+
+__device__ inline bool wait_count(const uint32_t* ctr, uint32_t target, uint32_t max_polls) {
+  for (uint32_t k = 0; k < max_polls; k++) {
+    const uint32_t v = __hip_atomic_load(ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if ((uint32_t)__builtin_amdgcn_readfirstlane(v) == target) return true;
+    __builtin_amdgcn_s_sleep(4);
+  }
+  return false;
+}
+
+// Redoes the regions of one parity that a phase flagged, none of which has
+// written anything.  Every workgroup exits at once when nothing was flagged.
+//
+// Up to GQF_WIDE_LIST of them (the phase's list, ordered by rank): with a
+// window of 128 blocks, then 256 for a push that outruns that too.  Regions
+// whose windows could meet are redone in ascending order; regions kWinWide
+// blocks or more apart cannot touch each other's blocks, so the flagged
+// regions are cut into chains of closer ones, and each chain runs on its own
+// workgroup.  The last of them to finish clears the count.
+//
+// More (loads near 95%), in stages of kWideClassGrid workgroups:
+//   * stage 0 redoes every flagged region as two halves, the second first,
+//     each with more push blocks than the region had (half_span): what both
+//     touch are the 2 R blocks that belong to the region while its parity runs,
+//     so all run at once.  A region whose second half needs more stays flagged,
+//     one whose first half does too, with flag kFirstHalf;
+//   * stage 1 + c redoes what is left of class c: regions of one parity whose
+//     indices differ by at least `apart` (the widest window, 256 blocks, in
+//     regions) have disjoint windows, so region parity + 2 i is in class i mod
+//     ncls (ncls = ceil(apart / 2)).
+// The stages run one after another in ONE launch: each workgroup takes a
+// ticket when it starts; tickets c * kWideClassGrid .. (c + 1) *
+// kWideClassGrid - 1 run stage c, after waiting for stage c - 1's finished
+// counter.  Every workgroup of stage c - 1 took its ticket before any of
+// stage c did, so it is running or done, and it waits only on earlier stages:
+// every wait ends.  (A wait past max_polls, 2^24 unless qf_set_wide_wait_bound
+// says otherwise, which no correct run reaches, flags the class's regions as
+// CLUSTER_OVERFLOW instead of rebuilding them.)  A workgroup takes every
+// kWideClassGrid-th region of its stage, so the flagged ones spread evenly.
+// The last workgroup to finish clears every counter for the next phase.
+//
+// 3.4 M inserts from 90% to 95% load at 2^26 slots (thousands of regions
+// flagged in the odd phase): 1,376 -> 532 us for the pass without stage 0 and
+// with a workgroup taking 64 regions side by side; with nothing flagged a
+// launch is 4.6 us, one instead of two a phase.
+constexpr uint8_t kFirstHalf = 2;
+
 extern "C" __global__ void __launch_bounds__(64)
 gqf_rebuild_wide(const QF* __restrict__ qfp, const uint64_t* __restrict__ items,
                  const uint64_t* __restrict__ counts, const uint32_t* __restrict__ region_start,
-                 int parity, int mode, uint8_t* __restrict__ wide_flags,
-                 uint32_t* __restrict__ wide_count) {
-  __shared__ Smem<kWinMid> smm;
-  __shared__ Smem<kWinWide> sm;
+                 int parity, int mode, uint8_t* __restrict__ wide_flags, uint32_t* __restrict__ wide_count,
+                 uint32_t ncls, uint32_t max_polls) {
+  __shared__ union {
+    Smem<kWinFast> fast;
+    Smem<kWinMid> mid;
+    Smem<kWinWide> wide;
+  } sm;
   __shared__ uint32_t icnt[kItemCap];
+  __shared__ uint32_t ticket;
   const uint32_t nflag = *(volatile uint32_t*)wide_count;
-  if (nflag == 0) return;
+  if (nflag == 0 || (nflag <= GQF_WIDE_LIST && blockIdx.x >= GQF_WIDE_LIST)) return;
   const QF qf = *qfp;
   const int lane = lane_id();
-  auto redo = [&](uint64_t rr) {
-    const uint64_t s = region_start[rr], e = region_start[rr + 1];
-    int res = rebuild_region<kWinMid>(qf, rr, items, counts, s, e, mode, smm, icnt, false);
-    __syncthreads();
-    if (res == kNeedWide) res = rebuild_region<kWinWide>(qf, rr, items, counts, s, e, mode, sm, icnt, false);
-    __syncthreads();
+  const uint64_t hmask = (mode & ~GQF_REBUILD_NO_SHIFT) == kSeq ? GQF_SEQ_HASH_MASK : ~0ULL;
+  // first item of region rr's second half
+  auto middle = [&](uint64_t rr) -> uint64_t {
+    const uint64_t bound = half_span(qf, rr, 1).B0 << 14;
+    uint64_t lo = region_start[rr], hi = region_start[rr + 1];
+    while (lo < hi) {
+      const uint64_t mid = (lo + hi) >> 1;
+      if ((items[mid] & hmask) < bound) lo = mid + 1; else hi = mid;
+    }
+    return lo;
+  };
+  auto report = [&](uint64_t rr, int res) {
     if (lane == 0) {
       wide_flags[rr] = 0;
       if (res == kNeedWide) atomicOr(qf.status, GQF_STATUS_CLUSTER_OVERFLOW);
@@ -2013,6 +2070,33 @@ gqf_rebuild_wide(const QF* __restrict__ qfp, const uint64_t* __restrict__ items,
     }
     __syncthreads();
   };
+  auto redo = [&](uint64_t rr) __attribute__((always_inline)) {
+    const uint64_t s = region_start[rr];
+    const uint64_t e = wide_flags[rr] == kFirstHalf ? middle(rr) : (uint64_t)region_start[rr + 1];
+    int res = rebuild_region<kWinMid>(qf, rr, items, counts, s, e, mode, sm.mid, icnt, false);
+    __syncthreads();
+    if (res == kNeedWide) res = rebuild_region<kWinWide>(qf, rr, items, counts, s, e, mode, sm.wide, icnt, false);
+    __syncthreads();
+    report(rr, res);
+  };
+  auto redo_halves = [&](uint64_t rr) __attribute__((always_inline)) {
+    // (a region that may find the table full is redone as a whole: it must
+    // stay unchanged then)
+    if ((rr + 2) * qf.region_blocks >= qf.nblocks) return;
+    const uint64_t s = region_start[rr], e = region_start[rr + 1], m = middle(rr);
+    int res = kOk;
+#pragma unroll 1
+    for (int half = 1; half >= 0 && res == kOk; half--) {
+      const uint64_t a = half ? m : s, z = half ? e : m;
+      if (a < z)
+        res = rebuild_span<kWinFast, false>(qf, half_span(qf, rr, half), items, counts, a, z, mode, sm.fast, icnt, 0);
+      __syncthreads();
+      if (res == kOk && half && lane == 0) wide_flags[rr] = kFirstHalf;
+      __syncthreads();
+    }
+    if (res == kOk) report(rr, res);  // else its flag says what is left
+  };
+  uint32_t* finished = &wide_count[1 + GQF_WIDE_LIST];
   if (nflag <= GQF_WIDE_LIST) {
     // distinct regions: each one's rank among them is its place in the order
     const uint32_t mine = (uint32_t)lane < nflag ? wide_count[1 + lane] : 0xFFFFFFFFu;
@@ -2039,100 +2123,46 @@ gqf_rebuild_wide(const QF* __restrict__ qfp, const uint64_t* __restrict__ items,
         }
       }
     }
-  } else {
-    return;  // more than GQF_WIDE_LIST flagged: the class launch takes them (gqf_rebuild_wide_class)
-  }
-  // the last workgroup to finish clears the count and the finish counter
-  if (lane == 0) {
-    __threadfence();
-    if (atomicAdd(&wide_count[1 + GQF_WIDE_LIST], 1u) == gridDim.x - 1) {
-      wide_count[1 + GQF_WIDE_LIST] = 0;
-      *(volatile uint32_t*)wide_count = 0;
+    // the last workgroup to finish clears the count and the finish counter
+    if (lane == 0) {
+      __threadfence();
+      if (atomicAdd(finished, 1u) == GQF_WIDE_LIST - 1) {
+        *finished = 0;
+        *(volatile uint32_t*)wide_count = 0;
+      }
     }
+    return;
   }
-}
-
-// The flagged regions of a phase when there are more than GQF_WIDE_LIST
-// (loads near 95%): regions of one parity whose indices differ by at least
-// `apart` (the widest window, 256 blocks, in regions) have disjoint
-// windows, so region parity + 2 i is in class i mod ncls (ncls =
-// ceil(apart / 2)) and the classes run one after another, in ONE launch of
-// ncls x kWideClassGrid workgroups.  Each workgroup takes a ticket when it
-// starts; tickets c * kWideClassGrid .. (c + 1) * kWideClassGrid - 1 run
-// class c, after waiting for class c - 1's finished counter.  Every
-// workgroup of class c - 1 took its ticket before any of class c did, so it
-// is running or done, and it waits only on earlier classes: every wait
-// ends.  (A wait past max_polls, 2^24 unless qf_set_wide_wait_bound says
-// otherwise, which no correct run reaches, flags the class's regions as
-// CLUSTER_OVERFLOW instead of rebuilding them.)  The last workgroup to
-// finish clears every counter for the next phase.  Nothing runs when
-// GQF_WIDE_LIST or fewer were flagged (gqf_rebuild_wide has taken them).
-constexpr uint32_t kWideMaxPolls = 1u << 24;
-
-__device__ inline bool wait_count(const uint32_t* ctr, uint32_t target, uint32_t max_polls) {
-  for (uint32_t k = 0; k < max_polls; k++) {
-    const uint32_t v = __hip_atomic_load(ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if ((uint32_t)__builtin_amdgcn_readfirstlane(v) == target) return true;
-    __builtin_amdgcn_s_sleep(4);
-  }
-  return false;
-}
-
-extern "C" __global__ void __launch_bounds__(64)
-gqf_rebuild_wide_class(const QF* __restrict__ qfp, const uint64_t* __restrict__ items,
-                       const uint64_t* __restrict__ counts, const uint32_t* __restrict__ region_start,
-                       int parity, int mode, uint8_t* __restrict__ wide_flags, uint32_t* __restrict__ wide_count,
-                       uint32_t ncls, uint32_t max_polls) {
-  __shared__ Smem<kWinMid> smm;
-  __shared__ Smem<kWinWide> sm;
-  __shared__ uint32_t icnt[kItemCap];
-  __shared__ uint32_t ticket;
-  const uint32_t nflag = *(volatile uint32_t*)wide_count;
-  if (nflag <= GQF_WIDE_LIST) return;
-  const QF qf = *qfp;
-  const int lane = lane_id();
-  uint32_t* finished = &wide_count[1 + GQF_WIDE_LIST];
   uint32_t* tickets = &wide_count[2 + GQF_WIDE_LIST];
-  uint32_t* class_done = &wide_count[3 + GQF_WIDE_LIST];
+  uint32_t* stage_done = &wide_count[3 + GQF_WIDE_LIST];
   if (lane == 0) ticket = atomicAdd(tickets, 1u);
   __syncthreads();
   const uint32_t t = ticket;
-  const uint32_t cls = t / kWideClassGrid, w = t % kWideClassGrid;
-  const bool ok = cls == 0 || wait_count(&class_done[cls - 1], kWideClassGrid, max_polls);
+  const uint32_t stage = t / kWideClassGrid, w = t % kWideClassGrid;
+  const bool ok = stage == 0 || wait_count(&stage_done[stage - 1], kWideClassGrid, max_polls);
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   const uint64_t nper = qf.nregions > (uint64_t)parity ? (qf.nregions - (uint64_t)parity + 1) / 2 : 0;
-  // candidate j of this class is i = cls + ncls j, region parity + 2 i;
-  // workgroups take 64 candidates at a time
-  const uint64_t ncand = nper > cls ? (nper - cls + ncls - 1) / ncls : 0;
-  for (uint64_t j0 = (uint64_t)w * 64; j0 < ncand; j0 += (uint64_t)kWideClassGrid * 64) {
-    const uint64_t j = j0 + (uint64_t)lane;
-    const uint64_t r = (uint64_t)parity + 2 * ((uint64_t)cls + (uint64_t)ncls * j);
-    uint64_t m = __ballot(j < ncand && wide_flags[r]);
+  // candidate j of stage 0 is region parity + 2 j, of class c region parity +
+  // 2 (c + ncls j); workgroup w takes j = w, w + kWideClassGrid, ..., 64 at a time
+  const uint64_t first = stage ? stage - 1 : 0, step = stage ? ncls : 1;
+  const uint64_t ncand = nper > first ? (nper - first + step - 1) / step : 0;
+  for (uint64_t j0 = w; j0 < ncand; j0 += (uint64_t)kWideClassGrid * 64) {
+    const uint64_t j = j0 + (uint64_t)kWideClassGrid * (uint64_t)lane;
+    uint64_t m = __ballot(j < ncand && wide_flags[(uint64_t)parity + 2 * (first + step * j)]);
     while (m) {
       const int l = __builtin_ctzll(m);
       m &= m - 1;
-      const uint64_t rr = (uint64_t)parity + 2 * ((uint64_t)cls + (uint64_t)ncls * (j0 + (uint64_t)l));
-      int res = kNeedWide;
-      if (ok) {
-        const uint64_t s = region_start[rr], e = region_start[rr + 1];
-        res = rebuild_region<kWinMid>(qf, rr, items, counts, s, e, mode, smm, icnt, false);
-        __syncthreads();
-        if (res == kNeedWide) res = rebuild_region<kWinWide>(qf, rr, items, counts, s, e, mode, sm, icnt, false);
-        __syncthreads();
-      }
-      if (lane == 0) {
-        wide_flags[rr] = 0;
-        if (res == kNeedWide) atomicOr(qf.status, GQF_STATUS_CLUSTER_OVERFLOW);
-        else if (res == kNoSpace) atomicOr(qf.status, GQF_STATUS_NO_SPACE);
-      }
-      __syncthreads();
+      const uint64_t rr = (uint64_t)parity + 2 * (first + step * (j0 + (uint64_t)kWideClassGrid * (uint64_t)l));
+      if (stage == 0) redo_halves(rr);
+      else if (ok) redo(rr);
+      else report(rr, kNeedWide);
     }
   }
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
   if (lane == 0) {
-    atomicAdd(&class_done[cls], 1u);
+    atomicAdd(&stage_done[stage], 1u);
     if (atomicAdd(finished, 1u) == gridDim.x - 1) {  // everyone is done: clear for the next phase
-      for (uint32_t c = 0; c < ncls; c++) class_done[c] = 0;
+      for (uint32_t c = 0; c <= ncls; c++) stage_done[c] = 0;
       *tickets = 0;
       *finished = 0;
       *(volatile uint32_t*)wide_count = 0;
@@ -2479,9 +2509,7 @@ void gqf_launch_rebuild(const QF* qf_dev, uint64_t nregions, uint64_t region_blo
                          list, list_count, parity, mode, wide_flags, wide_count);
     gqf_prof_end("rebuild_phase", s);
     gqf_prof_begin("rebuild_wide", s);
-    hipLaunchKernelGGL(gqf_rebuild_wide, dim3(GQF_WIDE_LIST), dim3(64), 0, s, qf_dev, items, counts, region_start,
-                       parity, mode, wide_flags, wide_count);
-    hipLaunchKernelGGL(gqf_rebuild_wide_class, dim3(ncls * kWideClassGrid), dim3(64), 0, s, qf_dev, items, counts,
+    hipLaunchKernelGGL(gqf_rebuild_wide, dim3((1 + ncls) * kWideClassGrid), dim3(64), 0, s, qf_dev, items, counts,
                        region_start, parity, mode, wide_flags, wide_count, ncls,
                        g_wide_max_polls.load(std::memory_order_relaxed));
     gqf_prof_end("rebuild_wide", s);
