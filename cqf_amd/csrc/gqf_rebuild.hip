@@ -655,14 +655,20 @@ __device__ __forceinline__ bool walk_block_table(Smem<W>& sm, int j, int nwin, u
 //   * drops by one, down to 0, at every empty slot (an empty slot absorbs
 //     one unit: the run after it is at home, max(q, ...) takes q);
 //   * is unchanged across used slots.
-// Each of these is a map x -> max(a, x + b), and maps compose, so lane j
-// folds slot-block j's events and empty slots (from the block's stored
-// used-slot mask) into one map and a wave scan gives the shift entering
-// every block.  The untouched bytes then move as whole stretches between
+// With Z(p) the empty slots before position p and D the growth of the events
+// so far, the shift just before event t is D - Z(t) + the greatest Z(s) - D(s)
+// of the events s up to t (D(s): the growth before s), so two scans over the
+// events (lanes in quotient order, which is position order) give every
+// event's shift, and the shift entering a block follows from the last event
+// before it.  The untouched bytes then move as whole stretches between
 // events and empty slots, instead of run by run; only the listed quotients'
 // runs are re-encoded (merge_quotient).  Offsets come from the new run-end
 // bits by rank: the runs of quotients < 64 j end at the k-th run end of the
 // window, k = runs ending before it + occupied quotients of blocks < j.
+// Bound by VALU issue (three waves a SIMD: the LDS rows).  Two loops over each
+// block's events, as long as the fullest block's, took the place of the scans
+// before: 3,399 instructions a region and 331 us a launch over half of 2^22
+// blocks at 190 items a region, now 2,835 and 293 us.
 
 // position of a listed quotient q's event: its old run [st, st + ol) if q
 // is occupied, else st = the slot its new run would start at (ol = 0);
@@ -840,83 +846,127 @@ __device__ __forceinline__ int rebuild_insert_shift(const QF& qf, uint64_t B0, i
   // straight-line merge where it applies.
   static_assert(kItemCap <= 4 * 64, "four rounds of listed quotients");
   uint32_t lean_lo[4], lean_hi[4], lean_meta[4] = {0, 0, 0, 0};
-  auto measure = [&](uint32_t t, int k) {
-    const uint32_t it0 = sm.tit0[t];
-    const uint32_t h0 = src.hash(sm.items, it0);
-    const int32_t q = (int32_t)(h0 >> 8);
-    int32_t st = q;
-    uint32_t ol = 0, nl = 0;
-    if (locate_run_or_slot(sm, nwin, q, st, ol)) {
-      const uint32_t it1 = t + 1 < nq ? sm.tit0[t + 1] : m;
-      uint32_t ln;
-      if (kStash && it1 - it0 <= 2 && ol <= 8 && lean_read(sm, src, it0, it1, st, ol, h0, lean_lo[k], lean_hi[k], ln))
-        nl = ln, lean_meta[k] = 1;
-      else
-        nl = merge_quotient<W, false>(sm, src, it0, it1, st, ol, 0, h0), lean_meta[k] = 0;
-      atomicAdd((uint32_t*)&sm.xnew[st >> 6], 1u);  // events per slot-block (st < 64 nwin)
-    } else {
-      atomicMin(&sm.first_invalid, -1);
-      st = 0;
-    }
-    if (ol > kRunLenMax<W> || nl > kRunLenMax<W>) {  // redone in a wider window
-      atomicMin(&sm.first_invalid, -1);
-      ol = nl = 0;
-    }
-    sm.tst[t] = (int16_t)st;
-    sm.tol[t] = (RunLen<W>)ol;
-    sm.tnl[t] = (RunLen<W>)nl;
+  // Until the rows are cleared, their space holds what the events leave for
+  // the blocks: each event's D and greatest Z - D (its own growth included in
+  // D); each block's valid empty slots and those before it; the slots of the
+  // old runs replaced in it; the shift its events add, as 2-bit fields of
+  // four words of 16 positions.
+  struct Events {
+    uint32_t dm[4 * 64];
+    uint32_t ev[64][4];
+    unsigned long long zero[64], skip[64];
+    int32_t zpre[64];
   };
-  sm.xnew[j] = 0;
-  __syncthreads();
-  if constexpr (kStash) {
-#pragma unroll
-    for (int k = 0; k < 4; k++)
-      if ((uint32_t)lane + 64u * (uint32_t)k < nq) measure((uint32_t)lane + 64u * (uint32_t)k, k);
-  } else {
-    for (uint32_t t = lane; t < nq; t += 64) measure(t, 0);
-  }
-  __syncthreads();
-  if (sm.first_invalid < 0) return kNeedWide;
-
-  // ---- the events of slot-block j: listed quotients e0 .. e1 - 1 (their
-  // positions ascend with the quotients, so a scan of the per-block counts
-  // gives each block's range)
-  uint32_t e0, e1;
-  {
-    const uint32_t c = (uint32_t)sm.xnew[j];
-    const uint32_t incl = wave_scan_add(c);
-    e0 = incl - c;
-    e1 = incl;
-  }
-
-  // ---- lane j's shift map: events and (valid) empty slots of slot-block j
+  static_assert(W == 64 && sizeof(Events) <= sizeof(sm.sout), "one lane a block, in the rows' space");
+  Events& es = *(Events*)sm.sout;
+  constexpr int kShiftFast = 24;
+  constexpr int32_t kGeneralBlock = 1 << 16;  // beside a block's count of events (at most kItemCap)
   uint32_t vlim = 0;
   if (j < nwin) {
     const uint64_t first = (B0 + (uint64_t)j) * 64;
     vlim = !table_end_in_window ? 64u : (first >= qf.xnslots ? 0u : (uint32_t)min((uint64_t)64, qf.xnslots - first));
   }
   const uint64_t zero_ok = ~used & gqf_mask(vlim);  // empty slots that absorb shift
-  int32_t A = kNegInf, Bm = 0;
-  {
-    int pos = 0;
-    for (uint32_t t = e0; t < e1; t++) {
-      const int rel = sm.tst[t] - 64 * j;
-      const int c = __popcll(zero_ok & range_mask(pos, rel));
-      if (c) compose(A, Bm, 0, -c);
-      compose(A, Bm, kNegInf, (int32_t)sm.tnl[t] - (int32_t)sm.tol[t]);
-      pos = rel;
+  const int32_t nzero = (int32_t)__popcll(zero_ok);
+  const int32_t zpre = (int32_t)wave_scan_add((uint32_t)nzero) - nzero;
+  es.zero[j] = zero_ok;
+  es.zpre[j] = zpre;
+  es.skip[j] = 0;
+  es.ev[j][0] = es.ev[j][1] = es.ev[j][2] = es.ev[j][3] = 0;
+  sm.xnew[j] = 0;
+  __syncthreads();
+
+  int32_t grown = 0, lead = kNegInf;  // D and the greatest Z - D of the earlier rounds
+  // all lanes call it; lanes without a quotient (t >= nq) only take part in the scans
+  auto measure = [&](uint32_t t, int k) {
+    const bool has = t < nq;
+    int32_t st = 0;
+    uint32_t ol = 0, nl = 0;
+    if (has) {
+      const uint32_t it0 = sm.tit0[t];
+      const uint32_t h0 = src.hash(sm.items, it0);
+      const int32_t q = (int32_t)(h0 >> 8);
+      if (locate_run_or_slot(sm, nwin, q, st, ol)) {
+        const uint32_t it1 = t + 1 < nq ? sm.tit0[t + 1] : m;
+        uint32_t ln;
+        if (kStash && it1 - it0 <= 2 && ol <= 8 && lean_read(sm, src, it0, it1, st, ol, h0, lean_lo[k], lean_hi[k], ln))
+          nl = ln, lean_meta[k] = 1;
+        else
+          nl = merge_quotient<W, false>(sm, src, it0, it1, st, ol, 0, h0), lean_meta[k] = 0;
+      } else {
+        atomicMin(&sm.first_invalid, -1);
+        st = 0, ol = 0;
+      }
+      if (ol > kRunLenMax<W> || nl > kRunLenMax<W>) {  // redone in a wider window
+        atomicMin(&sm.first_invalid, -1);
+        ol = nl = 0;
+      }
     }
-    const int c = __popcll(zero_ok & range_mask(pos, 64));
-    if (c) compose(A, Bm, 0, -c);
+    const int b = st >> 6, rel = st & 63;  // st < 64 nwin
+    const int32_t z = es.zpre[b] + (int32_t)__popcll(es.zero[b] & gqf_mask((uint64_t)rel));
+    const int32_t d = (int32_t)nl - (int32_t)ol;  // not below 0: an insert never shortens a run
+    const int32_t D = grown + (int32_t)wave_scan_add((uint32_t)d);
+    const int32_t best = max(lead, gqf_flat::wave_scan_max(has ? z - (D - d) : kNegInf));
+    if (has) {
+      const int32_t delta = D - d - z + best;
+      sm.tst[t] = (int16_t)st;
+      sm.tol[t] = (RunLen<W>)ol;
+      sm.tnl[t] = (RunLen<W>)nl;
+      sm.tsn[t] = (int16_t)(st + delta);
+      es.dm[t] = (uint32_t)D << 16 | (uint32_t)(best & 0xFFFF);
+      atomicAdd((uint32_t*)&sm.xnew[b], 1u);
+      if (d > 3 || delta + d > kShiftFast) atomicOr((uint32_t*)&sm.xnew[b], (uint32_t)kGeneralBlock);
+      atomicAdd(&es.ev[b][rel >> 4], (uint32_t)(d & 3) << (2 * (rel & 15)));
+      // the old run's slots, which may go on in the next blocks
+      int32_t p = st;
+      for (int32_t left = (int32_t)ol; left > 0;) {
+        const int at = p & 63, n = left < 64 - at ? left : 64 - at;
+        atomicOr(&es.skip[p >> 6], range_mask(at, at + n));
+        p += n, left -= n;
+      }
+    }
+    grown = __builtin_amdgcn_readlane(D, 63);
+    lead = __builtin_amdgcn_readlane(best, 63);
+  };
+  if constexpr (kStash) {
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+      if (64u * (uint32_t)k < nq) measure((uint32_t)lane + 64u * (uint32_t)k, k);
+  } else {
+    for (uint32_t t = lane; t - lane < nq; t += 64) measure(t, 0);
   }
-  // inclusive scan of the maps over the lanes; the shift entering block j
-  // is the exclusive prefix applied to 0
-  int32_t ia = A, ib = Bm;
-  wave_scan_compose(ia, ib);
-  const int32_t ea = wave_shr1(ia, kNegInf), eb = wave_shr1(ib, 0);
-  const int32_t delta_in = ea > eb ? ea : eb;  // max(a, 0 + b)
-  const int32_t la = __builtin_amdgcn_readlane(ia, 63), lb = __builtin_amdgcn_readlane(ib, 63);
-  const int32_t delta_end = la > lb ? la : lb;
+  __syncthreads();
+  if (sm.first_invalid < 0) return kNeedWide;
+
+  // ---- the events of slot-block j: listed quotients e0 .. e1 - 1 (their
+  // positions ascend with the quotients, so a scan of the per-block counts
+  // gives each block's range), and what they left
+  uint32_t e0, e1;
+  int32_t delta_in = 0;  // the shift entering block j
+  bool general;
+  uint32_t ew[4];
+  uint64_t skip;
+  {
+    const uint32_t c = (uint32_t)sm.xnew[j];
+    general = (c & (uint32_t)kGeneralBlock) != 0;
+    const uint32_t n = c & (uint32_t)(kGeneralBlock - 1);
+    e1 = wave_scan_add(n);
+    e0 = e1 - n;
+    const uint32_t before = e0 ? es.dm[e0 - 1] : 0u, after = e1 ? es.dm[e1 - 1] : 0u;
+    const int32_t D0 = (int32_t)(before >> 16);
+    if (e0) delta_in = max(0, D0 + (int32_t)(int16_t)before - zpre);
+#pragma unroll
+    for (int k = 0; k < 4; k++) ew[k] = es.ev[j][k];
+    skip = es.skip[j];
+    // a position's growth above 3 carried into the next field, which lowers
+    // the sum of the fields
+    int32_t fields = 0;
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+      fields += __popc(ew[k]) + __popc(ew[k] & 0xAAAAAAAAu);
+    if (fields != (int32_t)(after >> 16) - D0 || delta_in > kShiftFast) general = true;
+  }
+  const int32_t delta_end = nq ? max(0, grown + lead - __builtin_amdgcn_readlane(zpre + nzero, 63)) : 0;
 
   // ---- b*: the first block at or after R, past the last event's old run,
   // that no shift reaches; blocks [0, b*) are rewritten, the rest stay
@@ -951,58 +1001,16 @@ __device__ __forceinline__ int rebuild_insert_shift(const QF& qf, uint64_t B0, i
   if (j < bstar) sm.run_out[j] = 0;
   __syncthreads();
 
-  // ---- lane j moves the untouched bytes of slot-block j and records the
-  // new start of each of its events' runs; used_new is the block's new
-  // used-slot mask (the new runs' slots and what block j - 1 pushes in
-  // included), which only lane j writes and reads
+  // ---- lane j moves the untouched bytes of slot-block j; used_new is the
+  // block's new used-slot mask (the new runs' slots and what block j - 1
+  // pushes in included), which only lane j writes and reads
   uint64_t used_new = 0;
   if (j < bstar) {
     const uint64_t run_j = sm.run_in[j];
     const int32_t base = 64 * j;
-    int32_t cur = base;
-    if (e0 > 0) {  // an earlier event's old run may reach into this block
-      const int32_t pe = sm.tst[e0 - 1] + (int32_t)sm.tol[e0 - 1];
-      if (pe > cur) cur = pe;
-    }
-    // The events, in order: each one's new start; the slots of the old runs
-    // they replace (`skip`, with what an earlier block's last event covers);
-    // and the shift each event position adds, in 2-bit fields (ev[0]:
-    // positions 0..31, ev[1]: 32..63).  A position whose fields would pass
-    // 3, or a shift above kShiftFast, sends the block to the general loop
-    // below (at 2^24 inserts into 2^28 slots, one block in 60,000 passes
-    // 24).
-    constexpr int kShiftFast = 24;
-    uint64_t skip = cur > base ? gqf_mask((uint64_t)min(64, cur - base)) : 0ULL;
-    uint64_t ev[2] = {0ULL, 0ULL};
-    bool general = false;
-    {
-      int32_t delta = delta_in, emax = delta_in;
-      int pos = 0;
-      for (uint32_t t = e0; t < e1; t++) {
-        const int32_t st = sm.tst[t];
-        const int rel = st - base;
-        const int c = __popcll(zero_ok & range_mask(pos, rel));
-        delta = delta > c ? delta - c : 0;
-        sm.tsn[t] = (int16_t)(st + delta);
-        const int32_t d = (int32_t)sm.tnl[t] - (int32_t)sm.tol[t];
-        delta += d;
-        if (delta > emax) emax = delta;
-        pos = rel;
-        if (d < 0) general = true;  // inserts never shorten a run; kept general all the same
-        if (d > 0) {
-          const int sh = 2 * (rel & 31);
-          const uint64_t h = rel < 32 ? ev[0] : ev[1];
-          if ((int)((h >> sh) & 3ULL) + d > 3) general = true;
-          const uint64_t add = (uint64_t)(d & 3) << sh;
-          if (rel < 32) ev[0] += add; else ev[1] += add;
-        }
-        const int tol = (int)sm.tol[t];
-        if (tol) skip |= range_mask(rel, min(64, rel + tol));
-        const int32_t pe = st + tol;
-        if (pe > cur) cur = pe;
-      }
-      if (emax > kShiftFast) general = true;
-    }
+    // Blocks in which a position's events add more than 3 or a shift passes
+    // kShiftFast take the general loop below (at 2^24 inserts into 2^28
+    // slots, one block in 60,000 passes 24).
     if (!general) {
       // One straight pass over the block's 64 slots, the same code on every
       // lane.  e, the shift at slot i, grows by the slot's event fields; an
@@ -1026,7 +1034,6 @@ __device__ __forceinline__ int rebuild_insert_shift(const QF& qf, uint64_t B0, i
       const uint32_t cw[2] = {(uint32_t)copy, (uint32_t)(copy >> 32)};
       const uint32_t rc[2] = {(uint32_t)runc, (uint32_t)(runc >> 32)};
       const uint32_t zw[2] = {(uint32_t)zero_ok, (uint32_t)(zero_ok >> 32)};
-      const uint32_t ew[4] = {(uint32_t)ev[0], (uint32_t)(ev[0] >> 32), (uint32_t)ev[1], (uint32_t)(ev[1] >> 32)};
       uint8_t* dst = out + sin_off(base);  // row j; row j + 1 starts 68 bytes on
       auto slot = [&](auto ic) {
         constexpr int i = decltype(ic)::value;
