@@ -10,9 +10,9 @@
 //   1. every counter of the old window becomes an entry: each thread holds
 //      eight slots; a slot's quotient is the k-th occupied one of the window, k =
 //      run ends before the slot (a popcount, and a table of the occupied
-//      quotients by rank).  In a run of strictly ascending bytes every slot
-//      is a count-1 counter; the lane at the start of any other run marks
-//      the run's counter starts first;
+//      quotients by rank).  In a run whose bytes ascend, but for pairs of
+//      equal ones, every byte is a counter of 1 and every pair one of 2; the
+//      lane at the start of any other run marks its counter starts first;
 //   2. every distinct item hash finds its place among the old entries of its
 //      quotient's run; an entry that is there takes the new count, the others
 //      get a place among them (a bit map of the merged sequence);
@@ -27,14 +27,16 @@
 //
 // The result is the same canonical image as the single-wave rebuild's.
 //
-// Bound by instruction issue and the latency of its dozen steps (about 8,500
-// VALU instructions a region); 73 KB of LDS keep two workgroups, 16 waves, on
-// a CU.  The serial walk it replaces in dense batches, per launch: 943,718
-// keys into an empty table of 2^20 slots 268 -> 21 us; 14.1 M items into a
-// table of 2^25 slots, empty or half full, 854 -> 213 us on average.  With
-// 42 items a region (a served batch at 2^24 slots) the two are level (114 and
-// 97 us), and on a nearly empty table the walk is ahead (69 and 184 us at
-// 2^26 slots), hence the lines of gqf_launch_rebuild.
+// Bound by instruction issue, vector and LDS (9,900 VALU, 6,400 SALU and 950
+// LDS instructions for a region of a served batch); 54 KB of LDS keep three
+// workgroups, 24 waves, on a CU.  The serial walk it replaces in dense
+// batches, per launch: 943,718 keys into an empty table of 2^20 slots 268 ->
+// 20 us; 14.1 M items into a table of 2^25 slots in four chunks 214 -> 55 us a
+// chunk on average; a served batch at 2^24 slots, 42 items a region, 114 ->
+// 83 us.  On a nearly empty table the walk is ahead (69 and 184 us at 2^26
+// slots), hence the lines of gqf_launch_rebuild.
+// Decoding every counter of two slots, in code repeated for each of a
+// thread's slots, took 94 us for the served batch and 62 us a chunk.
 // One lane per slot with a scan per 64 slots took 294 us where the eight
 // consecutive slots or entries a thread takes here, scanned once, take 213.
 #pragma once
@@ -281,18 +283,25 @@ __device__ __forceinline__ bool window_entries(const QF& qf, uint64_t B0, int nw
     for (uint32_t b = (uint32_t)(occ >> sh) & 0xFFu; b; b &= b - 1)
       sm.quot[k++] = (uint16_t)(64 * j + sh + __builtin_ctz(b));
   }
-  // a byte not above its predecessor in the run: the run holds a counter
-  // of more than one slot
+  // A byte not above its predecessor in the run goes on with a counter: a
+  // counter's first slot is above the remainder that ends the one before it.
+  // Counters of three slots and more hold digits that may ascend as well: such
+  // a counter drops right after its first slot (x > 0: to a lower digit or a
+  // leading 0) or has two 0s in a row (x = 0), and its run is decoded below.
   {
     const uint32_t c = (uint32_t)((sm.cont[j] & sm.start[j]) >> sh) & 0xFFu;
     uint32_t prev = tid ? sm.sin[8 * tid - 1] : 0u;
-    uint32_t viol = 0;
+    uint32_t same = 0, viol = 0;
 #pragma unroll
     for (int k = 0; k < 8; k++) {
       const uint32_t b = ((k < 4 ? x.x : x.y) >> (8 * (k & 3))) & 0xFFu;
-      viol |= b <= prev ? 1u << k : 0u;
+      same |= b == prev ? 1u << k : 0u;
+      viol |= b < max(prev, 1u) ? 1u << k : 0u;
       prev = b;
     }
+    // (three equal bytes in a row are no counter's: decoded as well)
+    viol |= same & (same << 1 | (tid && sm.sin[8 * tid - 1] == sm.sin[8 * tid - 2] ? 1u : 0u));
+    if ((same | viol) & c) ((uint8_t*)sm.start)[tid] = (uint8_t)((uint32_t)(sm.start[j] >> sh) & ~((same | viol) & c));
     for (viol &= c; viol; viol &= viol - 1) {
       // the run starts behind the last run end or unused slot before the byte
       const int at = sh + __builtin_ctz(viol);
@@ -316,6 +325,7 @@ __device__ __forceinline__ bool window_entries(const QF& qf, uint64_t B0, int nw
       for (uint32_t k = 0; k < len;) {
         uint64_t rem, c;
         const uint32_t last = gqf_decode_counter(slot, len, k, &rem, &c);
+        if (k) atomicOr((unsigned long long*)&sm.start[(p + (int32_t)k) >> 6], 1ULL << ((p + (int32_t)k) & 63));
         for (uint32_t y = k + 1; y <= last; y++) {
           const int32_t q = p + (int32_t)y;
           atomicAnd((unsigned long long*)&sm.start[q >> 6], ~(1ULL << (q & 63)));
@@ -341,36 +351,42 @@ __device__ __forceinline__ bool window_entries(const QF& qf, uint64_t B0, int nw
     // slots whose next slot continues their counter
     const uint64_t inner = own & ~st;
     const uint32_t nextb = (uint32_t)((inner >> sh) >> 1) & 0x7Fu;
-    const uint32_t after = sh < 56 ? (uint32_t)(inner >> (sh + 8)) & 1u
-                                   : (j + 1 < nwin ? (uint32_t)(sm.own[j + 1] & ~sm.start[j + 1]) & 1u : 0u);
-    const uint32_t moreb = stb & ~runb & (nextb | after << 7);
+    const uint32_t after = sh < 56 ? (uint32_t)(inner >> (sh + 8)) & 3u
+                                   : (j + 1 < nwin ? (uint32_t)(sm.own[j + 1] & ~sm.start[j + 1]) & 3u : 0u);
+    const uint32_t moreb = stb & ~runb & (nextb | (after & 1u) << 7);
     auto count_at = [&](int32_t p) -> uint64_t {  // of the counter of several slots at slot p
       const uint32_t len = (uint32_t)(run_end_of(sm, p, nwin) - p + 1);
       uint64_t rem, c;
       gqf_decode_counter([&](uint32_t k) -> uint64_t { return sm.sin[p + (int32_t)k]; }, len, 0, &rem, &c);
       return c;
     };
+    // a counter of two slots is a count of 2
+    const uint32_t longb = moreb & (nextb >> 1 | after << 6);
     if constexpr (!kStore) {
-      out.sum = (uint64_t)__builtin_popcount(stb & ~moreb);
-      for (uint32_t m = moreb; m; m &= m - 1) out.sum += count_at(8 * tid + __builtin_ctz(m));
+      out.sum = (uint64_t)__builtin_popcount(stb) + (uint64_t)__builtin_popcount(moreb & ~longb);
+      for (uint32_t m = longb; m; m &= m - 1) out.sum += count_at(8 * tid + __builtin_ctz(m)) - 1;
       return true;
     } else {
-    uint32_t q[8];
+      uint32_t q[8];
 #pragma unroll
-    for (int i = 0; i < 8; i++)
-      if ((stb >> i) & 1u) q[i] = sm.quot[k0 + (uint32_t)__builtin_popcount(runb & ((1u << i) - 1))];
+      for (int i = 0; i < 8; i++)
+        if ((stb >> i) & 1u) q[i] = sm.quot[k0 + (uint32_t)__builtin_popcount(runb & ((1u << i) - 1))];
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-      const uint32_t ei = e0 + (uint32_t)__builtin_popcount(stb & ((1u << i) - 1));
-      if ((stb >> i) & 1u) {
-        const uint32_t h = q[i] << 8 | (((i < 4 ? x.x : x.y) >> (8 * (i & 3))) & 0xFFu);
-        uint32_t aux = 1;
-        if ((moreb >> i) & 1u) aux = push_count(sm, h, count_at(8 * tid + i));
-        sm.old[ei] = h << 12 | aux;
+      for (int i = 0; i < 8; i++) {
+        const uint32_t ei = e0 + (uint32_t)__builtin_popcount(stb & ((1u << i) - 1));
+        if ((stb >> i) & 1u) {
+          const uint32_t h = q[i] << 8 | (((i < 4 ? x.x : x.y) >> (8 * (i & 3))) & 0xFFu);
+          sm.old[ei] = h << 12 | (1u + ((moreb >> i) & 1u));
+        }
+        if ((runb >> i) & 1u)
+          sm.rend[k0 + (uint32_t)__builtin_popcount(runb & ((1u << i) - 1))] = (uint16_t)(ei + ((stb >> i) & 1u));
       }
-      if ((runb >> i) & 1u)
-        sm.rend[k0 + (uint32_t)__builtin_popcount(runb & ((1u << i) - 1))] = (uint16_t)(ei + ((stb >> i) & 1u));
-    }
+      for (uint32_t m = longb; m; m &= m - 1) {
+        const int i = __builtin_ctz(m);
+        uint32_t& y = sm.old[e0 + (uint32_t)__builtin_popcount(stb & ((1u << i) - 1))];
+        const uint32_t h = y >> 12;
+        y = h << 12 | push_count(sm, h, count_at(8 * tid + i));
+      }
     }
   }
   __syncthreads();
@@ -568,7 +584,9 @@ __device__ __forceinline__ int rebuild(const QF& qf, uint64_t r, const uint64_t*
     };
     auto slots_of = [&](uint32_t y) -> uint32_t {
       const uint32_t rem = (y >> 12) & 0xFFu, aux = y & 0xFFFu;
-      return aux < kAuxBig ? entry_len(rem, aux) : gqf_counter_len(rem, full_count(sm, y >> 12, aux, n_big));
+      uint32_t len = aux;  // counts up to 3
+      if (aux > 3) len = aux < kAuxBig ? entry_len(rem, aux) : gqf_counter_len(rem, full_count(sm, y >> 12, aux, n_big));
+      return len;
     };
     uint32_t sum = 0;
     int32_t lead = kNone, lastq = -1;  // max of quotient - slots before it in the share; the last quotient
