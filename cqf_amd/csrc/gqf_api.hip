@@ -75,6 +75,10 @@ struct EnumSpace {
   uint64_t move_cap = 0;
   uint64_t* move_items = nullptr;
   uint64_t* move_counts = nullptr;
+  uint64_t census_blocks = 0;           // blocks the census arrays below have room for
+  uint64_t* census_used = nullptr;      // a mask a block
+  uint32_t* census_starts = nullptr;    // clusters that start in each workgroup's blocks
+  uint64_t* census_base = nullptr;      // their exclusive sums, the total, the longest length
 };
 
 struct Filter {
@@ -129,7 +133,10 @@ void free_enum_space(EnumSpace& e) {
   dev_free(e.t.stats);
   dev_free(e.move_items);
   dev_free(e.move_counts);
-  e.groups = e.move_cap = 0;
+  dev_free(e.census_used);
+  dev_free(e.census_starts);
+  dev_free(e.census_base);
+  e.groups = e.move_cap = e.census_blocks = 0;
 }
 
 // room for `groups` groups (the caller holds e.mu)
@@ -1231,36 +1238,30 @@ extern "C" int qf_cluster_census(QF* qf, uint64_t* lengths, uint64_t cap, uint64
   if (hist && (nbins == 0 || nbins > 4096)) return -2;
   const uint64_t nb = f->host.nblocks;
   const uint64_t nwg = gqf_census_wgs(nb);
-  uint64_t* used = nullptr;
-  uint32_t* wg_starts = nullptr;
-  uint64_t* wg_base = nullptr;
-  unsigned long long* mx = nullptr;
-  dev_alloc(&used, nb);
-  dev_alloc(&wg_starts, nwg);
-  dev_alloc(&wg_base, nwg + 1);
-  dev_alloc(&mx, 1);
-  int rc = -3;
-  if (used && wg_starts && wg_base && mx) {
-    GQF_CHECK(hipDeviceSynchronize());
-    GQF_CHECK(hipMemset(mx, 0, sizeof(unsigned long long)));
-    gqf_launch_census(f->dev, nb, used, wg_starts, wg_base, lengths, lengths ? cap : 0,
-                      (unsigned long long*)hist, hist ? nbins : 0, mx, nullptr);
-    uint64_t nc = 0;
-    unsigned long long m = 0;
-    hipError_t e = hipMemcpy(&nc, wg_base + nwg, sizeof(nc), hipMemcpyDeviceToHost);
-    if (e == hipSuccess) e = hipMemcpy(&m, mx, sizeof(m), hipMemcpyDeviceToHost);
-    note_error(e, "qf_cluster_census");
-    if (e == hipSuccess) {
-      if (num_clusters) *num_clusters = nc;
-      if (max_len) *max_len = (uint64_t)m;
-      rc = 0;
-    }
+  std::lock_guard<std::mutex> lk(f->es.mu);
+  EnumSpace& e = f->es;
+  GQF_CHECK(hipDeviceSynchronize());
+  if (nb > e.census_blocks) {
+    dev_free(e.census_used);
+    dev_free(e.census_starts);
+    dev_free(e.census_base);
+    dev_alloc(&e.census_used, nb);
+    dev_alloc(&e.census_starts, nwg);
+    dev_alloc(&e.census_base, nwg + 2);
+    e.census_blocks = e.census_used && e.census_starts && e.census_base ? nb : 0;
+    if (!e.census_blocks) return -3;
   }
-  dev_free(used);
-  dev_free(wg_starts);
-  dev_free(wg_base);
-  dev_free(mx);
-  return rc;
+  uint64_t* total = e.census_base + nwg;  // the number of clusters, then the longest length
+  GQF_CHECK(hipMemset(total + 1, 0, sizeof(uint64_t)));
+  gqf_launch_census(f->dev, nb, e.census_used, e.census_starts, e.census_base, lengths, lengths ? cap : 0,
+                    (unsigned long long*)hist, hist ? nbins : 0, (unsigned long long*)(total + 1), nullptr);
+  uint64_t out[2] = {0, 0};
+  const hipError_t err = hipMemcpy(out, total, sizeof(out), hipMemcpyDeviceToHost);
+  note_error(err, "qf_cluster_census");
+  if (err != hipSuccess) return -3;
+  if (num_clusters) *num_clusters = out[0];
+  if (max_len) *max_len = out[1];
+  return 0;
 }
 
 extern "C" uint64_t qf_serialize(QF* qf, const char* filename) {

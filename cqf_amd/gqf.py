@@ -373,17 +373,20 @@ class GQF:
         """(lengths int64 device tensor or None, histogram or None, max length)."""
         import torch
         nc, mx = _u64(), _u64()
-        rc = self._lib.qf_cluster_census(self.handle, None, 0, None, 0, ctypes.byref(nc), ctypes.byref(mx))
-        if rc != 0:
-            raise RuntimeError(f"qf_cluster_census rc={rc}")
-        lens = torch.empty(int(nc.value), dtype=torch.int64, device="cuda") if lengths else None
-        hist = torch.zeros(nbins, dtype=torch.int64, device="cuda") if nbins else None
-        if lengths or nbins:
-            rc = self._lib.qf_cluster_census(self.handle, _ptr(lens) if lengths else None,
-                                             lens.numel() if lengths else 0, _ptr(hist) if nbins else None,
+
+        def census(lens, hist):
+            rc = self._lib.qf_cluster_census(self.handle, None if lens is None else _ptr(lens),
+                                             0 if lens is None else lens.numel(), None if hist is None else _ptr(hist),
                                              nbins, ctypes.byref(nc), ctypes.byref(mx))
             if rc != 0:
                 raise RuntimeError(f"qf_cluster_census rc={rc}")
+
+        lens = None
+        if lengths:  # one pass for their number
+            census(None, None)
+            lens = torch.empty(int(nc.value), dtype=torch.int64, device="cuda")
+        hist = torch.zeros(nbins, dtype=torch.int64, device="cuda") if nbins else None
+        census(lens, hist)
         return lens, hist, int(mx.value)
 
     def save(self, path):

@@ -314,8 +314,8 @@ int qf_get_stats(QF *qf, uint64_t *nelts, uint64_t *ndistinct_elts, uint64_t *no
  * of cap entries or NULL; hist: device array of nbins (<= 4096) u64
  * counters or NULL, ADDED to (bin i counts clusters of length i, the last
  * bin those of length >= nbins - 1); *num_clusters and *max_len are host
- * outputs, either may be NULL.  Allocates 8 bytes per 64-slot block for
- * the call.  Synchronises. */
+ * outputs, either may be NULL.  The first call allocates 8 bytes per 64-slot
+ * block, which the filter keeps.  Synchronises. */
 int qf_cluster_census(QF *qf, uint64_t *lengths, uint64_t cap, uint64_t *hist, uint32_t nbins,
                       uint64_t *num_clusters, uint64_t *max_len);
 
