@@ -16,15 +16,13 @@
 //      most frequent ids are three in four draws); the other keys of a wave
 //      are queued in LDS and taken 64 at a time (so the wave's lanes are
 //      full), hashed and counted in an 8192-entry LDS hash table.  The
-//      workgroup's (hash, count) entries then go to staging buckets chosen
-//      by hash, with one reserving atomic per bucket per workgroup;
+//      workgroup's (hash, count) entries then go to staging buckets, by the
+//      hash's top bits, with one reserving atomic per bucket per workgroup;
 //   3. gqf_agg_merge: one workgroup per bucket sums its entries by hash in
-//      LDS and writes the distinct ones out as (index << width) | hash, plus
-//      the count by index; an LSD sort of the low `width` bits (the bits the
-//      sort orders for the hash width, see gqf_sort_width) orders them;
-//   4. gqf_agg_extract / _scan_tiles / _positions split them into sorted
-//      hashes and counts (the reduce_by_key outputs) and the exclusive
-//      prefix sums of the counts;
+//      LDS and leaves the distinct ones in ascending order;
+//   4. gqf_agg_place puts the buckets one behind the other: sorted hashes and
+//      counts (the reduce_by_key outputs) and the exclusive prefix sums of
+//      the counts;
 //   5. gqf_agg_tile_starts / gqf_agg_expand write every hash count times
 //      into `keys`: the ascending hashes the sort would have left there.
 // Any table or bucket that runs out of room sets ctrl[2] and the batch
@@ -41,6 +39,8 @@ constexpr int kSampleLog = 13;
 constexpr int kSampleCap = 1 << kSampleLog;
 constexpr int kHot = GQF_AGG_HOT;
 constexpr int kBuckets = GQF_AGG_BUCKETS;
+constexpr int kBucketBits = 9;
+static_assert(kBuckets == 1 << kBucketBits, "buckets by top bits");
 constexpr uint32_t kBucketCap = GQF_AGG_BUCKET_CAP;
 constexpr int kTileThreads = 1024;       // threads per workgroup of gqf_agg_tiles
 constexpr int kTileWaves = kTileThreads / 64;
@@ -56,16 +56,19 @@ constexpr int kMergeThreads = 1024;
 constexpr int kMergeLog = 13;
 constexpr int kMergeCap = 1 << kMergeLog;  // distinct hashes a bucket may hold (3/4 of it used)
 constexpr int kMergeProbe = 64;
-constexpr int kScanItems = 16;
-constexpr int kScanTile = kThreads * kScanItems;  // 4096 entries per scan tile
+static_assert(kMergeCap <= (int)kBucketCap / 2 && kMergeLog + 40 - kBucketBits < 64, "a bucket's sorted entries");
 constexpr int kExpandTile = kThreads * 16;        // 4096 output keys per expand workgroup
 
 __device__ inline uint32_t slot_of(uint64_t h, int log_cap) {
   return (uint32_t)((h * 0x9E3779B97F4A7C15ULL) >> (64 - log_cap));
 }
 
-__device__ inline uint32_t bucket_of(uint64_t h) {  // staging bucket of a hash
-  return (uint32_t)(((h ^ (h >> 29)) * 0xBF58476D1CE4E5B9ULL) >> 55) & (kBuckets - 1);
+// The staging bucket of a hash of `bits` bits is its top bits, so the buckets
+// are in hash order.  The hash permutes the keys, so distinct keys spread
+// over the buckets evenly; a bucket that fills all the same sends the batch to
+// the sort.
+__host__ __device__ inline int bucket_shift(int bits) {
+  return bits > kBucketBits ? bits - kBucketBits : 0;
 }
 
 // exclusive scan of one value per thread over a workgroup of T threads;
@@ -102,7 +105,7 @@ __device__ inline uint32_t wave_sum(uint32_t v) {
 }  // namespace
 
 // ctrl[0] = distinct keys among kSample keys spread over the batch;
-// ctrl[1..3] = 0 (distinct hashes, overflow flag, output cursor);
+// ctrl[1..3] = 0 (distinct hashes, overflow flag, unused);
 // fill[0 .. kBuckets) = 0; hot[0] = number of hot keys, hot[1 ..] = the
 // masked keys seen at least twice in the sample, most frequent first
 extern "C" __global__ void __launch_bounds__(kThreads)
@@ -172,7 +175,7 @@ gqf_agg_sample(const uint64_t* __restrict__ keys, uint64_t n, uint64_t mask, uin
 }
 
 extern "C" __global__ void __launch_bounds__(kTileThreads)
-gqf_agg_tiles(const uint64_t* __restrict__ keys, uint64_t n, uint64_t mask, int vshift,
+gqf_agg_tiles(const uint64_t* __restrict__ keys, uint64_t n, uint64_t mask, int vshift, int bshift,
               const uint64_t* __restrict__ hot, uint64_t* __restrict__ stage, uint32_t* __restrict__ fill,
               uint32_t* __restrict__ ctrl) {
   // LDS entry: (hash << kCountBits) | count, kLocalEmpty when free (hashes
@@ -228,7 +231,7 @@ gqf_agg_tiles(const uint64_t* __restrict__ keys, uint64_t n, uint64_t mask, int 
       }
       s = (s + 1) & (kLocalCap - 1);
     }
-    const uint32_t b = bucket_of(h);
+    const uint32_t b = (uint32_t)(h >> bshift);
     const uint32_t at = atomicAdd(&fill[b], 1u);
     if (at < kBucketCap) stage[(uint64_t)b * kBucketCap + at] = tag | 1ULL;
     else atomicOr(&ctrl[2], 1u);
@@ -290,7 +293,7 @@ gqf_agg_tiles(const uint64_t* __restrict__ keys, uint64_t n, uint64_t mask, int 
       const uint32_t j = threadIdx.x;
       e[k] = j < nhot && hotsum[j] ? (((gqf_hash64(hot[1 + j], mask) << vshift) << kCountBits) | hotsum[j]) : kLocalEmpty;
     }
-    off[k] = e[k] != kLocalEmpty ? atomicAdd(&u.b.bcount[bucket_of(e[k] >> kCountBits)], 1u) : 0u;
+    off[k] = e[k] != kLocalEmpty ? atomicAdd(&u.b.bcount[(uint32_t)(e[k] >> kCountBits >> bshift)], 1u) : 0u;
   }
   __syncthreads();
   for (int b = threadIdx.x; b < kBuckets; b += kTileThreads)
@@ -299,25 +302,27 @@ gqf_agg_tiles(const uint64_t* __restrict__ keys, uint64_t n, uint64_t mask, int 
 #pragma unroll
   for (int k = 0; k <= kPer; k++) {
     if (e[k] == kLocalEmpty) continue;
-    const uint32_t b = bucket_of(e[k] >> kCountBits);
+    const uint32_t b = (uint32_t)(e[k] >> kCountBits >> bshift);
     const uint32_t at = u.b.bbase[b] + off[k];
     if (at < kBucketCap) stage[(uint64_t)b * kBucketCap + at] = e[k];
     else atomicOr(&ctrl[2], 1u);
   }
 }
 
-// one workgroup per staging bucket: sums the bucket's entries by hash in
-// LDS, then writes its distinct hashes as comp[idx] = (idx << width) | hash,
-// cnt[idx] = count, idx from the cursor ctrl[3] (one atomic per
-// workgroup); ctrl[1] += distinct hashes; ctrl[2] set when the LDS table
-// or cnt (cnt_cap entries) has no room
+// One workgroup per staging bucket: sums the bucket's entries by hash in LDS
+// and sorts the distinct ones (bitonic, of hash below the bucket's and table
+// slot), which it leaves at the start of the bucket (hashes) and of its second
+// half (counts).  fill[b] = their number, sums[b] = their counts' sum;
+// ctrl[1] += distinct hashes; ctrl[2] set when the LDS table has no room.
+// 217,000 distinct hashes of 2^26 keys: 41 us, and 6 us for gqf_agg_place; an
+// LSD sort of (index, hash) and the passes that split it again took fifteen
+// launches and 159 us behind a merge of 26 us.
 extern "C" __global__ void __launch_bounds__(kMergeThreads)
-gqf_agg_merge(const uint64_t* __restrict__ stage, const uint32_t* __restrict__ fill, int width,
-              uint64_t* __restrict__ comp, uint64_t* __restrict__ cnt, uint64_t cnt_cap, uint32_t* __restrict__ ctrl) {
+gqf_agg_merge(uint64_t* __restrict__ stage, uint32_t* __restrict__ fill, int bshift, uint64_t* __restrict__ sums,
+              uint32_t* __restrict__ ctrl) {
   __shared__ unsigned long long mk[kMergeCap];
   __shared__ unsigned long long mc[kMergeCap];
   __shared__ uint32_t mfill;
-  __shared__ uint32_t wg_base;
   for (int i = threadIdx.x; i < kMergeCap; i += kMergeThreads) {
     mk[i] = kEmpty;
     mc[i] = 0;
@@ -353,95 +358,85 @@ gqf_agg_merge(const uint64_t* __restrict__ stage, const uint32_t* __restrict__ f
   }
   __syncthreads();
   constexpr int kPer = kMergeCap / kMergeThreads;
+  const uint64_t low = (1ULL << bshift) - 1;  // at most 31 bits
+  uint64_t key[kPer];
   uint32_t mine = 0;
 #pragma unroll
-  for (int k = 0; k < kPer; k++) mine += mk[threadIdx.x * kPer + k] != kEmpty ? 1u : 0u;
-  uint64_t total;
-  const uint32_t before = (uint32_t)block_scan<kMergeThreads>(mine, &total);
-  if (threadIdx.x == 0) {
-    wg_base = total ? atomicAdd(&ctrl[3], (uint32_t)total) : 0u;
-    if (total) atomicAdd(&ctrl[1], (uint32_t)total);
-  }
-  __syncthreads();
-  uint64_t idx = (uint64_t)wg_base + before;
-#pragma unroll
   for (int k = 0; k < kPer; k++) {
-    const uint32_t s = threadIdx.x * kPer + k;
-    const uint64_t h = mk[s];
-    if (h == kEmpty) continue;
-    if (idx < cnt_cap) {
-      comp[idx] = (idx << width) | h;
-      cnt[idx] = mc[s];
-    } else {
-      atomicOr(&ctrl[2], 1u);
-    }
-    idx++;
+    const uint32_t s = threadIdx.x + (uint32_t)(k * kMergeThreads);
+    key[k] = mk[s] != kEmpty ? (mk[s] & low) << kMergeLog | s : kEmpty;
+    mine += key[k] != kEmpty ? 1u : 0u;
   }
-}
-
-// sorted comp -> ukeys (hashes) and ucounts; tile_sums[t] = sum of the counts of scan tile t
-extern "C" __global__ void __launch_bounds__(kThreads)
-gqf_agg_extract(const uint64_t* __restrict__ comp, uint64_t m, int width, const uint64_t* __restrict__ cnt,
-                uint64_t* __restrict__ ukeys, uint64_t* __restrict__ ucounts, uint64_t* __restrict__ tile_sums) {
-  const uint64_t hmask = (1ULL << width) - 1;
-  uint64_t sum = 0;
-  for (int k = 0; k < kScanItems; k++) {
-    const uint64_t i = (uint64_t)blockIdx.x * kScanTile + (uint64_t)k * kThreads + threadIdx.x;
-    if (i < m) {
-      const uint64_t c = comp[i];
-      const uint64_t v = cnt[c >> width];
-      ukeys[i] = c & hmask;
-      ucounts[i] = v;
-      sum += v;
+  uint64_t total;
+  uint32_t at = (uint32_t)block_scan<kMergeThreads>(mine, &total);  // all of mk is read
+#pragma unroll
+  for (int k = 0; k < kPer; k++)
+    if (key[k] != kEmpty) mk[at++] = key[k];
+  const uint32_t m = (uint32_t)total;
+  uint32_t size = 2;
+  while (size < m) size *= 2;
+  for (uint32_t i = m + threadIdx.x; i < size; i += kMergeThreads) mk[i] = kEmpty;  // above every key
+  __syncthreads();
+  for (uint32_t len = 2; len <= size; len *= 2) {
+    for (uint32_t stride = len / 2; stride > 0; stride /= 2) {
+      for (uint32_t t = threadIdx.x; t < size / 2; t += kMergeThreads) {
+        const uint32_t i = 2 * t - (t & (stride - 1)), j = i + stride;
+        const unsigned long long x = mk[i], y = mk[j];
+        if ((x > y) == ((i & len) == 0)) {
+          mk[i] = y;
+          mk[j] = x;
+        }
+      }
+      __syncthreads();
     }
   }
-  uint64_t total;
-  (void)block_scan<kThreads>(sum, &total);
-  if (threadIdx.x == 0) tile_sums[blockIdx.x] = total;
-}
-
-// exclusive scan in place of ntiles (<= kScanTile) tile sums, one workgroup
-extern "C" __global__ void __launch_bounds__(kThreads)
-gqf_agg_scan_tiles(uint64_t* __restrict__ tile_sums, uint32_t ntiles) {
-  uint64_t v[kScanItems];
+  uint64_t* out = stage + (uint64_t)b * kBucketCap;
   uint64_t sum = 0;
-#pragma unroll
-  for (int k = 0; k < kScanItems; k++) {
-    const uint32_t i = threadIdx.x * kScanItems + k;
-    v[k] = i < ntiles ? tile_sums[i] : 0;
-    sum += v[k];
+  for (uint32_t i = threadIdx.x; i < m; i += kMergeThreads) {
+    const uint64_t x = mk[i], c = mc[x & (kMergeCap - 1)];
+    out[i] = (uint64_t)b << bshift | x >> kMergeLog;
+    out[kBucketCap / 2 + i] = c;
+    sum += c;
   }
-  uint64_t total;
-  uint64_t run = block_scan<kThreads>(sum, &total);
-#pragma unroll
-  for (int k = 0; k < kScanItems; k++) {
-    const uint32_t i = threadIdx.x * kScanItems + k;
-    if (i < ntiles) tile_sums[i] = run;
-    run += v[k];
+  (void)block_scan<kMergeThreads>(sum, &total);
+  if (threadIdx.x == 0) {
+    fill[b] = m;
+    sums[b] = total;
+    if (m) atomicAdd(&ctrl[1], m);
   }
 }
 
-// upos[i] = sum of ucounts[0 .. i) for i < m, upos[m] = n
+// One workgroup per bucket: its distinct hashes and their counts to their
+// places in ukeys / ucounts, behind those of the buckets before it, and the
+// prefix sums of the counts to upos (upos[m] = n)
 extern "C" __global__ void __launch_bounds__(kThreads)
-gqf_agg_positions(const uint64_t* __restrict__ ucounts, uint64_t m, uint64_t n, const uint64_t* __restrict__ tile_sums,
-                  uint64_t* __restrict__ upos) {
-  // thread t takes kScanItems consecutive entries of the tile
-  const uint64_t first = (uint64_t)blockIdx.x * kScanTile + (uint64_t)threadIdx.x * kScanItems;
-  uint64_t v[kScanItems];
-  uint64_t sum = 0;
-#pragma unroll
-  for (int k = 0; k < kScanItems; k++) {
-    v[k] = first + k < m ? ucounts[first + k] : 0;
-    sum += v[k];
+gqf_agg_place(const uint64_t* __restrict__ stage, const uint32_t* __restrict__ fill, const uint64_t* __restrict__ sums,
+              uint64_t m, uint64_t n, uint64_t* __restrict__ ukeys, uint64_t* __restrict__ ucounts,
+              uint64_t* __restrict__ upos) {
+  const uint32_t b = blockIdx.x;
+  uint64_t before = 0, sum = 0;
+  for (uint32_t i = threadIdx.x; i < b; i += kThreads) {
+    before += fill[i];
+    sum += sums[i];
   }
-  uint64_t total;
-  uint64_t run = tile_sums[blockIdx.x] + block_scan<kThreads>(sum, &total);
-#pragma unroll
-  for (int k = 0; k < kScanItems; k++) {
-    if (first + k < m) upos[first + k] = run;
-    run += v[k];
+  uint64_t base, pos;
+  (void)block_scan<kThreads>(before, &base);
+  (void)block_scan<kThreads>(sum, &pos);
+  const uint64_t* in = stage + (uint64_t)b * kBucketCap;
+  const uint32_t nb = fill[b];
+  for (uint32_t i0 = 0; i0 < nb; i0 += kThreads) {
+    const uint32_t i = i0 + threadIdx.x;
+    const uint64_t c = i < nb ? in[kBucketCap / 2 + i] : 0;
+    uint64_t tot;
+    const uint64_t run = pos + block_scan<kThreads>(c, &tot);
+    pos += tot;
+    if (i < nb) {
+      ukeys[base + i] = in[i];
+      ucounts[base + i] = c;
+      upos[base + i] = run;
+    }
   }
-  if (blockIdx.x == 0 && threadIdx.x == 0) upos[m] = n;
+  if (b == 0 && threadIdx.x == 0) upos[m] = n;
 }
 
 // start[t] = the distinct index whose keys cover output position
@@ -498,37 +493,29 @@ void gqf_launch_agg_sample(const uint64_t* keys, uint64_t n, uint64_t mask, uint
   hipLaunchKernelGGL(gqf_agg_sample, dim3(1), dim3(kThreads), 0, s, keys, n, mask, ctrl, fill, hot);
 }
 
-void gqf_launch_agg_tiles(const uint64_t* keys, uint64_t n, uint64_t mask, int vshift, const uint64_t* hot,
+void gqf_launch_agg_tiles(const uint64_t* keys, uint64_t n, uint64_t mask, int vshift, int bits, const uint64_t* hot,
                           uint64_t* stage, uint32_t* fill, uint32_t* ctrl, hipStream_t s) {
   // one workgroup per tile (131072 keys), two resident per CU
   const uint64_t g = (n + kTileKeys - 1) / kTileKeys;
   gqf_prof_begin("reduce_count", s);
-  hipLaunchKernelGGL(gqf_agg_tiles, dim3((uint32_t)g), dim3(kTileThreads), 0, s, keys, n, mask, vshift, hot, stage,
-                     fill, ctrl);
+  hipLaunchKernelGGL(gqf_agg_tiles, dim3((uint32_t)g), dim3(kTileThreads), 0, s, keys, n, mask, vshift,
+                     bucket_shift(bits), hot, stage, fill, ctrl);
   gqf_prof_end("reduce_count", s);
 }
 
-void gqf_launch_agg_merge(const uint64_t* stage, const uint32_t* fill, int width, uint64_t* comp, uint64_t* cnt,
-                          uint64_t cnt_cap, uint32_t* ctrl, hipStream_t s) {
+void gqf_launch_agg_merge(uint64_t* stage, uint32_t* fill, int bits, uint64_t* sums, uint32_t* ctrl, hipStream_t s) {
   gqf_prof_begin("reduce_merge", s);
-  hipLaunchKernelGGL(gqf_agg_merge, dim3(kBuckets), dim3(kMergeThreads), 0, s, stage, fill, width, comp, cnt, cnt_cap,
+  hipLaunchKernelGGL(gqf_agg_merge, dim3(kBuckets), dim3(kMergeThreads), 0, s, stage, fill, bucket_shift(bits), sums,
                      ctrl);
   gqf_prof_end("reduce_merge", s);
 }
 
-void gqf_launch_agg_finish(uint64_t* keys, uint64_t n, uint64_t m, int width, uint64_t* comp, uint64_t* cnt,
-                           uint64_t* tmp, uint32_t* hist, uint32_t* totals, uint64_t* tile_sums, uint32_t* starts,
-                           uint64_t* ukeys, uint64_t* ucounts, uint64_t* upos, hipStream_t s) {
+void gqf_launch_agg_finish(uint64_t* keys, uint64_t n, uint64_t m, const uint64_t* stage, const uint32_t* fill,
+                           const uint64_t* sums, uint32_t* starts, uint64_t* ukeys, uint64_t* ucounts, uint64_t* upos,
+                           hipStream_t s) {
   gqf_prof_begin("reduce_finish", s);
-  // distinct hashes: the sort orders exactly the low `width` bits (its
-  // shape for `width` is the one that defined it) and carries the index along
-  gqf_launch_sort(comp, tmp, m, 0, 0, 0, width, 0, hist, totals, s);
-  const uint32_t stiles = (uint32_t)((m + kScanTile - 1) / kScanTile);
-  hipLaunchKernelGGL(gqf_agg_extract, dim3(stiles), dim3(kThreads), 0, s, (const uint64_t*)comp, m, width,
-                     (const uint64_t*)cnt, ukeys, ucounts, tile_sums);
-  hipLaunchKernelGGL(gqf_agg_scan_tiles, dim3(1), dim3(kThreads), 0, s, tile_sums, stiles);
-  hipLaunchKernelGGL(gqf_agg_positions, dim3(stiles), dim3(kThreads), 0, s, (const uint64_t*)ucounts, m, n,
-                     (const uint64_t*)tile_sums, upos);
+  hipLaunchKernelGGL(gqf_agg_place, dim3(kBuckets), dim3(kThreads), 0, s, stage, fill, sums, m, n, ukeys, ucounts,
+                     upos);
   const uint32_t etiles = (uint32_t)((n + kExpandTile - 1) / kExpandTile);
   hipLaunchKernelGGL(gqf_agg_tile_starts, dim3((etiles + 1 + 255) / 256), dim3(256), 0, s, (const uint64_t*)upos, m,
                      n, etiles, starts);

@@ -55,11 +55,9 @@ struct Workspace {
   uint8_t* wide_flags = nullptr;     // nregions, kept zero by the kernels
   uint32_t* wide_count = nullptr;    // GQF_WIDE_WORDS: count, flagged regions, finished workgroups
   unsigned long long* misses = nullptr;
-  // counting reduce (allocated on first use): hash table, counts by
-  // compaction index, scan tile sums, control words
+  // counting reduce (allocated on first use)
   uint64_t* agg_stage = nullptr;   // GQF_AGG_BUCKETS x GQF_AGG_BUCKET_CAP staged (hash, count) entries
-  uint64_t* agg_by_idx = nullptr;
-  uint64_t* agg_tiles = nullptr;
+  uint64_t* agg_sums = nullptr;    // the buckets' counts
   uint64_t* agg_hot = nullptr;
   uint32_t* agg_ctrl = nullptr;    // 4 control words, then the bucket fills
 };
@@ -201,8 +199,7 @@ void ensure_workspace(Filter* f, uint64_t n) {
 // count) pairs exactly as the sort and the run-length reduce would.
 // Batches of at least 2^22 keys whose sample of 4096 holds at most 2048
 // distinct keys try it; a batch whose distinct hashes do not fit (a staging
-// bucket, a bucket's LDS table or the 2^22 output entries) falls back to the
-// sort.  Reads the control words back, so it synchronises the stream twice
+// bucket or a bucket's LDS table) falls back to the sort.  Reads the control words back, so it synchronises the stream twice
 // (the reference's bulk_insert_reduce synchronises as well,
 // src/gqf.cu:3247-3250, and reads reduce_by_key's end back, :3273).
 // Returns false when not taken (nothing in `keys` changed); else *m_out =
@@ -217,18 +214,15 @@ bool stream_capturing(hipStream_t s) {
 
 bool reduce_by_counting(Filter* f, uint64_t n, uint64_t* keys, int bits, hipStream_t s, uint64_t* m_out) {
   Workspace& w = f->ws;
-  const int width = gqf_sort_width(bits, 0);
-  if (n < kAggMinKeys || bits > 40 || width + GQF_AGG_LOG_CAP > 64 || stream_capturing(s)) return false;
-  const uint64_t cap = 1ULL << GQF_AGG_LOG_CAP;
+  if (n < kAggMinKeys || bits > 40 || stream_capturing(s)) return false;
   {
     std::lock_guard<std::mutex> lk(f->mu);
     if (!w.agg_stage) {
       dev_alloc(&w.agg_stage, (uint64_t)GQF_AGG_BUCKETS * GQF_AGG_BUCKET_CAP);
-      dev_alloc(&w.agg_by_idx, cap);
-      dev_alloc(&w.agg_tiles, 4096);
+      dev_alloc(&w.agg_sums, GQF_AGG_BUCKETS);
       dev_alloc(&w.agg_hot, GQF_AGG_HOT + 1);
       dev_alloc(&w.agg_ctrl, 4 + GQF_AGG_BUCKETS);
-      if (!w.agg_stage || !w.agg_by_idx || !w.agg_tiles || !w.agg_hot || !w.agg_ctrl) return false;
+      if (!w.agg_stage || !w.agg_sums || !w.agg_hot || !w.agg_ctrl) return false;
     }
   }
   const uint64_t mask = gqf_mask(f->host.key_bits);
@@ -239,15 +233,13 @@ bool reduce_by_counting(Filter* f, uint64_t n, uint64_t* keys, int bits, hipStre
   GQF_CHECK(hipMemcpyAsync(ctrl, w.agg_ctrl, sizeof(ctrl), hipMemcpyDeviceToHost, s));
   GQF_CHECK(hipStreamSynchronize(s));
   if (ctrl[0] > GQF_AGG_SAMPLE / 2) return false;
-  gqf_launch_agg_tiles(keys, n, mask, vb, w.agg_hot, w.agg_stage, fill, w.agg_ctrl, s);
-  // comp goes to upos (free until the finish's prefix sums overwrite it)
-  gqf_launch_agg_merge(w.agg_stage, fill, width, w.upos, w.agg_by_idx, std::min(cap, w.cap), w.agg_ctrl, s);
+  gqf_launch_agg_tiles(keys, n, mask, vb, bits, w.agg_hot, w.agg_stage, fill, w.agg_ctrl, s);
+  gqf_launch_agg_merge(w.agg_stage, fill, bits, w.agg_sums, w.agg_ctrl, s);
   GQF_CHECK(hipMemcpyAsync(ctrl, w.agg_ctrl, sizeof(ctrl), hipMemcpyDeviceToHost, s));
   GQF_CHECK(hipStreamSynchronize(s));
   const uint64_t m = ctrl[1];
-  if (ctrl[2] != 0 || m > cap || m == 0) return false;
-  gqf_launch_agg_finish(keys, n, m, width, w.upos, w.agg_by_idx, w.tmp, w.hist, w.totals, w.agg_tiles, w.tile_heads,
-                        w.ukeys, w.ucounts, w.upos, s);
+  if (ctrl[2] != 0 || m == 0) return false;
+  gqf_launch_agg_finish(keys, n, m, w.agg_stage, fill, w.agg_sums, w.tile_heads, w.ukeys, w.ucounts, w.upos, s);
   *m_out = m;
   return true;
 }
@@ -499,8 +491,7 @@ void free_all_workspace(Workspace& w) {
   dev_free(w.wide_count);
   dev_free(w.misses);
   dev_free(w.agg_stage);
-  dev_free(w.agg_by_idx);
-  dev_free(w.agg_tiles);
+  dev_free(w.agg_sums);
   dev_free(w.agg_hot);
   dev_free(w.agg_ctrl);
 }

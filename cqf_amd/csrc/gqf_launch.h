@@ -13,9 +13,6 @@ uint64_t gqf_sort_hist_words(uint64_t n);
 // digit_bits: 6..10 fixes the radix digit (passes rounded up to even), 0 picks 4 passes
 void gqf_launch_sort(uint64_t* keys, uint64_t* tmp, uint64_t n, int hash_it, uint64_t mask, int vshift, int bits,
                      int digit_bits, uint32_t* hist, uint32_t* totals, hipStream_t s);
-// the low bits gqf_launch_sort orders for these arguments (passes x digit,
-// at least `bits`): bits above them ride along in their stable order
-int gqf_sort_width(int bits, int digit_bits);
 #define GQF_SORT_TOTALS 2048  // words of the `totals` buffer: digit totals, then bucket starts
 // slow: GQF_SORT_MAX_BUCKETS flags, zero between calls (the kernels leave them so)
 #define GQF_SORT_MAX_BUCKETS 1024
@@ -55,35 +52,32 @@ void gqf_launch_sort_fast(uint64_t* keys, uint64_t* tmp, uint64_t n, bool tagged
                           uint64_t tag = 0);
 
 // Counting reduce of duplicate-heavy batches (gqf_agg.hip).  ctrl: 4 words
-// (distinct keys in the sample, distinct hashes, overflow flag, output
-// cursor); fill: GQF_AGG_BUCKETS words; hot: GQF_AGG_HOT + 1 words; stage:
+// (distinct keys in the sample, distinct hashes, overflow flag, unused);
+// fill: GQF_AGG_BUCKETS words; sums: GQF_AGG_BUCKETS words; hot: GQF_AGG_HOT + 1 words; stage:
 // GQF_AGG_BUCKETS x GQF_AGG_BUCKET_CAP words.
 #define GQF_AGG_SAMPLE 4096
 #define GQF_AGG_HOT 8                // keys counted in registers (the sample's most frequent)
-#define GQF_AGG_BUCKETS 512          // staging buckets, by hash
+#define GQF_AGG_BUCKETS 512          // staging buckets, by the hash's top bits
 #define GQF_AGG_BUCKET_CAP 32768     // staging entries per bucket (2^24 in all)
-#define GQF_AGG_LOG_CAP 22           // distinct hashes a counted batch may hold
 // sample: ctrl[0] = distinct keys among 4096 spread over the batch, the hot
 // keys, ctrl[1..3] and fill zeroed
 void gqf_launch_agg_sample(const uint64_t* keys, uint64_t n, uint64_t mask, uint32_t* ctrl, uint32_t* fill,
                            uint64_t* hot, hipStream_t s);
 // counts every key's slot hash per 131072-key tile and stages the tiles'
-// (hash, count) entries by bucket; ctrl[2] != 0 if a bucket ran out of room
-void gqf_launch_agg_tiles(const uint64_t* keys, uint64_t n, uint64_t mask, int vshift, const uint64_t* hot,
+// (hash, count) entries by bucket; ctrl[2] != 0 if a bucket ran out of room.
+// bits: of the hashes, at most 40
+void gqf_launch_agg_tiles(const uint64_t* keys, uint64_t n, uint64_t mask, int vshift, int bits, const uint64_t* hot,
                           uint64_t* stage, uint32_t* fill, uint32_t* ctrl, hipStream_t s);
-// sums the staged entries by hash: comp[idx] = (idx << width) | hash,
-// cnt[idx] = count for the ctrl[1] distinct hashes (ctrl[2] != 0 if they
-// did not fit: LDS per bucket or cnt_cap)
-void gqf_launch_agg_merge(const uint64_t* stage, const uint32_t* fill, int width, uint64_t* comp, uint64_t* cnt,
-                          uint64_t cnt_cap, uint32_t* ctrl, hipStream_t s);
+// sums the staged entries by hash and leaves each bucket's distinct ones
+// sorted in its place; fill and sums: their numbers and counts, ctrl[1] the
+// number of all (ctrl[2] != 0 if a bucket's did not fit in LDS)
+void gqf_launch_agg_merge(uint64_t* stage, uint32_t* fill, int bits, uint64_t* sums, uint32_t* ctrl, hipStream_t s);
 // the m merged entries -> ascending ukeys / ucounts (m each), upos (m + 1
 // prefix sums) and keys = each hash count times in ascending order.
-// width = gqf_sort_width(hash bits, 0); comp: m words (may be upos);
-// tmp / hist / totals: a sort of m keys; tile_sums: 4096 words; starts:
-// n / 4096 + 2 words.
-void gqf_launch_agg_finish(uint64_t* keys, uint64_t n, uint64_t m, int width, uint64_t* comp, uint64_t* cnt,
-                           uint64_t* tmp, uint32_t* hist, uint32_t* totals, uint64_t* tile_sums, uint32_t* starts,
-                           uint64_t* ukeys, uint64_t* ucounts, uint64_t* upos, hipStream_t s);
+// starts: n / 4096 + 2 words.
+void gqf_launch_agg_finish(uint64_t* keys, uint64_t n, uint64_t m, const uint64_t* stage, const uint32_t* fill,
+                           const uint64_t* sums, uint32_t* starts, uint64_t* ukeys, uint64_t* ucounts, uint64_t* upos,
+                           hipStream_t s);
 
 // run-length reduce of sorted keys -> ukeys/ucounts, count -> *m_dev.
 // tile_heads: ceil(n/4096) words; upos: n words.

@@ -1254,12 +1254,6 @@ void sort_shape(int bits, int digit_bits, int* passes, int* digit) {
 }
 }  // namespace
 
-int gqf_sort_width(int bits, int digit_bits) {
-  int passes, digit;
-  sort_shape(bits, digit_bits, &passes, &digit);
-  return passes * digit;
-}
-
 void gqf_launch_sort(uint64_t* keys, uint64_t* tmp, uint64_t n, int hash_it, uint64_t mask, int vshift, int bits,
                      int digit_bits, uint32_t* hist, uint32_t* totals, hipStream_t s) {
   if (n == 0) return;
