@@ -299,43 +299,6 @@ gqf_seq_tag_kernel(const QF* __restrict__ qfp, uint64_t* __restrict__ keys, uint
   }
 }
 
-// The first of the n > 0 items of `mut`, sorted by hash, whose hash is not
-// below h, and `item`, that item (where it is not n).  Hashes are spread
-// evenly, so it is looked for at h's share of the range (`per`: items per
-// hash value) and twice more at the distance that the item there shows (about
-// sqrt(n) / 2 items off, then the square root of that, and its root), then
-// between steps that widen from there, and by halves; items with few distinct
-// hashes cost some steps more.  Bound by the rate of loads that miss L1, as
-// nearly all of these do (16 waves a CU pass through it): halving the whole
-// batch takes 20 of them for 0.7 M items and took 127 us for 1.65 M queries,
-// this takes 8 and 77 us.
-__device__ __forceinline__ uint64_t first_item_of(const uint64_t* __restrict__ mut, uint64_t n, uint64_t h, double per,
-                                                  uint64_t& item) {
-  auto guess = [&](double x) {
-    const uint64_t g = x > 0 ? (uint64_t)x : 0ULL;
-    return g < n ? g : n - 1;
-  };
-  uint64_t g = guess((double)h * per), v = mut[g];
-#pragma unroll
-  for (int k = 0; k < 2; k++) {
-    g = guess((double)g + ((double)h - (double)(v & GQF_SEQ_HASH_MASK)) * per);
-    v = mut[g];
-  }
-  const bool up = (v & GQF_SEQ_HASH_MASK) < h;
-  uint64_t lo = up ? g + 1 : 0, hi = up ? n : g;  // items before lo are below h, those from hi on are not
-  item = v;                                       // item hi, where hi < n
-  auto look = [&](uint64_t p) {
-    const uint64_t t = mut[p];
-    const bool below = (t & GQF_SEQ_HASH_MASK) < h;
-    if (below) lo = p + 1; else hi = p, item = t;
-    return below;
-  };
-  for (uint64_t step = 8; (up ? n - lo : hi) >= step; step *= 4)
-    if (look(up ? lo + step - 1 : hi - step) != up) break;
-  while (lo < hi) look((lo + hi) >> 1);
-  return lo;
-}
-
 // Query i (of request with sequence number qs) replays, on its count before
 // the mutation, the items of its hash from requests before qs, in order:
 // +1 for an insert, -1 floored at 0 for a delete (the reference's qf_insert
@@ -351,7 +314,7 @@ gqf_seq_adjust_kernel(const QF* __restrict__ qfp, const uint64_t* __restrict__ k
     const uint64_t qs = l.tag[seq_request_of(l, reqs.nreq, i)];
     const uint64_t h = gqf_key_hash(qf, keys[i]);
     uint64_t t = 0;
-    uint64_t j = first_item_of(mut, n_mut, h, (double)n_mut / (double)qf.range, t);
+    uint64_t j = gqf_first_item(mut, n_mut, GQF_SEQ_HASH_MASK, h, 0.0, (double)n_mut / (double)qf.range, t);
     if (j == n_mut || (t & GQF_SEQ_HASH_MASK) != h) continue;
     uint64_t c = counts[i];
     for (;;) {

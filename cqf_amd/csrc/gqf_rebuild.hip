@@ -2230,13 +2230,12 @@ gqf_region_bounds(const QF* __restrict__ qfp, const uint64_t* __restrict__ items
   const uint64_t r = wave * kBoundsPerWave + lane;
   const bool valid = r <= qf.nregions;
   const uint64_t n = n_dev ? *n_dev : n_host;
-  auto lower = [&](uint64_t bound) {
-    uint64_t lo = 0, hi = n;
-    while (lo < hi) {
-      const uint64_t mid = (lo + hi) >> 1;
-      if ((items[mid] & hmask) < bound) lo = mid + 1; else hi = mid;
-    }
-    return lo;
+  // first item not below a bound, from where even spreading between the first and the last puts it
+  const double first = n ? (double)(items[0] & hmask) : 0.0, last = n ? (double)(items[n - 1] & hmask) : 0.0;
+  const double per = (double)n / (last - first + 1.0);
+  auto lower = [&](uint64_t bound) -> uint64_t {
+    uint64_t item;
+    return n ? gqf_first_item(items, n, hmask, bound, first, per, item) : 0ULL;
   };
   uint64_t lo = 0;
   if (valid) {
