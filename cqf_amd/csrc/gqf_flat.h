@@ -677,9 +677,13 @@ __device__ __forceinline__ int rebuild(const QF& qf, uint64_t r, const uint64_t*
     const int32_t xn = max_i(max_i(below_i(incl, kNone), x0), 64 * lane - 1);
     const int32_t xo = sm.xold[lane];
     sm.xnew[lane] = xn;
-    // where the new layout meets the old one: the first block past the
-    // region whose earlier runs end where they did, inside the window
-    const uint64_t meet = __ballot(lane >= R && lane < nwin && xn == xo && xo < nslots);
+    // Where the new layout meets the old one: the first block past the region
+    // whose earlier runs end where they did, inside the window; for batches
+    // that the single-wave rebuild would walk, inside that block.  Which regions
+    // need the wide pass has to be the same there and here: in a table too full
+    // for a batch, what it keeps of the batch depends on the order.
+    const bool walked = kind != kAdd || n_items > 256;
+    const uint64_t meet = __ballot(lane >= R && lane < nwin && xn == xo && xo < nslots && (!walked || xo - 64 * lane < 63));
     if (lane == 0) {
       int res = kOk, bstar = nwin, bwrite = nwin;
       int32_t keep = INT32_MAX;

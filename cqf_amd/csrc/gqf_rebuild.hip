@@ -1201,18 +1201,6 @@ __device__ inline Span region_span(const QF& qf, uint64_t r, int W, bool concurr
   const uint64_t wmax = concurrent && 2 * R < (uint64_t)W ? 2 * R : (uint64_t)W;
   return {r * R, (int)R, (int)min(wmax, qf.nblocks - r * R)};
 }
-// Its first or second half, with what of the fast window stays inside the 2 R
-// blocks that are region r's while the other regions of its parity run: more
-// push blocks (40 behind the first half of 48 blocks, 40 behind the second).
-// nwin = 0 where the table ends before the half.
-__device__ inline Span half_span(const QF& qf, uint64_t r, int half) {
-  const int R = (int)qf.region_blocks, first = R / 2;
-  const uint64_t B0 = r * (uint64_t)R + (half ? (uint64_t)first : 0ULL);
-  if (B0 >= qf.nblocks) return {B0, 0, 0};
-  const int room = half ? 2 * R - first : 2 * R;
-  return {B0, half ? R - first : first, (int)min((uint64_t)(room < kWinFast ? room : kWinFast), qf.nblocks - B0)};
-}
-
 template <int W>
 __device__ __forceinline__ void load_lines(const QF& qf, const Span& sp, uint64_t s, uint64_t e,
                                            const uint64_t* __restrict__ items, Lines<W / 64>& L) {
@@ -2015,40 +2003,35 @@ __device__ inline bool wait_count(const uint32_t* ctr, uint32_t target, uint32_t
 // regions are cut into chains of closer ones, and each chain runs on its own
 // workgroup.  The last of them to finish clears the count.
 //
-// More (loads near 95%), in stages of kWideClassGrid workgroups:
-//   * stage 0 redoes every flagged region as two halves, the second first,
-//     each with more push blocks than the region had (half_span): what both
-//     touch are the 2 R blocks that belong to the region while its parity runs,
-//     so all run at once.  A region whose second half needs more stays flagged,
-//     one whose first half does too, with flag kFirstHalf;
-//   * stage 1 + c redoes what is left of class c: regions of one parity whose
-//     indices differ by at least `apart` (the widest window, 256 blocks, in
-//     regions) have disjoint windows, so region parity + 2 i is in class i mod
-//     ncls (ncls = ceil(apart / 2)).
-// The stages run one after another in ONE launch: each workgroup takes a
+// More (loads near 95%): class by class, kWideClassGrid workgroups each.
+// Regions of one parity whose indices differ by at least `apart` (the widest
+// window, 256 blocks, in regions) have disjoint windows, so region parity + 2 i
+// is in class i mod ncls (ncls = ceil(apart / 2)).
+// The classes run one after another in ONE launch: each workgroup takes a
 // ticket when it starts; tickets c * kWideClassGrid .. (c + 1) *
-// kWideClassGrid - 1 run stage c, after waiting for stage c - 1's finished
-// counter.  Every workgroup of stage c - 1 took its ticket before any of
-// stage c did, so it is running or done, and it waits only on earlier stages:
+// kWideClassGrid - 1 run class c, after waiting for class c - 1's finished
+// counter.  Every workgroup of class c - 1 took its ticket before any of
+// class c did, so it is running or done, and it waits only on earlier classes:
 // every wait ends.  (A wait past max_polls, 2^24 unless qf_set_wide_wait_bound
 // says otherwise, which no correct run reaches, flags the class's regions as
 // CLUSTER_OVERFLOW instead of rebuilding them.)  A workgroup takes every
-// kWideClassGrid-th region of its stage, so the flagged ones spread evenly.
+// kWideClassGrid-th region of its class, so the flagged ones spread evenly.
 // The last workgroup to finish clears every counter for the next phase.
 //
-// 3.4 M inserts from 90% to 95% load at 2^26 slots (thousands of regions
-// flagged in the odd phase): 1,376 -> 532 us for the pass without stage 0 and
-// with a workgroup taking 64 regions side by side; with nothing flagged a
-// launch is 4.6 us, one instead of two a phase.
-constexpr uint8_t kFirstHalf = 2;
-
+// With nothing flagged a launch is 4.6 us.  Two launches, one for each form,
+// took 9.2 us, and a workgroup that took 64 neighbouring candidates made the
+// pass 1,376 us instead of 800 for 3.4 M inserts from 90% to 95% load at 2^26
+// slots.
+// What a batch that a table cannot hold leaves in it depends on the order in
+// which its regions are redone and on which of them are given up whole, so
+// both stay as they are: redoing the flagged regions as halves of regions
+// first, all at once, took 532 us but kept other keys of such a batch.
 extern "C" __global__ void __launch_bounds__(64)
 gqf_rebuild_wide(const QF* __restrict__ qfp, const uint64_t* __restrict__ items,
                  const uint64_t* __restrict__ counts, const uint32_t* __restrict__ region_start,
                  int parity, int mode, uint8_t* __restrict__ wide_flags, uint32_t* __restrict__ wide_count,
                  uint32_t ncls, uint32_t max_polls) {
   __shared__ union {
-    Smem<kWinFast> fast;
     Smem<kWinMid> mid;
     Smem<kWinWide> wide;
   } sm;
@@ -2058,17 +2041,6 @@ gqf_rebuild_wide(const QF* __restrict__ qfp, const uint64_t* __restrict__ items,
   if (nflag == 0 || (nflag <= GQF_WIDE_LIST && blockIdx.x >= GQF_WIDE_LIST)) return;
   const QF qf = *qfp;
   const int lane = lane_id();
-  const uint64_t hmask = (mode & ~GQF_REBUILD_NO_SHIFT) == kSeq ? GQF_SEQ_HASH_MASK : ~0ULL;
-  // first item of region rr's second half
-  auto middle = [&](uint64_t rr) -> uint64_t {
-    const uint64_t bound = half_span(qf, rr, 1).B0 << 14;
-    uint64_t lo = region_start[rr], hi = region_start[rr + 1];
-    while (lo < hi) {
-      const uint64_t mid = (lo + hi) >> 1;
-      if ((items[mid] & hmask) < bound) lo = mid + 1; else hi = mid;
-    }
-    return lo;
-  };
   auto report = [&](uint64_t rr, int res) {
     if (lane == 0) {
       wide_flags[rr] = 0;
@@ -2079,29 +2051,12 @@ gqf_rebuild_wide(const QF* __restrict__ qfp, const uint64_t* __restrict__ items,
   };
   auto redo = [&](uint64_t rr) __attribute__((always_inline)) {
     const uint64_t s = region_start[rr];
-    const uint64_t e = wide_flags[rr] == kFirstHalf ? middle(rr) : (uint64_t)region_start[rr + 1];
+    const uint64_t e = region_start[rr + 1];
     int res = rebuild_region<kWinMid>(qf, rr, items, counts, s, e, mode, sm.mid, icnt, false);
     __syncthreads();
     if (res == kNeedWide) res = rebuild_region<kWinWide>(qf, rr, items, counts, s, e, mode, sm.wide, icnt, false);
     __syncthreads();
     report(rr, res);
-  };
-  auto redo_halves = [&](uint64_t rr) __attribute__((always_inline)) {
-    // (a region that may find the table full is redone as a whole: it must
-    // stay unchanged then)
-    if ((rr + 2) * qf.region_blocks >= qf.nblocks) return;
-    const uint64_t s = region_start[rr], e = region_start[rr + 1], m = middle(rr);
-    int res = kOk;
-#pragma unroll 1
-    for (int half = 1; half >= 0 && res == kOk; half--) {
-      const uint64_t a = half ? m : s, z = half ? e : m;
-      if (a < z)
-        res = rebuild_span<kWinFast, false>(qf, half_span(qf, rr, half), items, counts, a, z, mode, sm.fast, icnt, 0);
-      __syncthreads();
-      if (res == kOk && half && lane == 0) wide_flags[rr] = kFirstHalf;
-      __syncthreads();
-    }
-    if (res == kOk) report(rr, res);  // else its flag says what is left
   };
   uint32_t* finished = &wide_count[1 + GQF_WIDE_LIST];
   if (nflag <= GQF_WIDE_LIST) {
@@ -2141,35 +2096,33 @@ gqf_rebuild_wide(const QF* __restrict__ qfp, const uint64_t* __restrict__ items,
     return;
   }
   uint32_t* tickets = &wide_count[2 + GQF_WIDE_LIST];
-  uint32_t* stage_done = &wide_count[3 + GQF_WIDE_LIST];
+  uint32_t* class_done = &wide_count[3 + GQF_WIDE_LIST];
   if (lane == 0) ticket = atomicAdd(tickets, 1u);
   __syncthreads();
   const uint32_t t = ticket;
-  const uint32_t stage = t / kWideClassGrid, w = t % kWideClassGrid;
-  const bool ok = stage == 0 || wait_count(&stage_done[stage - 1], kWideClassGrid, max_polls);
+  const uint32_t cls = t / kWideClassGrid, w = t % kWideClassGrid;
+  const bool ok = cls == 0 || wait_count(&class_done[cls - 1], kWideClassGrid, max_polls);
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   const uint64_t nper = qf.nregions > (uint64_t)parity ? (qf.nregions - (uint64_t)parity + 1) / 2 : 0;
-  // candidate j of stage 0 is region parity + 2 j, of class c region parity +
-  // 2 (c + ncls j); workgroup w takes j = w, w + kWideClassGrid, ..., 64 at a time
-  const uint64_t first = stage ? stage - 1 : 0, step = stage ? ncls : 1;
-  const uint64_t ncand = nper > first ? (nper - first + step - 1) / step : 0;
+  // candidate j of class c is region parity + 2 (c + ncls j); workgroup w
+  // takes j = w, w + kWideClassGrid, ..., 64 at a time
+  const uint64_t ncand = nper > cls ? (nper - cls + ncls - 1) / ncls : 0;
   for (uint64_t j0 = w; j0 < ncand; j0 += (uint64_t)kWideClassGrid * 64) {
     const uint64_t j = j0 + (uint64_t)kWideClassGrid * (uint64_t)lane;
-    uint64_t m = __ballot(j < ncand && wide_flags[(uint64_t)parity + 2 * (first + step * j)]);
+    uint64_t m = __ballot(j < ncand && wide_flags[(uint64_t)parity + 2 * (cls + ncls * j)]);
     while (m) {
       const int l = __builtin_ctzll(m);
       m &= m - 1;
-      const uint64_t rr = (uint64_t)parity + 2 * (first + step * (j0 + (uint64_t)kWideClassGrid * (uint64_t)l));
-      if (stage == 0) redo_halves(rr);
-      else if (ok) redo(rr);
+      const uint64_t rr = (uint64_t)parity + 2 * (cls + ncls * (j0 + (uint64_t)kWideClassGrid * (uint64_t)l));
+      if (ok) redo(rr);
       else report(rr, kNeedWide);
     }
   }
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
   if (lane == 0) {
-    atomicAdd(&stage_done[stage], 1u);
+    atomicAdd(&class_done[cls], 1u);
     if (atomicAdd(finished, 1u) == gridDim.x - 1) {  // everyone is done: clear for the next phase
-      for (uint32_t c = 0; c <= ncls; c++) stage_done[c] = 0;
+      for (uint32_t c = 0; c < ncls; c++) class_done[c] = 0;
       *tickets = 0;
       *finished = 0;
       *(volatile uint32_t*)wide_count = 0;
@@ -2515,7 +2468,7 @@ void gqf_launch_rebuild(const QF* qf_dev, uint64_t nregions, uint64_t region_blo
                          list, list_count, parity, mode, wide_flags, wide_count);
     gqf_prof_end("rebuild_phase", s);
     gqf_prof_begin("rebuild_wide", s);
-    hipLaunchKernelGGL(gqf_rebuild_wide, dim3((1 + ncls) * kWideClassGrid), dim3(64), 0, s, qf_dev, items, counts,
+    hipLaunchKernelGGL(gqf_rebuild_wide, dim3(ncls * kWideClassGrid), dim3(64), 0, s, qf_dev, items, counts,
                        region_start, parity, mode, wide_flags, wide_count, ncls,
                        g_wide_max_polls.load(std::memory_order_relaxed));
     gqf_prof_end("rebuild_wide", s);
