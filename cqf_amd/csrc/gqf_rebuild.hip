@@ -2425,11 +2425,14 @@ std::atomic<uint32_t> g_wide_max_polls{kWideMaxPolls};
 uint32_t gqf_wide_wait_bound_set(uint32_t max_polls) { return g_wide_max_polls.exchange(max_polls); }
 
 // Batches of at least this many items per region on average take the
-// workgroup-wide rebuild (gqf_flat.h): inserts when regions start to outgrow
-// the item cache (256) and would walk their runs -- below that the shift path
-// is ahead (153 items a region at 2^26 slots: 97 us a launch against 280) --
-// and the other kinds sooner, as they always walk.
-constexpr uint64_t kFlatItems = 208, kFlatItemsMixed = 96;
+// workgroup-wide rebuild (gqf_flat.h): inserts when regions outgrow the item
+// cache (256) and would walk their runs, and sooner in tables whose phases of
+// single waves do not fill the chip; the other kinds sooner still, as they
+// always walk.  Filling to 65% load by shift path and walk, and dense: 2^23
+// slots, 212 items a region, 1,448 and 1,069 us; 2^24, 212, 1,760 and 1,710;
+// 2^25 (10,900 regions), 245, 2,394 and 2,679, 262, 2,587 and 2,420; 2^26, 215,
+// 3,244 and 5,429, 258, 4,018 and 4,428, 275, 4,767 and 4,401.
+constexpr uint64_t kFlatItems = 208, kFlatItemsMany = 260, kFlatManyRegions = 8192, kFlatItemsMixed = 96;
 bool gqf_rebuild_is_dense(uint64_t n_items, uint64_t nregions) { return n_items >= kFlatItems * nregions; }
 
 void gqf_launch_rebuild(const QF* qf_dev, uint64_t nregions, uint64_t region_blocks, const uint64_t* items,
@@ -2449,7 +2452,9 @@ void gqf_launch_rebuild(const QF* qf_dev, uint64_t nregions, uint64_t region_blo
     abort();
   }
   const int kind = mode == kSeq ? gqf_flat::kTagged : (counts ? gqf_flat::kCounts : gqf_flat::kAdd);
-  const bool flat = n_items >= (kind == gqf_flat::kAdd ? kFlatItems : kFlatItemsMixed) * nregions;
+  const uint64_t line = kind != gqf_flat::kAdd ? kFlatItemsMixed
+                        : nregions < kFlatManyRegions ? kFlatItems : kFlatItemsMany;
+  const bool flat = n_items >= line * nregions;
   mode |= gqf_rebuild_mode_flags();
   for (int parity = 0; parity < 2; parity++) {
     const uint32_t* list = region_list ? region_list + (size_t)parity * stride : nullptr;
