@@ -11,6 +11,8 @@ zipf_workload: n_draws samples of Zipf(s) over n_ids ids by inverse CDF
 key -- distinct in its low `distinct_bits` bits, so that a filter whose
 hash sees only key & (2^(q+8) - 1) counts every id separately.
 """
+import math
+
 import torch
 
 GAMMA = 0x9E3779B97F4A7C15
@@ -56,15 +58,30 @@ def distinct_keys(seed, n, distinct_bits, device="cpu"):
         extra *= 2
 
 
+def zipf_cdf(n_ids, s, device="cpu"):
+    """The CDF of Zipf(s) over ids 1..n_ids (float64), the same bits in every
+    call and on every device: a floating-point scan adds in an order that
+    depends on the device, and on a GPU on timing, and a last bit of the CDF
+    moves draws to a neighbouring id.  So the weights are formed on the CPU and
+    summed as integers, in two parts of 52 and 62 bits with their carries."""
+    w = torch.arange(1, n_ids + 1, dtype=torch.float64).pow(-s)
+    top = math.frexp(max(float(w[0]), float(w[-1])))[1]
+    n_bits = n_ids.bit_length()
+    w = w.to(device) * 2.0 ** (52 - n_bits - top)
+    whole = w.floor()
+    low = ((w - whole) * 2.0 ** (62 - n_bits)).round()
+    cdf = torch.cumsum(whole.to(torch.int64), 0).to(torch.float64)
+    cdf += torch.cumsum(low.to(torch.int64), 0).to(torch.float64) * 2.0 ** (n_bits - 62)
+    return cdf / cdf[-1].clone()
+
+
 def zipf_workload(n_ids, n_draws, s=1.5, seed=4, distinct_bits=36, device="cpu", chunk=1 << 24):
     """(keys[n_ids], draws[n_draws], multiplicity[n_ids]).
 
     Uniforms are u = (splitmix64(seed) output (2^40 + i) >> 11 + 0.5) / 2^53;
     the draw is the smallest id whose normalised CDF is >= u."""
     keys = distinct_keys(seed, n_ids, distinct_bits, device=device)
-    w = torch.arange(1, n_ids + 1, dtype=torch.float64, device=device).pow(-s)
-    cdf = torch.cumsum(w, 0)
-    cdf /= cdf[-1].clone()
+    cdf = zipf_cdf(n_ids, s, device)
     draws = torch.empty(n_draws, dtype=torch.int64, device=device)
     mult = torch.zeros(n_ids, dtype=torch.int64, device=device)
     for b in range(0, n_draws, chunk):
