@@ -490,18 +490,21 @@ constexpr uint32_t kBRound = kBThreads * kBItems;    // 8192
 constexpr uint32_t kBucketCap = 17408;               // 2^24 keys in 1024 buckets: mean 16384, sd 128
 constexpr int kBMaxPasses = 7;
 
-struct BucketSmem {
-  uint32_t buf[2][kBucketCap];
+struct PassSmem {
   uint32_t wcnt[kBWaves][256];        // per wave digit counts, then positions
-  uint32_t tot[kBMaxPasses][256];     // digit totals of every pass
   uint32_t run[256];                  // next free position of each digit
+};
+struct BucketSmem {
+  alignas(16) uint32_t buf[2][kBucketCap];
+  uint32_t tot[kBMaxPasses][256];     // digit totals of every pass
+  PassSmem pass;
 };
 
 // Stable scatter of src[0, m) into dst by digit (v >> sh) & 255, given the
 // digit totals; every thread of the workgroup calls it.
 template <typename V>
 __device__ __forceinline__ void bucket_pass(const V* src, V* dst, uint32_t m, int sh, const uint32_t* tot,
-                                            BucketSmem& sm) {
+                                            PassSmem& sm) {
   const int t = threadIdx.x, w = t >> 6, lane = t & 63;
   if (w == 0) {  // exclusive scan of the totals, 4 digits per lane
     uint32_t v[4], sum = 0;
@@ -559,6 +562,42 @@ __device__ __forceinline__ void bucket_pass(const V* src, V* dst, uint32_t m, in
       if (i < m) dst[sm.wcnt[w][(uint32_t)(keys[k] >> sh) & 255u] + rank[k]] = keys[k];
     }
   }
+}
+
+// Sorts the m values of a by their low 8 * passes bits, between the LDS
+// buffers a and b, and returns the one that holds the result; tot: `passes`
+// rows of digit totals.  A digit that all values share takes no pass (few
+// distinct keys, and of the request tags few bits, is what it is called for).
+// Every thread of the workgroup calls it, with a complete (a barrier passed).
+// Latency bound: buckets of 2,400 sequenced keys on 100 hashes 37 us, where a
+// table of their distinct (hash, request) pairs took 285.
+template <typename V>
+__device__ __forceinline__ V* lds_sort(V* a, V* b, uint32_t m, int passes, uint32_t (*tot)[256], PassSmem& sm) {
+  for (int k = threadIdx.x; k < passes * 256; k += kBThreads) (&tot[0][0])[k] = 0;
+  __syncthreads();
+  const uint32_t lane = threadIdx.x & 63;
+  for (uint32_t i0 = 0; i0 < m; i0 += kBThreads) {
+    const uint32_t i = i0 + threadIdx.x;
+    const V v = a[min(i, m - 1)];
+    for (int p = 0; p < passes; p++) {
+      // the wave's first digit once for all lanes that have it
+      const uint32_t d = (uint32_t)(v >> (8 * p)) & 255u;
+      const uint64_t same = __ballot(i < m && d == (uint32_t)__builtin_amdgcn_readfirstlane((int)d));
+      if (i < m && (lane == 0 || !((same >> lane) & 1)))
+        atomicAdd(&tot[p][d], lane == 0 ? (uint32_t)__popcll(same) : 1u);
+    }
+  }
+  __syncthreads();
+  const V any = a[0];
+  for (int p = 0; p < passes; p++) {
+    if (tot[p][(uint32_t)(any >> (8 * p)) & 255u] == m) continue;  // uniform
+    bucket_pass<V>(a, b, m, 8 * p, tot[p], sm);
+    __syncthreads();
+    V* t = a;
+    a = b;
+    b = t;
+  }
+  return a;
 }
 
 }  // namespace
@@ -733,15 +772,24 @@ gqf_sort_buckets_tagged(const uint64_t* __restrict__ in, uint64_t* __restrict__ 
 
 // A bucket that repeats few keys (at most kTableMax distinct ones, however
 // many times each): its distinct values are counted in an LDS hash table, the
-// table is sorted, and every value is written as often as it came.  Returns
-// false, with nothing written, if there are more.
+// table's entries are packed and sorted, and every value is written as often as
+// it came.  Returns false, with nothing written, if there are more.
+// Latency bound (a workgroup by itself): eight keys a thread are in flight, the
+// network sorts no more than the distinct values need, and values with many
+// copies are listed as they are met: buckets of 17,400 keys, 2,000 of them
+// distinct, 114 us; with one key in flight, a network over the whole table and a
+// second look at every value for the many copies 314 us, and the passes between
+// global buffers 100 us at 17,400 keys but longer with every repeat.
 constexpr uint32_t kTableCap = 8192;
 constexpr uint32_t kTableMax = 6144;
+constexpr uint32_t kTableMany = 4096;  // copies that the whole workgroup writes
+constexpr uint32_t kManyList = 64;
 struct BucketTable {
   uint64_t val[kTableCap];  // ~0: free
   uint32_t cnt[kTableCap];  // then the values' first output indexes
   uint32_t wsum[kBWaves];
-  uint32_t used;
+  uint32_t many[kManyList];
+  uint32_t used, n_many;
 };
 static_assert(sizeof(BucketTable) <= sizeof(BucketSmem), "shares the passes' LDS");
 
@@ -756,13 +804,9 @@ __device__ __forceinline__ bool sort_by_table(const uint64_t* in, uint64_t* out,
     tb.val[i] = ~0ULL;
     tb.cnt[i] = 0;
   }
-  if (t == 0) tb.used = 0;
+  if (t == 0) tb.used = tb.n_many = 0;
   __syncthreads();
-  for (uint32_t i0 = 0; i0 < m; i0 += kBThreads) {
-    if (*(volatile uint32_t*)&tb.used > kTableMax) break;  // checked again below
-    const uint32_t i = i0 + t;
-    bool left = i < m;
-    const uint64_t v = left ? (uint64_t)K::of(in[s + i], hi) : 0ULL;
+  auto count = [&](uint64_t v, bool left) {
     // a wave's repeats of one value are added together (two values' worth,
     // the rest one by one)
     uint32_t add = left ? 1u : 0u;
@@ -789,14 +833,54 @@ __device__ __forceinline__ bool sort_by_table(const uint64_t* in, uint64_t* out,
         at = (at + 1) & (kTableCap - 1);
       }
     }
+  };
+  for (uint32_t i0 = 0; i0 < m; i0 += kBThreads * kBItems) {
+    if (*(volatile uint32_t*)&tb.used > kTableMax) break;  // checked again below
+    uint64_t v[kBItems];
+#pragma unroll
+    for (int k = 0; k < kBItems; k++) v[k] = in[s + min(i0 + (uint32_t)k * kBThreads + t, m - 1)];
+#pragma unroll
+    for (int k = 0; k < kBItems; k++)
+      if (i0 + (uint32_t)k * kBThreads < m) count((uint64_t)K::of(v[k], hi), i0 + (uint32_t)k * kBThreads + t < m);
   }
   __syncthreads();
   if (tb.used > kTableMax) return false;
-  // bitonic, the free entries (~0) last
-  for (uint32_t k = 2; k <= kTableCap; k *= 2) {
+  // the entries to the front, then a bitonic network over them (~0 behind them)
+  const uint32_t used = tb.used;
+  constexpr int kE = kTableCap / kBThreads;  // entries of a thread
+  {
+    uint64_t val[kE];
+    uint32_t cnt[kE], mine = 0;
+#pragma unroll
+    for (int k = 0; k < kE; k++) {
+      val[k] = tb.val[k * kBThreads + t];
+      cnt[k] = tb.cnt[k * kBThreads + t];
+      mine += val[k] != ~0ULL ? 1u : 0u;
+    }
+    const uint32_t incl = wave_scan_add(mine);
+    if (lane == 63) tb.wsum[w] = incl;
+    __syncthreads();  // every entry is read
+    uint32_t at = incl - mine;
+    for (uint32_t k = 0; k < w; k++) at += tb.wsum[k];
+#pragma unroll
+    for (int k = 0; k < kE; k++) {
+      if (val[k] == ~0ULL) continue;
+      tb.val[at] = val[k];
+      tb.cnt[at] = cnt[k];
+      at++;
+    }
+  }
+  uint32_t size = 2;
+  while (size < used) size *= 2;
+  for (uint32_t i = used + t; i < size; i += kBThreads) {
+    tb.val[i] = ~0ULL;
+    tb.cnt[i] = 0;
+  }
+  __syncthreads();
+  for (uint32_t k = 2; k <= size; k *= 2) {
     for (uint32_t j = k / 2; j > 0; j /= 2) {
-      for (uint32_t i = t; i < kTableCap / 2; i += kBThreads) {
-        const uint32_t a = (i / j) * 2 * j + i % j, c = a + j;
+      for (uint32_t i = t; i < size / 2; i += kBThreads) {
+        const uint32_t a = 2 * i - (i & (j - 1)), c = a + j;  // the i-th pair at distance j
         const uint64_t x = tb.val[a], y = tb.val[c];
         if ((x > y) == ((a & k) == 0)) {
           tb.val[a] = y;
@@ -810,11 +894,11 @@ __device__ __forceinline__ bool sort_by_table(const uint64_t* in, uint64_t* out,
     }
   }
   // counts -> first indexes, eight entries a thread
-  constexpr int kE = kTableCap / kBThreads;
   uint32_t c[kE], sum = 0;
 #pragma unroll
   for (int k = 0; k < kE; k++) {
-    c[k] = tb.cnt[kE * t + (uint32_t)k];
+    const uint32_t e = kE * t + (uint32_t)k;
+    c[k] = e < used ? tb.cnt[e] : 0u;
     sum += c[k];
   }
   const uint32_t incl = wave_scan_add(sum);
@@ -824,23 +908,30 @@ __device__ __forceinline__ bool sort_by_table(const uint64_t* in, uint64_t* out,
   for (uint32_t k = 0; k < w; k++) run += tb.wsum[k];
 #pragma unroll
   for (int k = 0; k < kE; k++) {
-    tb.cnt[kE * t + (uint32_t)k] = run;
+    if (kE * t + (uint32_t)k < used) tb.cnt[kE * t + (uint32_t)k] = run;
     run += c[k];
   }
   __syncthreads();
-  const uint32_t used = tb.used;
   auto begin = [&](uint32_t e) { return e < used ? tb.cnt[e] : m; };
-  // a value's copies: a wave each, or, for many, the workgroup
-  constexpr uint32_t kMany = 4096;
+  // a value's copies: a wave each, or, for many, the workgroup (a listed value;
+  // more than the list holds stay with their waves)
   for (uint32_t e = w; e < used; e += kBWaves) {
     const uint32_t a = begin(e), z = begin(e + 1);
-    if (z - a >= kMany) continue;
+    if (z - a >= kTableMany) {
+      uint32_t k = 0;
+      if (lane == 0) k = atomicAdd(&tb.n_many, 1u);
+      k = (uint32_t)__builtin_amdgcn_readfirstlane((int)k);
+      if (k < kManyList) {
+        if (lane == 0) tb.many[k] = e;
+        continue;
+      }
+    }
     const uint64_t key = tag | K::key((typename K::V)tb.val[e], hi);
     for (uint32_t i = a + lane; i < z; i += 64) out[s + i] = key;
   }
-  for (uint32_t e = 0; e < used; e++) {
-    const uint32_t a = begin(e), z = begin(e + 1);
-    if (z - a < kMany) continue;
+  __syncthreads();
+  for (uint32_t k = 0; k < min(tb.n_many, kManyList); k++) {
+    const uint32_t e = tb.many[k], a = begin(e), z = begin(e + 1);
     const uint64_t key = tag | K::key((typename K::V)tb.val[e], hi);
     for (uint32_t i = a + t; i < z; i += kBThreads) out[s + i] = key;
   }
@@ -869,42 +960,31 @@ __device__ __forceinline__ void sort_flagged_bucket(uint64_t* in, uint64_t* out,
   const int passes = (low_bits + K::kExtra + 7) / 8;
   __syncthreads();  // every thread has read the flag
   if (t == 0) slow[b] = 0;
-  if ((kTagged || m > kBucketCap) &&
-      sort_by_table<kTagged>(in, out, s, n, m, low_bits, b, nbuckets, *(BucketTable*)&sm, ra, tag))
-    return;
-  __syncthreads();
-  for (int k = t; k < kBMaxPasses * 256; k += kBThreads) (&sm.tot[0][0])[k] = 0;
-  __syncthreads();
-  if (!kTagged && m <= kBucketCap) {
-    for (uint32_t i = t; i < m; i += kBThreads) {
-      const uint32_t v = (uint32_t)(in[s + i] - hi);
-      sm.buf[0][i] = v;
-      for (int p = 0; p < passes; p++) atomicAdd(&sm.tot[p][(v >> (8 * p)) & 255u], 1u);
-    }
+  if (m <= K::kCap) {
+    using V = typename K::V;
+    V* const first = (V*)sm.buf[0];
+    for (uint32_t i = t; i < m; i += kBThreads) first[i] = K::of(in[s + i], hi);
     __syncthreads();
-    int src = 0;
-    for (int p = 0; p < passes; p++) {
-      bucket_pass<uint32_t>(sm.buf[src], sm.buf[src ^ 1], m, 8 * p, sm.tot[p], sm);
-      __syncthreads();
-      src ^= 1;
-    }
-    for (uint32_t i = t; i < m; i += kBThreads) out[s + i] = tag | hi | sm.buf[src][i];
-    const uint32_t* sorted = sm.buf[src];
+    const V* sorted = lds_sort<V>(first, (V*)sm.buf[1], m, passes, sm.tot, sm.pass);
+    for (uint32_t i = t; i < m; i += kBThreads) out[s + i] = tag | K::key(sorted[i], hi);
     bucket_region_starts(ra, b, nbuckets, low_bits, s, n, [&](uint32_t x) {
       uint32_t lo = 0, hi2 = m;
       while (lo < hi2) {
         const uint32_t mid = (lo + hi2) >> 1;
-        if (sorted[mid] < x) lo = mid + 1; else hi2 = mid;
+        if (sorted[mid] < K::bound(x)) lo = mid + 1; else hi2 = mid;
       }
       return lo;
     });
     return;
   }
-  // too large for LDS, or tagged: the same passes, over the keys as they are
-  // ordered, between the bucket's ranges of in and out, plus a pass on a zero
-  // digit when the count is even, so the result lands in out; other waves'
-  // stores are published between passes with agent-scope fences around the
-  // barrier
+  if (sort_by_table<kTagged>(in, out, s, n, m, low_bits, b, nbuckets, *(BucketTable*)&sm, ra, tag)) return;
+  __syncthreads();
+  for (int k = t; k < kBMaxPasses * 256; k += kBThreads) (&sm.tot[0][0])[k] = 0;
+  __syncthreads();
+  // too large for LDS: the same passes, over the keys as they are ordered,
+  // between the bucket's ranges of in and out, plus a pass on a zero digit when
+  // the count is even, so the result lands in out; other waves' stores are
+  // published between passes with agent-scope fences around the barrier
   const int gpasses = passes | 1;
   uint64_t* a = in + s;
   uint64_t* o = out + s;
@@ -917,7 +997,7 @@ __device__ __forceinline__ void sort_flagged_bucket(uint64_t* in, uint64_t* out,
   __syncthreads();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   for (int p = 0; p < gpasses; p++) {
-    bucket_pass<uint64_t>(p & 1 ? o : a, p & 1 ? a : o, m, 8 * p, sm.tot[p], sm);
+    bucket_pass<uint64_t>(p & 1 ? o : a, p & 1 ? a : o, m, 8 * p, sm.tot[p], sm.pass);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
     __syncthreads();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
@@ -936,10 +1016,10 @@ __device__ __forceinline__ void sort_flagged_bucket(uint64_t* in, uint64_t* out,
 
 // The flagged buckets (skips the others, and clears the flags it takes):
 // stable 8-bit passes over the bucket's low bits in two LDS buffers, or, for
-// a bucket above kBucketCap, the same passes over its 64-bit keys between
-// its ranges of in and out in global memory.  A grid of at most one
-// workgroup per CU strides over the buckets, so an all-clear call costs
-// one short launch.
+// a bucket that they have no room for, its distinct keys by a table, or, for
+// more of those, the passes over its 64-bit keys between its ranges of in and
+// out in global memory.  A grid of at most one workgroup per CU strides over
+// the buckets, so an all-clear call costs one short launch.
 extern "C" __global__ void __launch_bounds__(kBThreads)
 gqf_sort_buckets_slow(uint64_t* in, uint64_t* out, uint64_t n, int low_bits, const uint32_t* __restrict__ starts,
                       uint32_t nbuckets, uint32_t* __restrict__ slow, gqf_region_args ra, uint64_t tag) {
@@ -965,8 +1045,8 @@ gqf_sort_buckets_slow_tagged(uint64_t* in, uint64_t* out, uint64_t n, int low_bi
 // instead of a dozen.  As the bucket sort: the keys are counted by their top
 // (up to) 12 bits, put into sub-bucket order in LDS, and each one's place is
 // its rank among the keys of its sub-bucket (two on average at 8192 uniform
-// keys).  A sub-bucket above kSubCap keys (repeats) makes the workgroup run a
-// bitonic network over all of them instead.  Latency bound: 12 us for 5000
+// keys).  A sub-bucket above kSubCap keys (repeats) makes the workgroup sort all
+// of them by digits instead (lds_sort).  Latency bound: 12 us for 5000
 // keys, against 63 us for the four passes (12 launches) of the LSD sort plus 9
 // for the region bounds.
 
@@ -976,7 +1056,9 @@ constexpr uint32_t kTinyCap = GQF_SORT_TINY;
 constexpr int kTLoad = kTinyCap / kTThreads;
 constexpr int kTSubBits = 12;
 constexpr uint32_t kTSub = 1u << kTSubBits;
+constexpr int kTPasses = (42 + 16 + 7) / 8;  // of the widest tagged keys (gqf_sort_fast_fits)
 static_assert(kTSub == 4 * kTThreads, "four sub-buckets per thread in the scan");
+static_assert(kTThreads == kBThreads, "lds_sort's workgroup");
 }  // namespace
 
 template <bool kTagged>
@@ -984,8 +1066,13 @@ __device__ __forceinline__ void sort_tiny(uint64_t* __restrict__ keys, uint32_t 
                                           const gqf_list_args& la) {
   __shared__ uint64_t buf[kTinyCap];
   __shared__ uint64_t sorted[kTinyCap];
-  __shared__ uint32_t sub_end[kTSub];
+  __shared__ union {
+    uint32_t sub_end[kTSub];
+    PassSmem pass;  // the digit passes come after the sub-buckets
+  } u;
+  __shared__ uint32_t tot[kTPasses][256];
   __shared__ uint32_t wsum[kTThreads / 64];
+  uint32_t* const sub_end = u.sub_end;
   __shared__ uint32_t oversize, nlist[2];
   const uint32_t t = threadIdx.x, w = t >> 6, lane = t & 63;
   // tagged keys as seq_order has them: hash bits above 16 tag bits
@@ -1029,27 +1116,10 @@ __device__ __forceinline__ void sort_tiny(uint64_t* __restrict__ keys, uint32_t 
   for (int k = 0; k < kTLoad; k++)
     if ((uint32_t)k * kTThreads + t < n) buf[atomicAdd(&sub_end[(uint32_t)(v[k] >> sb)], 1u)] = v[k];
   const uint64_t* res = sorted;
+  __syncthreads();
   if (oversize) {
-    uint32_t p = 2;
-    while (p < n) p *= 2;
-    for (uint32_t i = n + t; i < p; i += kTThreads) buf[i] = ~0ULL;
-    __syncthreads();
-    for (uint32_t k = 2; k <= p; k *= 2) {
-      for (uint32_t j = k / 2; j > 0; j /= 2) {
-        for (uint32_t i = t; i < p / 2; i += kTThreads) {
-          const uint32_t a = (i / j) * 2 * j + i % j, b = a + j;  // the i-th pair at distance j
-          const uint64_t x = buf[a], y = buf[b];
-          if ((x > y) == ((a & k) == 0)) {
-            buf[a] = y;
-            buf[b] = x;
-          }
-        }
-        __syncthreads();
-      }
-    }
-    res = buf;
+    res = lds_sort<uint64_t>(buf, sorted, n, (all + 7) / 8, tot, u.pass);
   } else {
-    __syncthreads();
     for (uint32_t i = t; i < n; i += kTThreads) {
       const uint64_t x = buf[i];
       const uint32_t d = (uint32_t)(x >> sb);
