@@ -564,6 +564,22 @@ __device__ __forceinline__ void bucket_pass(const V* src, V* dst, uint32_t m, in
   }
 }
 
+// A bitonic network of `size` (a power of two) places: order(a, c, up) puts
+// places a < c into ascending order if up, else descending.  Every thread of the
+// workgroup calls it.
+template <typename F>
+__device__ __forceinline__ void lds_network(uint32_t size, F order) {
+  for (uint32_t k = 2; k <= size; k *= 2) {
+    for (uint32_t j = k / 2; j > 0; j /= 2) {
+      for (uint32_t i = threadIdx.x; i < size / 2; i += kBThreads) {
+        const uint32_t a = 2 * i - (i & (j - 1));  // the i-th pair at distance j
+        order(a, a + j, (a & k) == 0);
+      }
+      __syncthreads();
+    }
+  }
+}
+
 // Sorts the m values of a by their low 8 * passes bits, between the LDS
 // buffers a and b, and returns the one that holds the result; tot: `passes`
 // rows of digit totals.  A digit that all values share takes no pass (few
@@ -877,22 +893,16 @@ __device__ __forceinline__ bool sort_by_table(const uint64_t* in, uint64_t* out,
     tb.cnt[i] = 0;
   }
   __syncthreads();
-  for (uint32_t k = 2; k <= size; k *= 2) {
-    for (uint32_t j = k / 2; j > 0; j /= 2) {
-      for (uint32_t i = t; i < size / 2; i += kBThreads) {
-        const uint32_t a = 2 * i - (i & (j - 1)), c = a + j;  // the i-th pair at distance j
-        const uint64_t x = tb.val[a], y = tb.val[c];
-        if ((x > y) == ((a & k) == 0)) {
-          tb.val[a] = y;
-          tb.val[c] = x;
-          const uint32_t z = tb.cnt[a];
-          tb.cnt[a] = tb.cnt[c];
-          tb.cnt[c] = z;
-        }
-      }
-      __syncthreads();
+  lds_network(size, [&](uint32_t a, uint32_t c, bool up) {
+    const uint64_t x = tb.val[a], y = tb.val[c];
+    if ((x > y) == up) {
+      tb.val[a] = y;
+      tb.val[c] = x;
+      const uint32_t z = tb.cnt[a];
+      tb.cnt[a] = tb.cnt[c];
+      tb.cnt[c] = z;
     }
-  }
+  });
   // counts -> first indexes, eight entries a thread
   uint32_t c[kE], sum = 0;
 #pragma unroll
@@ -1046,7 +1056,9 @@ gqf_sort_buckets_slow_tagged(uint64_t* in, uint64_t* out, uint64_t n, int low_bi
 // (up to) 12 bits, put into sub-bucket order in LDS, and each one's place is
 // its rank among the keys of its sub-bucket (two on average at 8192 uniform
 // keys).  A sub-bucket above kSubCap keys (repeats) makes the workgroup sort all
-// of them by digits instead (lds_sort).  Latency bound: 12 us for 5000
+// of them by digits instead (lds_sort), or, up to kTNetwork keys, by a bitonic
+// network: repeats of a few of 300 / 1,000 / 2,000 keys, a whole delete, 30 / 37 /
+// 47 us by the network and 43 / 48 / 53 by digits; 8,192 go the other way.  Latency bound: 12 us for 5000
 // keys, against 63 us for the four passes (12 launches) of the LSD sort plus 9
 // for the region bounds.
 
@@ -1056,6 +1068,7 @@ constexpr uint32_t kTinyCap = GQF_SORT_TINY;
 constexpr int kTLoad = kTinyCap / kTThreads;
 constexpr int kTSubBits = 12;
 constexpr uint32_t kTSub = 1u << kTSubBits;
+constexpr uint32_t kTNetwork = 2048;
 constexpr int kTPasses = (42 + 16 + 7) / 8;  // of the widest tagged keys (gqf_sort_fast_fits)
 static_assert(kTSub == 4 * kTThreads, "four sub-buckets per thread in the scan");
 static_assert(kTThreads == kBThreads, "lds_sort's workgroup");
@@ -1118,7 +1131,22 @@ __device__ __forceinline__ void sort_tiny(uint64_t* __restrict__ keys, uint32_t 
   const uint64_t* res = sorted;
   __syncthreads();
   if (oversize) {
-    res = lds_sort<uint64_t>(buf, sorted, n, (all + 7) / 8, tot, u.pass);
+    if (n <= kTNetwork) {
+      uint32_t size = 2;
+      while (size < n) size *= 2;
+      for (uint32_t i = n + t; i < size; i += kTThreads) buf[i] = ~0ULL;
+      __syncthreads();
+      lds_network(size, [&](uint32_t a, uint32_t c, bool up) {
+        const uint64_t x = buf[a], y = buf[c];
+        if ((x > y) == up) {
+          buf[a] = y;
+          buf[c] = x;
+        }
+      });
+      res = buf;
+    } else {
+      res = lds_sort<uint64_t>(buf, sorted, n, (all + 7) / 8, tot, u.pass);
+    }
   } else {
     for (uint32_t i = t; i < n; i += kTThreads) {
       const uint64_t x = buf[i];
