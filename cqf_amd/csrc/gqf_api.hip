@@ -51,7 +51,7 @@ struct Workspace {
   uint64_t* m_dev = nullptr;
   uint32_t* region_start = nullptr;  // nregions + 1
   uint32_t* region_list = nullptr;   // non-empty regions of each parity
-  uint32_t* list_count = nullptr;    // 2 counts
+  uint32_t* list_count = nullptr;    // GQF_LIST_WORDS: 2 counts, the form of the rebuild
   uint8_t* wide_flags = nullptr;     // nregions, kept zero by the kernels
   uint32_t* wide_count = nullptr;    // GQF_WIDE_WORDS: count, flagged regions, finished workgroups
   unsigned long long* misses = nullptr;
@@ -166,7 +166,7 @@ void init_region_workspace(Workspace& w, uint64_t nblocks) {
     const uint64_t maxreg = (nblocks + GQF_REGION_BLOCKS_MIN - 1) / GQF_REGION_BLOCKS_MIN;
     dev_alloc(&w.region_start, maxreg + 2);
     dev_alloc(&w.region_list, 2 * ((maxreg + 1) / 2 + 1));
-    dev_alloc(&w.list_count, 2);
+    dev_alloc(&w.list_count, GQF_LIST_WORDS);
     dev_alloc(&w.wide_flags, maxreg + 1);
     GQF_CHECK(hipMemset(w.wide_flags, 0, maxreg + 1));
     dev_alloc(&w.wide_count, GQF_WIDE_WORDS);
@@ -313,7 +313,10 @@ void run_mutation(Filter* f, Workspace& w, uint64_t n, uint64_t* keys, uint8_t f
   // would put many of them into one bucket: it keeps the LSD sort)
   const bool fast = hash_it && gqf_sort_fast_fits(n, bits, false) &&
                     !(reduce && n > GQF_SORT_TINY && n < (1ULL << 20));
-  const bool listed = n < f->host.nregions || n <= GQF_SORT_TINY;
+  // (a reduce batch of any size may have keys in a few regions only, and
+  // workgroups that find theirs empty leave the others badly spread: 33,000 keys
+  // with items in half of 5,463 regions, 46 us a phase unlisted and 37 listed)
+  const bool listed = reduce || n < f->host.nregions || n <= GQF_SORT_TINY;
   const gqf_region_args ra = all_regions(f, w);
   const gqf_list_args la = listed_regions(f, w);
   if (fast)
@@ -346,7 +349,7 @@ void run_mutation(Filter* f, Workspace& w, uint64_t n, uint64_t* keys, uint8_t f
   if (!fast || reduce)
     gqf_launch_region_bounds(f->dev, f->host.nregions, items, n, n_dev, w.region_start, list, w.list_count, ~0ULL, s);
   gqf_launch_rebuild(f->dev, f->host.nregions, f->host.region_blocks, items, counts, n, w.region_start, list,
-                     w.list_count, mode, w.wide_flags, w.wide_count, s);
+                     w.list_count, mode, w.wide_flags, w.wide_count, s, n_dev);
   GQF_CHECK(hipGetLastError());
 }
 
@@ -635,7 +638,7 @@ constexpr uint64_t kNaTotals = na_round(GQF_SORT_TOTALS * 4);
 constexpr uint64_t kNaSlow = na_round(GQF_SORT_MAX_BUCKETS * 4);
 constexpr uint64_t kNaStart = na_round((kNoAllocMaxRegions + 2) * 4);
 constexpr uint64_t kNaList = na_round(2 * ((kNoAllocMaxRegions + 1) / 2 + 1) * 4);
-constexpr uint64_t kNaCount = na_round(2 * 4);
+constexpr uint64_t kNaCount = na_round(GQF_LIST_WORDS * 4);
 constexpr uint64_t kNaWideFlags = na_round(kNoAllocMaxRegions + 1);
 constexpr uint64_t kNaWideCount = na_round(GQF_WIDE_WORDS * 4);
 constexpr uint64_t kNoAllocBytes =
@@ -1125,8 +1128,10 @@ int64_t move_items(Filter* f, const QF* dst_dev, const QF& dst, Workspace& dst_w
                            (int)dst.value_bits, gqf_mask(src.key_bits), items, counts, nullptr, cap, s);
       gqf_launch_region_bounds(dst_dev, dst.nregions, items, n, nullptr, dst_ws.region_start, dst_ws.region_list,
                                dst_ws.list_count, ~0ULL, s);
+      // a chunk's items lie in its groups' share of the table
+      const uint64_t reach = (uint64_t)((double)dst.nregions * (double)(v - u) / (double)groups) + 1;
       gqf_launch_rebuild(dst_dev, dst.nregions, dst.region_blocks, items, counts, n, dst_ws.region_start, dst_ws.region_list,
-                         dst_ws.list_count, kModeInsert, dst_ws.wide_flags, dst_ws.wide_count, s);
+                         dst_ws.list_count, kModeInsert, dst_ws.wide_flags, dst_ws.wide_count, s, nullptr, reach);
     }
     u = v;
   }

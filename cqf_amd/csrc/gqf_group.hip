@@ -293,7 +293,7 @@ void enqueue_insert(Group* g, const gqf_group_dev& dev, uint64_t* keys, uint64_t
   }
   hipLaunchKernelGGL(gqf_group_reset, dim3(1), dim3(64), 0, s, g->d_counters);
   const uint64_t n_even = g->h_tab[2 * (size_t)(g->nf + 1) - 1], n_odd = g->h_tab[3 * (size_t)(g->nf + 1) - 1];
-  const bool dense = gqf_rebuild_is_dense(n, n_even + n_odd);
+  const bool dense = gqf_group_is_dense(n, n_even + n_odd);
   gqf_launch_group_rebuild(dev, keys, mode, gqf_group_rebuild_grid(g->per_cu), n_even, n_odd, dense, s);
   hipLaunchKernelGGL(gqf_group_untag, dim3(flat_grid(n)), dim3(256), 0, s, keys, n, dev.tag_shift);
 }

@@ -124,6 +124,10 @@ void gqf_launch_seq_adjust(const QF* qf_dev, const uint64_t* keys, uint64_t n, c
 // both even/odd phases (+ wide fallback passes) of a merge-rebuild over
 // the listed regions (n_items bounds their number), or over all of them
 // where region_list is null (every entry of region_start is set).
+// n_dev, if set, points at the number of items, of which n_items is a bound
+// then; reach: regions that the items can be in (0: all).
+// list_count: GQF_LIST_WORDS words (the lists' counts, then which form of the
+// rebuild takes the batch, where that is found on the device).
 // wide_flags: one byte per region; wide_count: GQF_WIDE_WORDS words (the
 // number of regions flagged in a phase, the first GQF_WIDE_LIST of them, a
 // counter of finished wide workgroups, a ticket counter and one finished
@@ -131,13 +135,14 @@ void gqf_launch_seq_adjust(const QF* qf_dev, const uint64_t* keys, uint64_t n, c
 // leave them so)
 // the class waits' poll bound (qf_set_wide_wait_bound); returns the previous one
 uint32_t gqf_wide_wait_bound_set(uint32_t max_polls);
+#define GQF_LIST_WORDS 3
 #define GQF_WIDE_LIST 64
 #define GQF_WIDE_MAX_CLASSES 8  // classes of the wide pass: ceil(ceil(256 / R) / 2), R >= 16
 #define GQF_WIDE_WORDS (3 + GQF_WIDE_LIST + GQF_WIDE_MAX_CLASSES)
 void gqf_launch_rebuild(const QF* qf_dev, uint64_t nregions, uint64_t region_blocks, const uint64_t* items,
                         const uint64_t* counts, uint64_t n_items, const uint32_t* region_start,
-                        const uint32_t* region_list, const uint32_t* list_count, int mode, uint8_t* wide_flags,
-                        uint32_t* wide_count, hipStream_t s);
+                        const uint32_t* region_list, uint32_t* list_count, int mode, uint8_t* wide_flags,
+                        uint32_t* wide_count, hipStream_t s, const uint64_t* n_dev = nullptr, uint64_t reach = 0);
 
 void gqf_launch_bulk_get(const QF* qf_dev, const uint64_t* vals, uint64_t n, uint64_t* returns, hipStream_t s);
 void gqf_launch_misses(const QF* qf_dev, const uint64_t* vals, uint64_t n, unsigned long long* misses,
@@ -224,8 +229,8 @@ struct gqf_group_dev {
 };
 #define GQF_GROUP_MAX_POLLS (1u << 22)  // default bound: about 1 s of polls, far above any region's rebuild
 
-// whether a batch of inserts is dense enough for the workgroup-wide rebuild
-bool gqf_rebuild_is_dense(uint64_t n_items, uint64_t nregions);
+// whether a group's batch is dense enough for the workgroup-wide rebuild
+bool gqf_group_is_dense(uint64_t n_items, uint64_t nregions);
 // the rebuild over every filter's regions, then the wide redo tail: dense
 // batches one workgroup per region, even regions then odd ones (n_even /
 // n_odd of them); others the persistent launch of `grid` workgroups (even

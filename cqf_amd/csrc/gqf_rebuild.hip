@@ -31,6 +31,7 @@
 // window, in ascending region order, after the phase.
 #include <stdlib.h>
 
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 #include <utility>
@@ -1905,9 +1906,11 @@ __device__ __forceinline__ void rebuild_phase_item(const QF* __restrict__ qfp, c
                                                    const uint64_t* __restrict__ counts,
                                                    const uint32_t* __restrict__ region_start,
                                                    const uint32_t* __restrict__ region_list,
-                                                   const uint32_t* __restrict__ list_count, int parity, int mode,
+                                                   const uint32_t* __restrict__ list_count,
+                                                   const uint32_t* __restrict__ dense, int parity, int mode,
                                                    uint8_t* __restrict__ wide_flags, uint32_t* __restrict__ wide_count,
                                                    Smem<kWinFast>& sm, uint32_t* lcnt) {
+  if (dense && *dense) return;  // gqf_rebuild_flat takes the batch
   const QF qf = *qfp;
   if (region_list && blockIdx.x >= list_count[parity]) return;
   const uint64_t r = region_list ? region_list[blockIdx.x] : 2 * (uint64_t)blockIdx.x + (uint64_t)parity;
@@ -1927,22 +1930,23 @@ __device__ __forceinline__ void rebuild_phase_item(const QF* __restrict__ qfp, c
 extern "C" __global__ void __launch_bounds__(64)
 gqf_rebuild_phase(const QF* __restrict__ qfp, const uint64_t* __restrict__ items,
                   const uint32_t* __restrict__ region_start, const uint32_t* __restrict__ region_list,
-                  const uint32_t* __restrict__ list_count, int parity, int mode, uint8_t* __restrict__ wide_flags,
-                  uint32_t* __restrict__ wide_count) {
+                  const uint32_t* __restrict__ list_count, const uint32_t* __restrict__ dense, int parity, int mode,
+                  uint8_t* __restrict__ wide_flags, uint32_t* __restrict__ wide_count) {
   __shared__ Smem<kWinFast> sm;
-  rebuild_phase_item(qfp, items, nullptr, region_start, region_list, list_count, parity, mode, wide_flags, wide_count,
-                     sm, nullptr);
+  rebuild_phase_item(qfp, items, nullptr, region_start, region_list, list_count, dense, parity, mode, wide_flags,
+                     wide_count, sm, nullptr);
 }
 
 extern "C" __global__ void __launch_bounds__(64)
 gqf_rebuild_phase_counts(const QF* __restrict__ qfp, const uint64_t* __restrict__ items,
                          const uint64_t* __restrict__ counts, const uint32_t* __restrict__ region_start,
                          const uint32_t* __restrict__ region_list, const uint32_t* __restrict__ list_count,
-                         int parity, int mode, uint8_t* __restrict__ wide_flags, uint32_t* __restrict__ wide_count) {
+                         const uint32_t* __restrict__ dense, int parity, int mode, uint8_t* __restrict__ wide_flags,
+                         uint32_t* __restrict__ wide_count) {
   __shared__ Smem<kWinFast> sm;
   __shared__ uint32_t icnt[kItemCap];
-  rebuild_phase_item(qfp, items, counts, region_start, region_list, list_count, parity, mode, wide_flags, wide_count,
-                     sm, icnt);
+  rebuild_phase_item(qfp, items, counts, region_start, region_list, list_count, dense, parity, mode, wide_flags,
+                     wide_count, sm, icnt);
 }
 
 // One workgroup of gqf_flat::kThreads per non-empty region of one parity
@@ -1950,9 +1954,10 @@ gqf_rebuild_phase_counts(const QF* __restrict__ qfp, const uint64_t* __restrict_
 extern "C" __global__ void __launch_bounds__(gqf_flat::kThreads)
 gqf_rebuild_flat(const QF* __restrict__ qfp, const uint64_t* __restrict__ items, const uint64_t* __restrict__ counts,
                  const uint32_t* __restrict__ region_start, const uint32_t* __restrict__ region_list,
-                 const uint32_t* __restrict__ list_count, int parity, int kind, uint8_t* __restrict__ wide_flags,
-                 uint32_t* __restrict__ wide_count) {
+                 const uint32_t* __restrict__ list_count, const uint32_t* __restrict__ dense, int parity, int kind,
+                 uint8_t* __restrict__ wide_flags, uint32_t* __restrict__ wide_count) {
   __shared__ gqf_flat::Smem sm;
+  if (dense && !*dense) return;  // gqf_rebuild_phase or gqf_rebuild_phase_counts takes the batch
   const QF qf = *qfp;
   if (region_list && blockIdx.x >= list_count[parity]) return;
   const uint64_t r = region_list ? region_list[blockIdx.x] : 2 * (uint64_t)blockIdx.x + (uint64_t)parity;
@@ -2424,21 +2429,74 @@ std::atomic<uint32_t> g_wide_max_polls{kWideMaxPolls};
 
 uint32_t gqf_wide_wait_bound_set(uint32_t max_polls) { return g_wide_max_polls.exchange(max_polls); }
 
-// Batches of at least this many items per region on average take the
-// workgroup-wide rebuild (gqf_flat.h): inserts when regions outgrow the item
-// cache (256) and would walk their runs, and sooner in tables whose phases of
-// single waves do not fill the chip; the other kinds sooner still, as they
-// always walk.  Filling to 65% load by shift path and walk, and dense: 2^23
-// slots, 212 items a region, 1,448 and 1,069 us; 2^24, 212, 1,760 and 1,710;
-// 2^25 (10,900 regions), 245, 2,394 and 2,679, 262, 2,587 and 2,420; 2^26, 215,
-// 3,244 and 5,429, 258, 4,018 and 4,428, 275, 4,767 and 4,401.
-constexpr uint64_t kFlatItems = 208, kFlatItemsMany = 260, kFlatManyRegions = 8192, kFlatItemsMixed = 96;
-bool gqf_rebuild_is_dense(uint64_t n_items, uint64_t nregions) { return n_items >= kFlatItems * nregions; }
+// Which batches take the workgroup-wide rebuild (gqf_flat.h): those of at least
+// so many items for each region that they can reach.  A region by itself is
+// faster that way, with counts or request tags however few its items, with
+// inserts by one (which have the shift path) from about 200; but single waves do
+// four times as many regions at once, so the line rises with the regions until
+// these fill the chip, and then stands where regions outgrow the item cache
+// (256), as the walk reads what is past it from memory.  us for a whole call,
+// single waves / dense:
+//   counts    342 regions, 3 items a region: 49 / 44 into an empty table, 107 / 60 at 70%
+//             load; 683, 8: 58 / 54 and 121 / 72; 1,366, 32: 121 / 132 and 184 / 160; 2,731,
+//             95: 200 / 214 and 272 / 255; 5,463, 150: 245 / 265 and 368 / 330; 10,923,
+//             230: 319 / 300 and, at 50%, 583 / 399; 21,846, 230: 560 / 608 and 920 / 774,
+//             260: 670 / 632 and 1,313 / 791; 43,691, 260: 1,213 / 1,194 and 2,410 / 1,506.
+//   sequenced 342, 3: 35 / 35 and 96 / 52; 683, 8: 43 / 42 and 106 / 61; 2,731, 48: 66 / 85
+//             and 153 / 138; 5,463, 95: 119 / 144 and 244 / 214; 10,923, 200: 301 / 301 and
+//             445 / 411; 21,846, 260: 812 / 716 and 1,548 / 907.
+//   inserts   2,731, 212 on the way to 65% load: 1,448 / 1,069 in all; 5,463: 1,760 /
+//             1,710; 21,846, 262: 368 / 482 into an empty table, 596 / 592 at 25%,
+//             740 / 640 at 50%, 400: 527 / 553, 833 / 656 and 1,039 / 713; 43,691 and
+//             87,382 alike.
+// Between two lines the load of the table decides, which the device finds
+// (gqf_rebuild_form).
+struct DenseLine {
+  uint64_t loaded, empty;  // items a region, in a table at kLoaded or above and in an empty one
+};
+constexpr double kLoaded = 0.25;
+static DenseLine dense_line(int kind, uint64_t regions) {
+  if (kind == gqf_flat::kAdd) {
+    if (regions < 4096) return {208, 208};
+    return regions < 8192 ? DenseLine{208, 280} : DenseLine{270, 420};
+  }
+  const uint64_t line = regions < 1024 ? 0 : regions / (kind == gqf_flat::kCounts ? 32 : 64);
+  return {std::min<uint64_t>(line, 225), std::min<uint64_t>(2 * line, 256)};
+}
+
+// *dense = 1 if the n items (or *n_dev) reach the line: `loaded` of them, and
+// up to `empty` in a table whose load is below kLoaded, by the used slots of 256
+// blocks spread over it.  One short launch ahead of the phases (which change the
+// table), only for batches that the host cannot tell by their size.
+extern "C" __global__ void __launch_bounds__(256)
+gqf_rebuild_form(const QF* __restrict__ qfp, uint64_t n, const uint64_t* __restrict__ n_dev, uint64_t loaded,
+                 uint64_t empty, uint32_t* __restrict__ dense) {
+  __shared__ uint32_t sum[4];
+  const QF& qf = *qfp;
+  const uint64_t b = (uint64_t)threadIdx.x * qf.nblocks / 256;
+  const uint64_t used = ((const GQF_GLOBAL uint64_t*)gqf_block_ptr(qf, b))[3];
+  const uint32_t incl = wave_scan_add((uint32_t)__popcll(used));
+  if ((threadIdx.x & 63) == 63) sum[threadIdx.x >> 6] = incl;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const double load = (double)(sum[0] + sum[1] + sum[2] + sum[3]) / (256.0 * 64.0);
+    const double line = (double)loaded + (load < kLoaded ? (double)(empty - loaded) * (1.0 - load / kLoaded) : 0.0);
+    *dense = (double)(n_dev ? *n_dev : n) >= line ? 1u : 0u;
+  }
+}
+
+// Groups: from 208 items a region on, however many regions: their launch for
+// fewer (gqf_group_rebuild) is a persistent one whose workgroups search for every
+// region's items and wait for their neighbours.  24 filters of 2^22 .. 2^24 slots
+// (75,000 regions): 6,371 us by that at 200 items a region, dense 3,301 at 212; 8
+// filters, 3,700 regions: 326 and 234.
+constexpr uint64_t kGroupDense = 208;
+bool gqf_group_is_dense(uint64_t n_items, uint64_t nregions) { return n_items >= kGroupDense * nregions; }
 
 void gqf_launch_rebuild(const QF* qf_dev, uint64_t nregions, uint64_t region_blocks, const uint64_t* items,
                         const uint64_t* counts, uint64_t n_items, const uint32_t* region_start,
-                        const uint32_t* region_list, const uint32_t* list_count, int mode, uint8_t* wide_flags,
-                        uint32_t* wide_count, hipStream_t s) {
+                        const uint32_t* region_list, uint32_t* list_count, int mode, uint8_t* wide_flags,
+                        uint32_t* wide_count, hipStream_t s, const uint64_t* n_dev, uint64_t reach) {
   // at most one workgroup per non-empty region: no more than the regions
   // of a parity, nor than the items
   const uint64_t per_parity = (nregions + 1) / 2;
@@ -2451,26 +2509,36 @@ void gqf_launch_rebuild(const QF* qf_dev, uint64_t nregions, uint64_t region_blo
     fprintf(stderr, "gqf: %u wide classes for %llu-block regions\n", ncls, (unsigned long long)region_blocks);
     abort();
   }
+  const bool del = mode == kDelete;
   const int kind = mode == kSeq ? gqf_flat::kTagged : (counts ? gqf_flat::kCounts : gqf_flat::kAdd);
-  const uint64_t line = kind != gqf_flat::kAdd ? kFlatItemsMixed
-                        : nregions < kFlatManyRegions ? kFlatItems : kFlatItemsMany;
-  const bool flat = n_items >= line * nregions;
+  if (!reach || reach > nregions) reach = nregions;
+  const DenseLine line = dense_line(kind, reach);
+  const bool maybe = !del && n_items >= line.loaded * reach;            // dense, if at all
+  const bool surely = maybe && (!n_dev || !line.empty) && n_items >= line.empty * reach;
+  uint32_t* form = nullptr;
+  if (maybe && !surely) {
+    form = list_count + 2;
+    hipLaunchKernelGGL(gqf_rebuild_form, dim3(1), dim3(256), 0, s, qf_dev, n_items, n_dev, line.loaded * reach,
+                       line.empty * reach, form);
+  }
   mode |= gqf_rebuild_mode_flags();
   for (int parity = 0; parity < 2; parity++) {
     const uint32_t* list = region_list ? region_list + (size_t)parity * stride : nullptr;
     gqf_prof_begin("rebuild_phase", s);
-    if ((mode & ~GQF_REBUILD_NO_SHIFT) == kDelete)
+    if (del)
       hipLaunchKernelGGL(gqf_rebuild_delete, dim3(g), dim3(64), 0, s, qf_dev, items, region_start,
                          list, list_count, parity, wide_flags, wide_count);
-    else if (flat)
+    if (maybe)
       hipLaunchKernelGGL(gqf_rebuild_flat, dim3(g), dim3(gqf_flat::kThreads), 0, s, qf_dev, items, counts, region_start,
-                         list, list_count, parity, kind, wide_flags, wide_count);
-    else if (counts || (mode & ~GQF_REBUILD_NO_SHIFT) == kSeq)
-      hipLaunchKernelGGL(gqf_rebuild_phase_counts, dim3(g), dim3(64), 0, s, qf_dev, items, counts, region_start,
-                         list, list_count, parity, mode, wide_flags, wide_count);
-    else
-      hipLaunchKernelGGL(gqf_rebuild_phase, dim3(g), dim3(64), 0, s, qf_dev, items, region_start,
-                         list, list_count, parity, mode, wide_flags, wide_count);
+                         list, list_count, form, parity, kind, wide_flags, wide_count);
+    if (!del && !surely) {
+      if (kind != gqf_flat::kAdd)
+        hipLaunchKernelGGL(gqf_rebuild_phase_counts, dim3(g), dim3(64), 0, s, qf_dev, items, counts, region_start,
+                           list, list_count, form, parity, mode, wide_flags, wide_count);
+      else
+        hipLaunchKernelGGL(gqf_rebuild_phase, dim3(g), dim3(64), 0, s, qf_dev, items, region_start,
+                           list, list_count, form, parity, mode, wide_flags, wide_count);
+    }
     gqf_prof_end("rebuild_phase", s);
     gqf_prof_begin("rebuild_wide", s);
     hipLaunchKernelGGL(gqf_rebuild_wide, dim3(ncls * kWideClassGrid), dim3(64), 0, s, qf_dev, items, counts,
