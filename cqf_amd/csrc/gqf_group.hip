@@ -9,10 +9,12 @@
 //            above the hash bits: (f << S) | hash;
 //   sort     one radix sort of all tagged keys (filters come out in
 //            segment order, each sorted by hash);
-//   rebuild  ONE persistent launch over every filter's regions: workgroup
+//   rebuild  batches of many items a region: a launch over every filter's
+//            even regions and one over the odd ones, a workgroup each
+//            (gqf_group_is_dense); others ONE persistent launch: workgroup
 //            w takes work items w, w + G, w + 2G, ... (even regions of
 //            every filter first, then odd ones that wait for their even
-//            neighbours; gqf_rebuild.hip), plus a wide-redo tail that
+//            neighbours; gqf_rebuild.hip); then a wide-redo tail that
 //            exits at once when nothing overflowed;
 //   untag    each segment is left holding its filter's ascending hashes,
 //            as bulk_insert leaves its keys.
@@ -550,11 +552,19 @@ namespace {
 // Workgroups per CU of the group's persistent rebuild: times the group
 // insert of a batch cut like `offsets` into scratch filters of the same
 // sizes and region size, for each candidate up to what the GPU keeps
-// resident, and returns the fastest (0 if nothing could be timed).
+// resident, and returns the fastest (0 if nothing could be timed, or if such
+// a batch is dense: that form has no grid to choose, and timing it picked one
+// for the group's sparse batches by chance).
 uint32_t tune_per_cu(Group* g, const uint64_t* offsets) {
   const uint64_t n = offsets[g->nf];
   const uint32_t mx = gqf_group_rebuild_max_per_cu();
-  if (n == 0) return 0;
+  uint64_t regions = 0;
+  for (uint32_t f = 0; f < g->nf; f++) {
+    QF d;
+    if (!gqf_filter_host(g->handles[f], &d)) return 0;
+    regions += d.nregions;
+  }
+  if (n == 0 || gqf_group_is_dense(n, regions)) return 0;
   std::vector<QF*> scratch(g->nf, nullptr);
   bool ok = true;
   for (uint32_t f = 0; f < g->nf && ok; f++) {

@@ -2280,8 +2280,8 @@ __device__ inline void region_hash_bounds(const gqf_group_dev& g, const QF& qf, 
 // polled value.  (A workgroup is one wave, so its __syncthreads() is only a
 // wave barrier: it does not keep lanes in the same loop iteration, and a
 // per-lane loop condition would let the compiler split the lanes.)
-// Three waves per SIMD (168 VGPRs, no spills) keep 12 workgroups per CU
-// resident, as many as the LDS allows.
+// Three waves per SIMD (168 VGPRs, three of them spilled) keep 12 workgroups
+// per CU resident, as many as the LDS allows.
 extern "C" __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3)))
 gqf_group_rebuild(gqf_group_dev g, const uint64_t* __restrict__ items, int mode) {
   __shared__ Smem<kWinFast> sm;
@@ -2552,8 +2552,7 @@ void gqf_launch_rebuild(const QF* qf_dev, uint64_t nregions, uint64_t region_blo
 // grid must be: see gqf_group_rebuild), and the grid for `per_cu` of them
 // (0: the default, clamped to what is resident).  Up to 12 are resident
 // (3 waves per SIMD; 13,088 B of LDS each); the default is 8, and
-// gqf_group_autotune times the candidates for a group's own shape (10 for
-// the 256-filter k-mer workload).
+// gqf_group_autotune times the candidates for a group's own shape.
 uint32_t gqf_group_rebuild_max_per_cu() {
   static int per_cu = 0;
   if (!per_cu) {

@@ -193,8 +193,9 @@ int qf_bulk_get_seq_adjust(QF *qf, uint64_t n, const uint64_t *keys, uint32_t nr
  * [offsets[f], offsets[f+1]) (offsets: host array of nfilters + 1, offsets[0]
  * = 0).  gqf_group_bulk_insert gives every segment bulk_insert semantics
  * (the segment is left holding its filter's ascending hashes) with one
- * radix sort and ONE persistent rebuild launch for all filters, captured
- * into a hipGraph per shape and replayed; gqf_group_bulk_get fills
+ * radix sort and one rebuild over all filters -- one persistent launch, or,
+ * from 208 keys per rebuild region on, one launch per region parity --
+ * captured into a hipGraph per shape and replayed; gqf_group_bulk_get fills
  * returns[i] with the count of vals[i] in its segment's filter, in one
  * launch.  Stream-ordered; a call whose segments or filter tuning differ
  * from the previous one synchronises first.  A group insert takes at most
@@ -217,10 +218,10 @@ int gqf_autotune(int nbits, double load, uint32_t *region_blocks, uint32_t *sort
  * outside 16..56 or a digit width other than 0 (default) or 6..10 */
 int gqf_autotune_set(int nbits, double load, uint32_t region_blocks, uint32_t sort_digit_bits);
 /* gqf_autotune for every filter of the group at the load its segment
- * brings, applied with qf_set_tuning; then the workgroups per CU of the
- * group's persistent rebuild, timed for a batch cut like `offsets` on
- * scratch filters of the same sizes (candidates 4..16 up to what the GPU
- * keeps resident); synchronises */
+ * brings, applied with qf_set_tuning; then, for a batch that takes the
+ * persistent rebuild, its workgroups per CU, timed for a batch cut like
+ * `offsets` on scratch filters of the same sizes (candidates 4..16 up to what
+ * the GPU keeps resident; other batches leave the setting); synchronises */
 int gqf_group_autotune(gqf_group *g, const uint64_t *offsets);
 /* bound on the polls of an odd region's wait for its even neighbours in
  * the persistent rebuild (default 2^22).  A region whose wait runs out is

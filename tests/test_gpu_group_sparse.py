@@ -135,3 +135,23 @@ def test_queued_runs_in_a_group(gpu, run, queued):
         group.close()
         for f in filters:
             f.close()
+
+
+def test_autotune_of_a_dense_shape_leaves_the_grid(gpu, oracle):
+    """A batch that takes the dense form has no grid: what sparse batches use
+    stays as it was set; a sparse shape's grid is one of the candidates."""
+    from cqf_amd.gqf import GQF, GQFGroup
+    print("case autotune dense and sparse shapes", flush=True)
+    filters = [GQF(q) for q in QS]
+    group = GQFGroup(filters)
+    try:
+        group.workgroups_per_cu = 3
+        regions = [f.info["nregions"] for f in filters]
+        group.autotune(np.cumsum([0] + [1000 * r for r in regions]).tolist())
+        assert group.workgroups_per_cu == 3
+        group.autotune(np.cumsum([0] + [100 * f.info["nregions"] for f in filters]).tolist())
+        assert group.workgroups_per_cu in (4, 6, 8, 10, 12, 16)
+    finally:
+        group.close()
+        for f in filters:
+            f.close()
