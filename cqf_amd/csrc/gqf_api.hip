@@ -31,6 +31,7 @@ int g_last_error = 0;
 
 void note_error(hipError_t e, const char* what) {
   if (e == hipSuccess) return;
+  (void)hipGetLastError();  // reported here: not again by a later launch's check
   std::lock_guard<std::mutex> lk(g_mu);
   if (!g_last_error) g_last_error = (int)e;
   fprintf(stderr, "libgqf: %s failed: %s\n", what, hipGetErrorString(e));
@@ -123,6 +124,13 @@ void free_workspace(Workspace& w) {
   w.cap = 0;
 }
 
+void free_agg_workspace(Workspace& w) {
+  dev_free(w.agg_stage);
+  dev_free(w.agg_sums);
+  dev_free(w.agg_hot);
+  dev_free(w.agg_ctrl);
+}
+
 void free_enum_space(EnumSpace& e) {
   dev_free(e.t.items);
   dev_free(e.t.slots);
@@ -155,8 +163,21 @@ bool ensure_enum_space(EnumSpace& e, uint64_t groups) {
   return ok;
 }
 
-// the per-table part of a workspace: region tables of the rebuild
-void init_region_workspace(Workspace& w, uint64_t nblocks) {
+void free_region_workspace(Workspace& w) {
+  dev_free(w.totals);
+  dev_free(w.slow_buckets);
+  dev_free(w.m_dev);
+  dev_free(w.region_start);
+  dev_free(w.region_list);
+  dev_free(w.list_count);
+  dev_free(w.wide_flags);
+  dev_free(w.wide_count);
+  dev_free(w.misses);
+}
+
+// the per-table part of a workspace: region tables of the rebuild; false (and
+// none of them) if an allocation failed
+bool init_region_workspace(Workspace& w, uint64_t nblocks) {
   if (!w.totals) {
     dev_alloc(&w.totals, GQF_SORT_TOTALS);
     dev_alloc(&w.slow_buckets, GQF_SORT_MAX_BUCKETS);
@@ -172,15 +193,23 @@ void init_region_workspace(Workspace& w, uint64_t nblocks) {
     dev_alloc(&w.wide_count, GQF_WIDE_WORDS);
     GQF_CHECK(hipMemset(w.wide_count, 0, GQF_WIDE_WORDS * sizeof(uint32_t)));
     dev_alloc(&w.misses, 1);
+    if (!w.totals || !w.slow_buckets || !w.m_dev || !w.region_start || !w.region_list || !w.list_count ||
+        !w.wide_flags || !w.wide_count || !w.misses) {
+      free_region_workspace(w);
+      return false;
+    }
   }
+  return true;
 }
 
-// grow the per-key buffers to hold n keys (synchronises when it allocates)
-void ensure_workspace(Filter* f, uint64_t n) {
+// grow the per-key buffers to hold n keys (synchronises when it allocates);
+// false if an allocation failed (qf_last_error has it): nothing may be
+// launched on the workspace then
+bool ensure_workspace(Filter* f, uint64_t n) {
   std::lock_guard<std::mutex> lk(f->mu);
   Workspace& w = f->ws;
-  init_region_workspace(w, f->host.nblocks);
-  if (n <= w.cap) return;
+  if (!init_region_workspace(w, f->host.nblocks)) return false;
+  if (n <= w.cap) return true;
   GQF_CHECK(hipDeviceSynchronize());
   free_workspace(w);
   uint64_t cap = n < 4096 ? 4096 : n;
@@ -190,7 +219,12 @@ void ensure_workspace(Filter* f, uint64_t n) {
   dev_alloc(&w.ukeys, cap);
   dev_alloc(&w.upos, cap);
   dev_alloc(&w.ucounts, cap);
+  if (!w.tmp || !w.hist || !w.tile_heads || !w.ukeys || !w.upos || !w.ucounts) {
+    free_workspace(w);
+    return false;
+  }
   w.cap = cap;
+  return true;
 }
 
 // Counting reduce of a duplicate-heavy batch of hashed keys: the hashes are
@@ -217,12 +251,15 @@ bool reduce_by_counting(Filter* f, uint64_t n, uint64_t* keys, int bits, hipStre
   if (n < kAggMinKeys || bits > 40 || stream_capturing(s)) return false;
   {
     std::lock_guard<std::mutex> lk(f->mu);
-    if (!w.agg_stage) {
+    if (!w.agg_ctrl) {  // the last of them
       dev_alloc(&w.agg_stage, (uint64_t)GQF_AGG_BUCKETS * GQF_AGG_BUCKET_CAP);
       dev_alloc(&w.agg_sums, GQF_AGG_BUCKETS);
       dev_alloc(&w.agg_hot, GQF_AGG_HOT + 1);
       dev_alloc(&w.agg_ctrl, 4 + GQF_AGG_BUCKETS);
-      if (!w.agg_stage || !w.agg_sums || !w.agg_hot || !w.agg_ctrl) return false;
+      if (!w.agg_stage || !w.agg_sums || !w.agg_hot || !w.agg_ctrl) {
+        free_agg_workspace(w);
+        return false;
+      }
     }
   }
   const uint64_t mask = gqf_mask(f->host.key_bits);
@@ -266,7 +303,7 @@ void mutate(QF* qf, uint64_t n, uint64_t* keys, uint8_t flags, int mode, bool re
     for (uint32_t k = 0; k < np; k++) mutate(qf, start[k + 1] - start[k], keys + start[k], flags, mode, reduce, s);
     return;
   }
-  ensure_workspace(f, n);
+  if (!ensure_workspace(f, n)) return;
   run_mutation(f, f->ws, n, keys, flags, mode, reduce, s);
 }
 
@@ -357,7 +394,7 @@ uint64_t count_misses(QF* qf, uint64_t* vals, uint64_t n) {
   if (n == 0) return 0;
   Filter* f = lookup(qf);
   if (!f) return 0;
-  ensure_workspace(f, 0);
+  if (!ensure_workspace(f, 0)) return n;
   GQF_CHECK(hipMemsetAsync(f->ws.misses, 0, sizeof(unsigned long long), 0));
   gqf_launch_misses(f->dev, vals, n, f->ws.misses, 0);
   unsigned long long h = 0;
@@ -484,19 +521,8 @@ Filter* create_filter(int nbits, int vb) {
 
 void free_all_workspace(Workspace& w) {
   free_workspace(w);
-  dev_free(w.totals);
-  dev_free(w.slow_buckets);
-  dev_free(w.m_dev);
-  dev_free(w.region_start);
-  dev_free(w.region_list);
-  dev_free(w.list_count);
-  dev_free(w.wide_flags);
-  dev_free(w.wide_count);
-  dev_free(w.misses);
-  dev_free(w.agg_stage);
-  dev_free(w.agg_sums);
-  dev_free(w.agg_hot);
-  dev_free(w.agg_ctrl);
+  free_region_workspace(w);
+  free_agg_workspace(w);
 }
 
 }  // namespace
@@ -560,7 +586,7 @@ extern "C" uint64_t point_get_wrapper(QF* qf, uint64_t* hashes, uint64_t nitems)
   if (nitems == 0) return 0;
   Filter* f = lookup(qf);
   if (!f) return 0;
-  ensure_workspace(f, 0);
+  if (!ensure_workspace(f, 0)) return nitems;
   GQF_CHECK(hipMemsetAsync(f->ws.misses, 0, sizeof(unsigned long long), 0));
   gqf_launch_point_query(f->dev, hashes, nitems, 0, nullptr, 0, f->ws.misses, 0);
   unsigned long long h = 0;
@@ -773,7 +799,7 @@ extern "C" int qf_bulk_mutate_seq(QF* qf, uint64_t n, uint64_t* keys, uint32_t n
   gqf_seq_reqs reqs;
   if (!seq_requests(n, nreq, req_end, req_tag, true, reqs)) return -3;
   if (n == 0) return 0;
-  ensure_workspace(f, n);
+  if (!ensure_workspace(f, n)) return -4;
   Workspace& w = f->ws;
   const hipStream_t s = (hipStream_t)stream;
   gqf_launch_seq_tag(f->dev, keys, n, reqs, s);
@@ -951,8 +977,7 @@ extern "C" int qf_set_tuning(QF* qf, uint32_t region_blocks, uint32_t sort_digit
 extern "C" int qf_reserve(QF* qf, uint64_t max_batch) {
   Filter* f = lookup(qf);
   if (!f) return -1;
-  ensure_workspace(f, max_batch);
-  return f->ws.cap >= max_batch ? 0 : -2;
+  return ensure_workspace(f, max_batch) ? 0 : -2;
 }
 
 extern "C" uint32_t qf_batch_pieces(uint64_t n, uint64_t max_piece, uint64_t* starts, uint32_t cap) {
@@ -1118,7 +1143,7 @@ int64_t move_items(Filter* f, const QF* dst_dev, const QF& dst, Workspace& dst_w
   }
   uint64_t* items = dst_es.move_items;
   uint64_t* counts = dst_es.move_counts;
-  init_region_workspace(dst_ws, dst.nblocks);
+  if (!init_region_workspace(dst_ws, dst.nblocks)) return -3;
   for (uint64_t u = 0; u < groups;) {
     uint64_t v = u + 1;
     while (v < groups && base[v + 1] - base[u] <= cap) v++;

@@ -119,7 +119,8 @@ int qf_import_image_device(QF *qf, const void *dev_src, uint64_t nbytes, void *s
 /* empty the table (stream-ordered); mirrors qf_reset, src/gqf.cu:2283-2299 */
 int qf_reset_device(QF *qf, void *stream);
 /* size the per-filter workspace for batches up to max_batch keys so that
- * later bulk calls allocate nothing */
+ * later bulk calls allocate nothing; -2 if there is no memory for it (a bulk
+ * call that finds none launches nothing, and qf_last_error has the reason) */
 int qf_reserve(QF *qf, uint64_t max_batch);
 /* tuning (0 keeps a value): blocks per rebuild region, 16..56 (the push
  * window is min(64, 2 x region) minus that), and radix digit bits of the
@@ -342,8 +343,10 @@ int64_t qf_resize_device(QF *qf, int new_nbits);
 
 /* qfc += every item of qfa and qfb, counts added (qf_merge,
  * src/gqf.cu:3896-3938).  All filters must have the same key_bits, and qfc
- * at least the value bits of each input.  Returns the number of items
- * inserted, or < 0 on error. */
+ * at least the value bits of each input.  qfc keeps the buffers that the
+ * items pass through (at most 64 MB) and every input its tables of a count
+ * pass (24 bytes per 62 blocks) until they are destroyed.  Returns the number
+ * of items inserted, or < 0 on error. */
 int64_t qf_merge_device(QF *qfa, QF *qfb, QF *qfc);
 /* qfr += every item of the nqf filters (qf_multi_merge, src/gqf.cu:3943-4008) */
 int64_t qf_multi_merge_device(QF *const *qfs, int nqf, QF *qfr);
