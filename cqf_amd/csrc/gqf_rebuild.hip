@@ -2461,6 +2461,8 @@ static DenseLine dense_line(int kind, uint64_t regions) {
     return regions < 8192 ? DenseLine{208, 280} : DenseLine{270, 420};
   }
   const uint64_t line = regions < 1024 ? 0 : regions / (kind == gqf_flat::kCounts ? 32 : 64);
+  // (served tables are loaded: asking the device takes 6 us of such a call)
+  if (kind == gqf_flat::kTagged && regions < 8192) return {line, line};
   return {std::min<uint64_t>(line, 225), std::min<uint64_t>(2 * line, 256)};
 }
 
