@@ -33,8 +33,9 @@
 // batches, per launch: 943,718 keys into an empty table of 2^20 slots 268 ->
 // 20 us; 14.1 M items into a table of 2^25 slots in four chunks 214 -> 55 us a
 // chunk on average; a served batch at 2^24 slots, 42 items a region, 114 ->
-// 83 us.  On a nearly empty table the walk is ahead (69 and 184 us at 2^26
-// slots), hence the lines of gqf_launch_rebuild.
+// 83 us.  On regions with few entries the other forms are ahead (counted items
+// into a nearly empty table of 2^26 slots: 69 us by the walk, 184 here), hence
+// dense_line.
 // Decoding every counter of two slots, in code repeated for each of a
 // thread's slots, took 94 us for the served batch and 62 us a chunk.
 // One lane per slot with a scan per 64 slots took 294 us where the eight

@@ -1565,12 +1565,13 @@ __device__ __forceinline__ int rebuild_span(const QF& qf, const Span& sp, const 
 // The run ends follow from the marks: a kept byte is its run's last if no
 // kept byte follows it up to the old run end.
 //
-// Bound by VALU issue: 2,900 instructions a region wave (128 VGPRs, 15.9 KB
-// of LDS: ten waves on a CU), a third of what the run walk below took for it
-// (8,050), which paired every run with its quotient one by one on its block's
-// lane, in both passes.  7.55 M deletes from 2^28 slots at 88% load: 770 ->
-// 304 us a launch; 5,000 from 2^24 slots: 33 -> 17 us (only blocks that change
-// are stored).  Slots in 16 bits with their flags need no bound on the shift;
+// Bound by VALU issue: 2,900 instructions a region wave at 86 deletes a region,
+// 3,200 at 173 (128 VGPRs, 15.9 KB of LDS: ten waves on a CU), where the run
+// walk below took 8,050, which paired every run with its quotient one by one on
+// its block's lane, in both passes.  2^28 slots at 88% load, a launch (half the
+// regions) of a batch of 7.55 M: 770 -> 300 us; of a batch of 15.1 M: 740 -> 348
+// us; 5,000 from 2^24 slots: 33 -> 17 us (only blocks that change are stored).
+// Slots in 16 bits with their flags need no bound on the shift;
 // reading the caps again in the second pass instead of keeping them would
 // cost 64 more LDS reads a lane.
 struct DeleteSmem {
