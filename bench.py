@@ -49,7 +49,7 @@ def parse():
                          "(default: profiles/traffic_q28.md, profiles/traffic_table_q28.md for --workload table)")
     ap.add_argument("--workload", choices=["bulk", "zipf", "groups", "serve", "table", "loadcurve"], default="bulk",
                     help="bulk: uniform insert/get/delete (default); zipf: skewed bulk_insert_reduce; "
-                         "groups: 256 k-mer filters in one persistent launch; serve: served request stream; "
+                         "groups: 256 k-mer filters in one group call; serve: served request stream; "
                          "table: enumeration, census, statistics, file image and growth of a full table; "
                          "loadcurve: insert and lookup rates at every 5% load step to 95%")
     ap.add_argument("--serve-requests", type=int, default=6000)

@@ -1057,10 +1057,10 @@ gqf_sort_buckets_slow_tagged(uint64_t* in, uint64_t* out, uint64_t n, int low_bi
 // its rank among the keys of its sub-bucket (two on average at 8192 uniform
 // keys).  A sub-bucket above kSubCap keys (repeats) makes the workgroup sort all
 // of them by digits instead (lds_sort), or, up to kTNetwork keys, by a bitonic
-// network: repeats of a few of 300 / 1,000 / 2,000 keys, a whole delete, 30 / 37 /
-// 47 us by the network and 43 / 48 / 53 by digits; 8,192 go the other way.  Latency bound: 12 us for 5000
-// keys, against 63 us for the four passes (12 launches) of the LSD sort plus 9
-// for the region bounds.
+// network: a whole delete of 300 / 1,000 / 2,000 keys that repeat a few, 30 / 37 /
+// 47 us by the network and 43 / 48 / 53 by digits; a reduce of 8,192 equal keys,
+// 135 and 85.  Latency bound: 12 us for 5000 keys, against 63 us for the four
+// passes (12 launches) of the LSD sort plus 9 for the region bounds.
 
 namespace {
 constexpr int kTThreads = 1024;
